@@ -3,241 +3,14 @@
 
 #include <atomic>
 
-#include "gemm_rows.h"
-#include "gemm_fwd256.h"
-#include "gemm_bwdx256.h"
-#include "gemm_ws256.h"
-#include "gemm_wgrad256.h"
-#include "gemm_wgrad.h"
+#include "host_util.h"
+#include "ir_grad.h"
 #include "misc_kernels.h"
 #include "weight_kernels.h"
 #include "select_kernels.h"
 #include "prepare_sel.h"
 
 using namespace amoe;
-
-namespace {
-
-inline bool aligned(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
-inline int launch_rc() {
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? AMOE_OK : (int)e;
-}
-inline int check_bounds(int n_tiles, const int32_t* b, int K) {
-  if (n_tiles < 1 || n_tiles > AMOE_MAX_TILES) return AMOE_EINVAL;
-  if (b[0] != 0 || b[n_tiles] != K) return AMOE_ESHAPE;
-  for (int t = 0; t < n_tiles; t++)
-    if (b[t + 1] <= b[t]) return AMOE_ESHAPE;
-  return AMOE_OK;
-}
-inline bool bounds_multiple_of(int n_tiles, const int32_t* b, int m) {
-  for (int t = 0; t <= n_tiles; t++)
-    if (b[t] % m) return false;
-  return true;
-}
-inline size_t esize(int dtype) { return dtype == AMOE_F32 ? 4 : 2; }
-// Whether every DAC code of a quantiser with step inp_res (codes -1/inp_res .. 1/inp_res) is exact in the type.
-inline bool dac_codes_fit(int dtype, float inp_res) {
-  if (dtype == AMOE_F32 || !(inp_res > 0.f)) return true;
-  return 1.0f / inp_res <= (dtype == AMOE_BF16 ? 256.f : 2048.f) * (1.0f + 1e-6f);
-}
-inline int max_row_tiles(int64_t M, int E) { return (int)(M / kTileRows) + E; }
-
-// Compute units of the current device (read once; the value cannot change while the process lives).
-inline int num_compute_units() {
-  static const int n = [] {
-    int dev = 0, cu = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0) return 256;
-    return cu;
-  }();
-  return n;
-}
-
-// Persistent grid of the row-gather GEMM: two workgroups per compute unit, more if a workgroup
-// would otherwise get more work items than its descriptor table holds, rounded up to a multiple
-// of the column-block count (so that the column blocks of one row tile run side by side), never
-// more than there are work items.
-inline int persistent_grid(int row_tiles, int col_blocks, int per_cu = 2) {
-  const long long work = (long long)row_tiles * col_blocks;
-  long long g = (long long)per_cu * num_compute_units();
-  const long long need = (work + kMaxDesc - 1) / kMaxDesc;
-  if (need > g) g = need;
-  if (g % col_blocks) g += col_blocks - g % col_blocks;
-  if (g > work) g = work;
-  return g < 1 ? 1 : (int)g;
-}
-
-// Every tile of the launch is interior: the FAST instantiation applies.
-inline bool rows_all_interior(const RowsParams& p, int mode, int bk) {
-  if (!p.a_vec || !p.w_vec || !p.out_stage || !p.buf_ok || p.abs_max != nullptr) return false;
-  if (p.xq_out != nullptr && !p.xq_stage) return false;
-  if (p.xc_out != nullptr && !p.xc_vec) return false;
-  // forward: the edge-free code has the clip-and-quantise input stage or none at all
-  if (mode != MODE_BWDX && (p.ir != nullptr) != (p.inp_res > 0.f)) return false;
-  if (p.noise != nullptr && !p.noise_vec) return false;
-  if (p.xf != nullptr && !p.xf_vec) return false;
-  for (int t = 0; t < p.n_col_tiles; t++)
-    if ((p.col_bounds[t + 1] - p.col_bounds[t]) % kTileCols) return false;
-  for (int t = 0; t < p.n_kd_tiles; t++)
-    if ((p.kd_bounds[t + 1] - p.kd_bounds[t]) % bk) return false;
-  return true;
-}
-
-template <typename T, bool W_KC, bool FAST>
-int launch_rows_mode(const RowsParams& p, int mode, int grid, hipStream_t st) {
-  if (mode == MODE_FWD) {
-    auto k = &gemm_rows_kernel<T, W_KC, MODE_FWD, FAST>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, st, p);
-  } else if (mode == MODE_FWD_SPLIT) {
-    auto k = &gemm_rows_kernel<T, W_KC, MODE_FWD_SPLIT, FAST>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, st, p);
-  } else {
-    auto k = &gemm_rows_kernel<T, W_KC, MODE_BWDX, FAST>;
-    hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, st, p);
-  }
-  return launch_rc();
-}
-
-template <typename T, bool W_KC>
-int launch_rows(const RowsParams& p, int mode, int grid, hipStream_t st) {
-  return rows_all_interior(p, mode, Elem<T>::kBK) ? launch_rows_mode<T, W_KC, true>(p, mode, grid, st)
-                                            : launch_rows_mode<T, W_KC, false>(p, mode, grid, st);
-}
-
-// The 128 x 256 forward kernel for the usual training shapes (bf16 or fp16, every tile interior, per-expert input
-// ranges, one max |W| per expert).  AMOE_EUNSUPPORTED: this launch is not one of them; the general kernel runs.
-template <typename T, int A_MODE, bool ANALOG, bool NOISE, bool SPLIT2, bool ZCODES = false>
-int launch_fwd256_as(const RowsParams& p, int grid, hipStream_t st) {
-  auto k = &fwd256_kernel<T, A_MODE, ANALOG, NOISE, SPLIT2, ZCODES>;
-  hipLaunchKernelGGL(k, dim3(grid), dim3(kThreads), 0, st, p);
-  return launch_rc();
-}
-
-// The input gradient reads the forward input x (through xf_index) only for the features that need it: the
-// input-range clip, the ReLU mask, the clipped-input output.  A caller that passes x without any of them has not
-// been asked for xf_index, and its launch is a plain product.
-inline bool bwdx_reads_x(const amoe_bwd_x_args* a) {
-  return a->x != nullptr && a->xf_index != nullptr && (a->ir != nullptr || a->relu_mask != 0 || a->xc_out != nullptr);
-}
-
-// The 128 x 256 input-gradient kernel, for the same launches (and column tiles that are multiples of 256).  The
-// partial sums of the input-range gradient then cover 256 columns each; *n_count_blocks is the grid that ran.
-template <typename T, int COLS>
-int launch_bwdx256_cols(RowsParams p, const amoe_bwd_x_args* a, hipStream_t st, int* n_count_blocks) {
-  p.n_col_blocks = count_col_blocks(p.col_bounds, p.n_col_tiles, COLS);
-  const int grid = persistent_grid(max_row_tiles(a->M, a->E), p.n_col_blocks, COLS == 128 ? 3 : 2);
-  *n_count_blocks = grid;
-  const bool relu = a->relu_mask != 0, xc = a->xc_out != nullptr;
-  if (!bwdx_reads_x(a)) {
-    hipLaunchKernelGGL((&bwdx256_kernel<T, false, false, false, COLS>), dim3(grid), dim3(kThreads), 0, st, p);
-  } else if (!relu) {
-    if (xc) hipLaunchKernelGGL((&bwdx256_kernel<T, true, false, true, COLS>), dim3(grid), dim3(kThreads), 0, st, p);
-    else hipLaunchKernelGGL((&bwdx256_kernel<T, true, false, false, COLS>), dim3(grid), dim3(kThreads), 0, st, p);
-  } else {
-    if (xc) hipLaunchKernelGGL((&bwdx256_kernel<T, true, true, true, COLS>), dim3(grid), dim3(kThreads), 0, st, p);
-    else hipLaunchKernelGGL((&bwdx256_kernel<T, true, true, false, COLS>), dim3(grid), dim3(kThreads), 0, st, p);
-  }
-  return launch_rc();
-}
-
-// The kernel that keeps the weights in registers (gemm_ws256.h): a contraction of exactly 256, output columns in
-// groups of 256, interior launches.  Two workgroups per CU, in equal shares per column group, and more if a
-// workgroup's run of 32-row blocks would not fit its descriptor table; returns the grid, or 0 when the launch is not
-// one of these.
-inline int ws256_plan(RowsParams& p, int64_t out_rows, int64_t out_row_bytes) {
-  if (p.KD != kWsK || p.ND % 256 || !p.a_vec || !p.w_vec || !p.buf_ok || p.abs_max != nullptr) return 0;
-  if (out_rows * out_row_bytes >= (int64_t)kWsOutLimit || (int64_t)p.M * 4 >= (1LL << 31)) return 0;
-  p.n_col_blocks = p.ND / 256;
-  const long long blocks = (long long)p.M / kWsRows + p.E;                 // bound on the 32-row blocks
-  long long runs = 2LL * num_compute_units() / p.n_col_blocks;
-  if (runs < 1) runs = 1;
-  if (runs * kMaxDesc < blocks) runs = (blocks + kMaxDesc - 1) / kMaxDesc;
-  if (runs > blocks) runs = blocks;
-  return (int)(runs * p.n_col_blocks);
-}
-
-template <typename T>
-int launch_bwdx256(RowsParams p, const amoe_bwd_x_args* a, hipStream_t st, int* n_count_blocks, int* block_cols) {
-  if (!rows_all_interior(p, MODE_BWDX, kFBK)) return AMOE_EUNSUPPORTED;
-  if (!bwdx_reads_x(a) && a->ir == nullptr && a->gate == nullptr && p.out_stage) {
-    // a plain product with a contraction of 256: the weights stay in registers and the rows stream past them
-    RowsParams q = p;
-    if (const int grid = ws256_plan(q, a->M, a->ldo * 2)) {
-      hipLaunchKernelGGL((&ws256_kernel<T, true, 64, WS_PLAIN, false>), dim3(grid), dim3(kThreads), 0, st, q);
-      return launch_rc();
-    }
-  }
-  if (a->ir != nullptr && !a->ir_by_expert) return AMOE_EUNSUPPORTED;
-  if (a->x != nullptr && (!aligned(a->x, 16) || a->ldx % 8)) return AMOE_EUNSUPPORTED;   // 16-byte pieces of x rows
-  // With a short contraction an item is mostly its mask stage: 128-column tiles at three workgroups per CU then
-  // hide more of it (C3's up-projection, contraction 256: 0.197 vs 0.212 ms; at 512 the wide tile wins again).
-  const bool narrow = bwdx_reads_x(a) && a->N <= 256;
-  const int cols = narrow ? 128 : kFCols;
-  for (int t = 0; t < a->n_tiles; t++)
-    if ((a->tile_bounds[t + 1] - a->tile_bounds[t]) % cols) return AMOE_EUNSUPPORTED;
-  *block_cols = cols;
-  return narrow ? launch_bwdx256_cols<T, 128>(p, a, st, n_count_blocks)
-                : launch_bwdx256_cols<T, kFCols>(p, a, st, n_count_blocks);
-}
-
-template <typename T>
-int launch_fwd256(RowsParams p, int mode, const amoe_fwd_args* a, hipStream_t st) {
-  if (!rows_all_interior(p, mode, kFBK) || a->N % kFCols) return AMOE_EUNSUPPORTED;
-  if (a->noise != nullptr || a->n_tiles > 2) return AMOE_EUNSUPPORTED;
-  const bool dac = a->ir != nullptr;                 // (interior launches have the range and the quantiser, or neither)
-  if (dac && !a->ir_by_expert) return AMOE_EUNSUPPORTED;
-  const bool adc = a->out_bound > 0.f, noisy = a->noise_std > 0.f;
-  const bool analog = adc && a->out_res > 0.f && a->wmax_cols == 1 && dac;
-  if ((adc || noisy) && !analog) return AMOE_EUNSUPPORTED;
-  if (a->n_tiles == 2 && !(analog && !a->x_is_quantized)) return AMOE_EUNSUPPORTED;
-  // the two-K-tile variant parks the first tile's ADC codes as bytes (code + 128): a finer output quantiser than
-  // 254 states does not fit them, and the general kernel (fp32 partial results) serves the launch
-  if (a->n_tiles == 2 && !(p.out_half_states <= 127.f)) return AMOE_EUNSUPPORTED;
-  if (a->code_out && !analog) return AMOE_EUNSUPPORTED;
-  if (a->code_out && (!amoe_fwd_codes_supported(a) || !aligned(a->code_out, 16))) return AMOE_EUNSUPPORTED;
-  if (a->n_tiles == 1 && !a->relu && !a->xq_out && (a->x_is_quantized || !dac) && (a->code_out || !analog)) {
-    // one K-tile of 256, the operand plain or already coded, the result plain, rescaled or as ADC codes: the
-    // weights stay in registers and the rows stream past them
-    RowsParams q = p;
-    const int grid = a->code_out ? ws256_plan(q, a->n_out_rows, a->ldcode) : ws256_plan(q, a->n_out_rows, a->ldo * 2);
-    if (grid > 0) {
-      if (a->code_out) {
-        if (noisy) hipLaunchKernelGGL((&ws256_kernel<T, false, 64, WS_ZCODES, true>), dim3(grid), dim3(kThreads), 0, st, q);
-        else hipLaunchKernelGGL((&ws256_kernel<T, false, 64, WS_ZCODES, false>), dim3(grid), dim3(kThreads), 0, st, q);
-      } else if (dac) {
-        hipLaunchKernelGGL((&ws256_kernel<T, false, 64, WS_SCALE, false>), dim3(grid), dim3(kThreads), 0, st, q);
-      } else {
-        hipLaunchKernelGGL((&ws256_kernel<T, false, 64, WS_PLAIN, false>), dim3(grid), dim3(kThreads), 0, st, q);
-      }
-      return launch_rc();
-    }
-  }
-  p.n_col_blocks = a->N / kFCols;
-  const int grid = persistent_grid(max_row_tiles(a->M, a->E), p.n_col_blocks);
-  if (!dac) return launch_fwd256_as<T, FA_PLAIN, false, false, false>(p, grid, st);
-  if (!analog)
-    return a->x_is_quantized ? launch_fwd256_as<T, FA_CODES, false, false, false>(p, grid, st)
-                             : launch_fwd256_as<T, FA_DAC, false, false, false>(p, grid, st);
-  if (a->code_out) {
-    // codes leave instead of values: one output quantiser whose half range fits a byte, no second output
-    if (a->x_is_quantized)
-      return noisy ? launch_fwd256_as<T, FA_CODES, true, true, false, true>(p, grid, st)
-                   : launch_fwd256_as<T, FA_CODES, true, false, false, true>(p, grid, st);
-    return noisy ? launch_fwd256_as<T, FA_DAC, true, true, false, true>(p, grid, st)
-                 : launch_fwd256_as<T, FA_DAC, true, false, false, true>(p, grid, st);
-  }
-  if (a->x_is_quantized)
-    return noisy ? launch_fwd256_as<T, FA_CODES, true, true, false>(p, grid, st)
-                 : launch_fwd256_as<T, FA_CODES, true, false, false>(p, grid, st);
-  if (a->n_tiles == 2)
-    return noisy ? launch_fwd256_as<T, FA_DAC, true, true, true>(p, grid, st)
-                 : launch_fwd256_as<T, FA_DAC, true, false, true>(p, grid, st);
-  return noisy ? launch_fwd256_as<T, FA_DAC, true, true, false>(p, grid, st)
-               : launch_fwd256_as<T, FA_DAC, true, false, false>(p, grid, st);
-}
-
-}  // namespace
 
 extern "C" {
 
@@ -259,7 +32,8 @@ const char* amoe_strerror(int rc) {
 // ------------------------------------------------------------------------------ selection
 size_t amoe_prepare_sel_workspace(int64_t M, int32_t E) {
   if (M < 0 || E < 1) return 0;
-  const int64_t units = (M + sel_unit(M) - 1) / sel_unit(M);
+  const int64_t per = sel_by_groups(M, E) ? sel_span(M) : sel_unit(M);
+  const int64_t units = (M + per - 1) / per;
   return (size_t)(units > 0 ? units : 1) * (size_t)E * sizeof(int32_t);
 }
 
@@ -275,22 +49,30 @@ int amoe_prepare_sel(const void* sel, int32_t sel_is_i64, int64_t M, int32_t E, 
   if (workspace_bytes < amoe_prepare_sel_workspace(M, E)) return AMOE_EWORKSPACE;
   SelParams p;
   p.sel = sel; p.sel_is_i64 = sel_is_i64; p.M = M; p.E = E; p.k = k;
-  p.unit = sel_unit(M);
+  const bool by_groups = sel_by_groups(M, E);
+  p.unit = by_groups ? sel_span(M) : sel_unit(M);
   p.n_units = (int)((M + p.unit - 1) / p.unit);
   p.key_bits = 0;
   while ((1 << p.key_bits) < E) p.key_bits++;
   p.sel_sorted = sel_sorted; p.perm = perm; p.in_index = in_index; p.offsets = offsets;
   p.bad_flag = bad_flag; p.unit_hist = static_cast<int32_t*>(workspace);
+  p.table_vec = aligned(workspace, 16) && E % 4 == 0;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (by_groups) {
+    const int groups = p.n_units > 0 ? p.n_units : 1;        // (no elements: the offsets are still written)
+    if (M <= kSelSmall) {
+      hipLaunchKernelGGL((&sel_group_scatter_kernel<true>), dim3(groups), dim3(kThreads), 0, st, p);
+      return launch_rc();
+    }
+    hipLaunchKernelGGL(sel_group_hist_kernel, dim3(groups), dim3(kThreads), 0, st, p);
+    if (int rc = launch_rc()) return rc;
+    hipLaunchKernelGGL((&sel_group_scatter_kernel<false>), dim3(groups), dim3(kThreads), 0, st, p);
+    return launch_rc();
+  }
   const int blocks = (p.n_units + 3) / 4;
   if (blocks > 0) {
     hipLaunchKernelGGL(sel_hist_kernel, dim3(blocks), dim3(kThreads), 0, st, p);
     if (int rc = launch_rc()) return rc;
-  }
-  if (blocks > 0 && E <= kThreads && (long long)p.n_units * E <= kSelFuseMax && aligned(workspace, 16)) {
-    // a small table of unit counts: every workgroup of the scatter pass scans it for itself
-    hipLaunchKernelGGL(sel_scan_scatter_kernel, dim3(blocks), dim3(kThreads), 0, st, p);
-    return launch_rc();
   }
   hipLaunchKernelGGL(sel_unit_scan_kernel, dim3((E + 3) / 4), dim3(kThreads), 0, st, p);
   if (int rc = launch_rc()) return rc;
@@ -448,144 +230,12 @@ int amoe_cvmm_fwd(const amoe_fwd_args* a, void* stream) {
   const int mode = a->n_tiles > 1 ? MODE_FWD_SPLIT : MODE_FWD;
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (a->dtype != AMOE_F32 && !w_kc) {
-    const int rc = a->dtype == AMOE_F16 ? launch_fwd256<f16_t>(p, mode, a, st) : launch_fwd256<uint16_t>(p, mode, a, st);
+    const int rc = launch_fwd256(p, mode, a, st);
     if (rc != AMOE_EUNSUPPORTED) return rc;
   }
   if (a->code_out) return AMOE_EUNSUPPORTED;      // only the kernel above writes codes
   const int grid = persistent_grid(max_row_tiles(a->M, a->E), p.n_col_blocks);
-  if (a->dtype == AMOE_F32)
-    return w_kc ? launch_rows<float, true>(p, mode, grid, st) : launch_rows<float, false>(p, mode, grid, st);
-  if (a->dtype == AMOE_F16)
-    return w_kc ? launch_rows<f16_t, true>(p, mode, grid, st) : launch_rows<f16_t, false>(p, mode, grid, st);
-  return w_kc ? launch_rows<uint16_t, true>(p, mode, grid, st) : launch_rows<uint16_t, false>(p, mode, grid, st);
-}
-
-// ------------------------------------------------------------------------------ weight gradient
-namespace {
-// Rows per chunk of the weight gradient: enough (expert, chunk, tile) workgroups to fill the chip
-// twice over, chunks of 256 .. 4096 rows; 0 when one chunk per expert already does that.
-struct WgradSplit { int rows_per_chunk; long long slots; int tiles; };
-WgradSplit wgrad_split(const amoe_bwd_w_args* a) {
-  WgradSplit s{0, 0, 0};
-  const int kb = count_col_blocks(a->tile_bounds, a->n_tiles);
-  const int nb = (a->N + kTileCols - 1) / kTileCols;
-  s.tiles = kb * nb;
-  long long R;
-  if (a->rows_per_chunk > 0) {
-    R = ((long long)a->rows_per_chunk + 63) / 64 * 64;
-  } else {
-    const long long target = 4LL * num_compute_units();
-    const long long chunks = (target + s.tiles - 1) / s.tiles;
-    R = chunks > 0 ? (a->M + chunks - 1) / chunks : a->M;
-    R = (R + 255) / 256 * 256;
-    R = R < 256 ? 256 : (R > 4096 ? 4096 : R);
-  }
-  if (R >= a->M) return s;                 // a single chunk everywhere
-  s.rows_per_chunk = (int)R;
-  s.slots = 2LL * a->M / R + 1;            // bound on the chunks of the experts that are cut
-  return s;
-}
-}  // namespace
-
-size_t amoe_bwd_w_workspace(const amoe_bwd_w_args* a) {
-  if (!a || a->M < 1 || a->N < 1 || a->K < 1 || a->E < 1) return 0;
-  if (check_bounds(a->n_tiles, a->tile_bounds, a->K)) return 0;
-  const WgradSplit s = wgrad_split(a);
-  if (s.rows_per_chunk == 0) return 0;
-  return (size_t)s.slots * s.tiles * kWgradTileElems * sizeof(float);
-}
-
-int amoe_cvmm_bwd_w(const amoe_bwd_w_args* a, void* stream) {
-  if (!a) return AMOE_ENULL;
-  if (a->dtype != AMOE_F32 && a->dtype != AMOE_BF16 && a->dtype != AMOE_F16) return AMOE_EINVAL;
-  if (a->M < 0 || a->N < 1 || a->K < 1 || a->E < 1 || a->n_x_rows < 0 || a->n_g_rows < 0) return AMOE_EINVAL;
-  if (!a->grad_w || !a->offsets) return AMOE_ENULL;
-  if (a->M > 0 && (!a->x || !a->g || !a->in_index)) return AMOE_ENULL;
-  if (int rc = check_bounds(a->n_tiles, a->tile_bounds, a->K)) return rc;
-  if (a->M > 0 && (a->ldx < a->K || a->ldg < a->N)) return AMOE_ESHAPE;
-  const size_t es = esize(a->dtype);
-  if (!aligned(a->x, es) || !aligned(a->g, es) || !aligned(a->grad_w, es) || !aligned(a->offsets, 4) ||
-      !aligned(a->in_index, 4) || !aligned(a->g_index, 4) || !aligned(a->ir, 4) || !aligned(a->g_scale, es))
-    return AMOE_EALIGN;
-  const int CH = a->dtype == AMOE_F32 ? 4 : 8;
-  WgradParams p{};
-  p.M = a->M; p.N = a->N; p.K = a->K; p.E = a->E;
-  p.x = a->x; p.ldx = a->ldx; p.g = a->g; p.ldg = a->ldg; p.grad_w = a->grad_w;
-  p.offsets = a->offsets; p.in_index = a->in_index; p.g_index = a->g_index;
-  p.ir = a->ir; p.ir_by_expert = a->ir_by_expert; p.g_scale = a->g_scale; p.n_tiles = a->n_tiles;
-  for (int t = 0; t <= a->n_tiles; t++) p.bounds[t] = a->tile_bounds[t];
-  p.n_k_blocks = count_col_blocks(p.bounds, p.n_tiles);
-  p.n_n_blocks = (a->N + kTileCols - 1) / kTileCols;
-  p.x_vec = aligned(a->x, 16) && (a->ldx % CH == 0) && bounds_multiple_of(a->n_tiles, a->tile_bounds, CH);
-  p.g_vec = aligned(a->g, 16) && (a->ldg % CH == 0);
-  p.out_vec = aligned(a->grad_w, 16) && (a->N % 4 == 0);
-  p.out_stage = aligned(a->grad_w, 16) && (a->N % CH == 0);
-  p.buf_ok = a->n_x_rows > 0 && a->n_g_rows > 0 && a->n_x_rows * a->ldx * (long long)es < (1LL << 31) &&
-             a->n_g_rows * a->ldg * (long long)es < (1LL << 31);
-  hipStream_t st = static_cast<hipStream_t>(stream);
-  long long pairs = a->E;                  // (expert, chunk) pairs, worst case
-  if (a->workspace != nullptr && a->M > 0) {
-    const WgradSplit s = wgrad_split(a);
-    if (s.rows_per_chunk > 0) {
-      if (!aligned(a->workspace, 16)) return AMOE_EALIGN;
-      if (a->workspace_bytes < amoe_bwd_w_workspace(a)) return AMOE_EWORKSPACE;
-      if (a->E > kSelMaxExperts) return AMOE_EUNSUPPORTED;
-      p.rows_per_chunk = s.rows_per_chunk;
-      p.partial = static_cast<float*>(a->workspace);
-      pairs = a->M / s.rows_per_chunk + a->E;
-    }
-  }
-  const long long grid = 8LL * ((pairs + 7) / 8) * p.n_k_blocks * p.n_n_blocks;   // see the id mapping in the kernel
-  if (grid > 0x7fffffffLL) return AMOE_EUNSUPPORTED;
-  const long long rgrid = (long long)a->E * p.n_k_blocks * p.n_n_blocks * kWgradReduceSplit;
-  if (rgrid > 0x7fffffffLL) return AMOE_EUNSUPPORTED;
-  // the 256 x 256 kernel for the training shapes (16-bit elements, interior tiles, per-expert ranges)
-  bool wide = a->dtype != AMOE_F32 && p.x_vec && p.g_vec && p.out_stage && p.buf_ok && a->N % kW256Tile == 0 &&
-              (a->ir == nullptr || a->ir_by_expert);
-  for (int t = 0; t < a->n_tiles && wide; t++) wide = (a->tile_bounds[t + 1] - a->tile_bounds[t]) % kW256Tile == 0;
-  if (wide) {
-    const long long grid256 = 8LL * ((pairs + 7) / 8) * (p.n_k_blocks / 2) * (p.n_n_blocks / 2);
-    if (a->dtype == AMOE_BF16) {
-      hipLaunchKernelGGL((&wgrad256_kernel<uint16_t>), dim3((unsigned)grid256), dim3(kW256Threads), 0, st, p);
-    } else {
-      hipLaunchKernelGGL((&wgrad256_kernel<f16_t>), dim3((unsigned)grid256), dim3(kW256Threads), 0, st, p);
-    }
-    if (int rc = launch_rc()) return rc;
-    if (p.rows_per_chunk > 0) {
-      if (a->dtype == AMOE_BF16) {
-        hipLaunchKernelGGL((&wgrad_reduce_kernel<uint16_t>), dim3((unsigned)rgrid), dim3(kThreads), 0, st, p);
-      } else {
-        hipLaunchKernelGGL((&wgrad_reduce_kernel<f16_t>), dim3((unsigned)rgrid), dim3(kThreads), 0, st, p);
-      }
-    }
-    return launch_rc();
-  }
-  if (a->dtype == AMOE_F32) {
-    auto k = &gemm_wgrad_kernel<float>;
-    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kThreads), 0, st, p);
-    if (int rc = launch_rc()) return rc;
-    if (p.rows_per_chunk > 0) {
-      auto r = &wgrad_reduce_kernel<float>;
-      hipLaunchKernelGGL(r, dim3((unsigned)rgrid), dim3(kThreads), 0, st, p);
-    }
-  } else if (a->dtype == AMOE_BF16) {
-    auto k = &gemm_wgrad_kernel<uint16_t>;
-    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kThreads), 0, st, p);
-    if (int rc = launch_rc()) return rc;
-    if (p.rows_per_chunk > 0) {
-      auto r = &wgrad_reduce_kernel<uint16_t>;
-      hipLaunchKernelGGL(r, dim3((unsigned)rgrid), dim3(kThreads), 0, st, p);
-    }
-  } else {
-    auto k = &gemm_wgrad_kernel<f16_t>;
-    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kThreads), 0, st, p);
-    if (int rc = launch_rc()) return rc;
-    if (p.rows_per_chunk > 0) {
-      auto r = &wgrad_reduce_kernel<f16_t>;
-      hipLaunchKernelGGL(r, dim3((unsigned)rgrid), dim3(kThreads), 0, st, p);
-    }
-  }
-  return launch_rc();
+  return launch_rows(a->dtype, p, w_kc, mode, grid, st);
 }
 
 // ------------------------------------------------------------------------------ input gradient
@@ -651,14 +301,11 @@ int amoe_cvmm_bwd_x(const amoe_bwd_x_args* a, void* stream) {
   int rc = AMOE_EUNSUPPORTED;
   if (a->dtype != AMOE_F32) {
     int cols = kTileCols;
-    rc = a->dtype == AMOE_F16 ? launch_bwdx256<f16_t>(p, a, st, &n_count_blocks, &cols)
-                              : launch_bwdx256<uint16_t>(p, a, st, &n_count_blocks, &cols);
+    rc = launch_bwdx256(p, a, st, &n_count_blocks, &cols);
     if (rc == AMOE_OK) block_cols = cols;
   }
   if (rc == AMOE_EUNSUPPORTED)
-    rc = a->dtype == AMOE_F32   ? launch_rows<float, true>(p, MODE_BWDX, grid, st)
-         : a->dtype == AMOE_F16 ? launch_rows<f16_t, true>(p, MODE_BWDX, grid, st)
-                                : launch_rows<uint16_t, true>(p, MODE_BWDX, grid, st);
+    rc = launch_rows(a->dtype, p, true, MODE_BWDX, grid, st);
   if (rc) return rc;
   if (use_ir) {
     IrFinalizeParams f{};
@@ -1058,15 +705,15 @@ int amoe_segment_sum(const float* v, const int32_t* offsets, int32_t E, int32_t 
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (out_dtype == AMOE_F32) {
     auto kf = &segment_sum_kernel<float>;
-    hipLaunchKernelGGL(kf, grid, dim3(kThreads), 0, st, v, offsets, (int)n_tiles, static_cast<float*>(out),
+    hipLaunchKernelGGL(kf, grid, dim3(kSegThreads), 0, st, v, offsets, (int)n_tiles, static_cast<float*>(out),
                        (long long)ldout);
   } else if (out_dtype == AMOE_BF16) {
     auto kf = &segment_sum_kernel<uint16_t>;
-    hipLaunchKernelGGL(kf, grid, dim3(kThreads), 0, st, v, offsets, (int)n_tiles, static_cast<uint16_t*>(out),
+    hipLaunchKernelGGL(kf, grid, dim3(kSegThreads), 0, st, v, offsets, (int)n_tiles, static_cast<uint16_t*>(out),
                        (long long)ldout);
   } else {
     auto kf = &segment_sum_kernel<f16_t>;
-    hipLaunchKernelGGL(kf, grid, dim3(kThreads), 0, st, v, offsets, (int)n_tiles, static_cast<f16_t*>(out),
+    hipLaunchKernelGGL(kf, grid, dim3(kSegThreads), 0, st, v, offsets, (int)n_tiles, static_cast<f16_t*>(out),
                        (long long)ldout);
   }
   return launch_rc();
@@ -1327,3 +974,4 @@ int amoe_select_bwd(int32_t dtype, const void* logits, int64_t T, int32_t E, int
 }
 
 }  // extern "C"
+

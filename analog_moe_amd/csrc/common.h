@@ -40,8 +40,8 @@ __device__ __forceinline__ void unpack_f16x2(uint32_t w, float& lo, float& hi) {
   lo = v[0];
   hi = v[1];
 }
-template <typename T> constexpr bool kIsF16 = false;
-template <> constexpr bool kIsF16<f16_t> = true;
+template <typename T> inline constexpr bool kIsF16 = false;
+template <> inline constexpr bool kIsF16<f16_t> = true;
 // the 16 bits of one element, whatever its type
 template <typename T> __device__ __forceinline__ uint32_t elem_bits16(T v) {
   return (uint32_t)__builtin_bit_cast(uint16_t, v);

@@ -5,7 +5,7 @@
 //   pass 3  per wave: rank every element among equal keys of its 64-lane batch with a
 //           match-any built from ballots over the key bits, add the running per-key base kept
 //           in LDS, scatter (sorted id, flat index, flat index / k)
-// (small tables: passes 2 and 3 are one launch, sel_scan_scatter_kernel)
+// (up to 256 experts: two launches or one, sel_group_hist_kernel / sel_group_scatter_kernel)
 // Stable by construction: batches, units and lanes are all visited in ascending flat index.
 #pragma once
 #include "common.h"
@@ -25,6 +25,7 @@ struct SelParams {
   long long M; int E, k, n_units, key_bits, unit;
   int32_t* sel_sorted; int32_t* perm; int32_t* in_index; int32_t* offsets; int32_t* bad_flag;
   int32_t* unit_hist;               // workspace [n_units][E]
+  int table_vec;                    // its rows are on 16-byte pieces
 };
 
 __device__ __forceinline__ int sel_key(const SelParams& p, long long i, bool& bad) {
@@ -154,33 +155,100 @@ __global__ __launch_bounds__(kThreads) void sel_scatter_kernel(const SelParams p
   }
 }
 
-// Passes 2 and 3 in one launch, for tables small enough that every workgroup can afford to read all of it
-// (n_units * E <= kSelFuseMax counts, E <= kThreads): each workgroup sums the whole table of unit counts itself --
-// per expert: the total, and the part that belongs to the units before its own four -- scans the totals into the
-// experts' segment starts, and scatters its units as sel_scatter_kernel does.  Workgroup 0 also writes offsets.
-// Two launches and no pass over the table in between: the sort is on the path to the first GEMM of every step.
-constexpr int kSelFuseMax = 32768;
-__global__ __launch_bounds__(kThreads) void sel_scan_scatter_kernel(const SelParams p) {
+// ---- the same sort with at most kThreads experts --------------------------------------------------------------
+// A group is `span` consecutive elements, one workgroup, a quarter per wave.  Two launches: the groups' histograms as a
+// table [n_groups][E], then every workgroup sums the whole table for itself (per expert: the total, and the part of the
+// groups before its own), scans the totals into the experts' segment starts, counts its own waves' keys again in LDS
+// and scatters.  Up to kSelSmall elements the second launch counts the keys themselves instead of a table and is the
+// only one.  The sort is on the path to the first GEMM of every step, so what matters is the number of launches and
+// the length of the dependent chain inside them, not the bytes.
+//   Span: the smallest that leaves at most kSelGroups groups, so that the table every workgroup reads stays at or
+//   below 128 KB.  One table row per wave, as the general path has it, is a table four times as large, and at 131 072
+//   elements and 128 experts it was too large for every workgroup to read: 19.4 us there and 19.0 at 64 experts,
+//   12.8 and 11.4 us as it is now (back to back in a graph).
+//   kSelSmall: one launch that counts all keys takes 3.3 us at 8 elements, 4.0 at 512 (two launches: 5.9, 8.1) and grows
+//   by 0.8 us per 1024 elements; two launches take 7 us from there on.
+constexpr int kSelSmall = 4096;
+constexpr int kSelGroups = 128;
+constexpr int kSelSpanMax = 16384;
+__host__ __device__ inline int sel_span(long long M) {
+  int s = kThreads;
+  if (M > kSelSmall)
+    while (s < kSelSpanMax && (M + s - 1) / s > kSelGroups) s <<= 1;
+  return s;
+}
+__host__ __device__ inline bool sel_by_groups(long long M, int E) {
+  return E <= kThreads && (M + sel_span(M) - 1) / sel_span(M) <= kSelGroups;
+}
+
+// counts of n keys from `first` into hist (LDS, zeroed), eight loads in flight per thread; true: an id out of range
+__device__ __forceinline__ bool sel_count(const SelParams& p, long long first, long long n, int* hist) {
+  bool any_bad = false;
+  for (long long i0 = threadIdx.x; i0 < n; i0 += 8 * kThreads) {
+    int key[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const long long i = i0 + j * kThreads;
+      bool bad = false;
+      key[j] = i < n ? sel_key(p, first + i, bad) : -1;
+      any_bad |= bad;
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+      if (key[j] >= 0) atomicAdd(&hist[key[j]], 1);
+  }
+  return any_bad;
+}
+
+__global__ __launch_bounds__(kThreads) void sel_group_hist_kernel(const SelParams p) {
+  __shared__ int hist[kThreads];
+  const int tid = threadIdx.x;
+  hist[tid] = 0;
+  __syncthreads();
+  const long long first = (long long)blockIdx.x * p.unit;
+  const long long n = p.M - first < p.unit ? p.M - first : p.unit;
+  const bool any_bad = sel_count(p, first, n, hist);
+  if (any_bad && p.bad_flag != nullptr) atomicOr(p.bad_flag, 1);
+  __syncthreads();
+  if (tid < p.E) p.unit_hist[(long long)blockIdx.x * p.E + tid] = hist[tid];
+}
+
+template <bool SMALL>
+__global__ __launch_bounds__(kThreads) void sel_group_scatter_kernel(const SelParams p) {
   __shared__ int base[4 * kThreads];          // [wave][expert]: where the next element of that expert goes
   __shared__ __attribute__((aligned(16))) int part_total[4 * kThreads], part_before[4 * kThreads];
   __shared__ int wave_sums[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int E = p.E;
-  const int first_unit = blockIdx.x * 4;
-  // per expert: the total over all units and the part before this workgroup's first unit.  The table is read in rows
-  // (one unit's counts), several rows per pass of the workgroup, four experts per thread where E allows it.
+  const int E = p.E, group = blockIdx.x;
+  const long long first = (long long)group * p.unit;      // this workgroup's elements
+  const int per_wave = p.unit / 4;
+#pragma unroll
+  for (int w = 0; w < 4; w++) base[w * kThreads + tid] = 0;
   int my_total = 0, my_before = 0;                  // thread e < E: the expert's two sums
-  if ((E & 3) == 0) {
+  if constexpr (SMALL) {
+    part_before[tid] = part_total[tid] = 0;
+    __syncthreads();
+    bool bad = sel_count(p, 0, first < p.M ? first : p.M, part_before);
+    bad |= sel_count(p, first, p.M - first, part_total);
+    if (bad && group == 0 && p.bad_flag != nullptr) atomicOr(p.bad_flag, 1);
+    __syncthreads();
+    if (tid < E) {
+      my_before = part_before[tid];
+      my_total = my_before + part_total[tid];
+    }
+  } else if (p.table_vec) {
+    // the table in rows (one group's counts), several rows per pass of the workgroup, four experts per thread
     typedef __attribute__((ext_vector_type(4))) int i32x4v;
     const int tpr = E >> 2;                         // threads per row (<= 64)
     const int rpp = kThreads / tpr;                 // rows per pass
     const int c4 = tid % tpr, row = tid / tpr;
     i32x4v tot = {0, 0, 0, 0}, bef = {0, 0, 0, 0};
     if (row < rpp) {
+#pragma unroll 4
       for (int u = row; u < p.n_units; u += rpp) {
         const i32x4v c = *reinterpret_cast<const i32x4v*>(p.unit_hist + (long long)u * E + 4 * c4);
         tot += c;
-        if (u < first_unit) bef += c;
+        if (u < group) bef += c;
       }
       *reinterpret_cast<i32x4v*>(&part_total[row * E + 4 * c4]) = tot;
       *reinterpret_cast<i32x4v*>(&part_before[row * E + 4 * c4]) = bef;
@@ -201,7 +269,7 @@ __global__ __launch_bounds__(kThreads) void sel_scan_scatter_kernel(const SelPar
       for (int u = grp; u < p.n_units; u += groups) {
         const int c = p.unit_hist[(long long)u * E + e];
         total += c;
-        before += u < first_unit ? c : 0;
+        before += u < group ? c : 0;
       }
     }
     part_total[tid] = total;
@@ -212,6 +280,12 @@ __global__ __launch_bounds__(kThreads) void sel_scan_scatter_kernel(const SelPar
         my_total += part_total[g * epad + tid];
         my_before += part_before[g * epad + tid];
       }
+  }
+  // the waves' own counts (base was cleared before the barriers above)
+  for (int it = 0; it < per_wave; it += 64) {
+    const long long i = first + (long long)wave * per_wave + it + lane;
+    bool bad;
+    if (i < p.M) atomicAdd(&base[wave * kThreads + sel_key(p, i, bad)], 1);
   }
   // exclusive scan of the totals over the experts (thread = expert)
   int incl = my_total;
@@ -225,24 +299,24 @@ __global__ __launch_bounds__(kThreads) void sel_scan_scatter_kernel(const SelPar
   int start = incl - my_total;
   for (int w = 0; w < wave; w++) start += wave_sums[w];
   if (tid < E) {
-    if (blockIdx.x == 0) {
+    if (group == 0) {
       p.offsets[tid] = start;
       if (tid == E - 1) p.offsets[E] = (int)p.M;
     }
     int run = start + my_before;
+#pragma unroll
     for (int w = 0; w < 4; w++) {
+      const int c = base[w * kThreads + tid];
       base[w * kThreads + tid] = run;
-      const int u = first_unit + w;
-      if (u < p.n_units) run += p.unit_hist[(long long)u * E + tid];
+      run += c;
     }
   }
   __syncthreads();
-  const int unit = first_unit + wave;
   int* my_base = &base[wave * kThreads];
   const uint64_t lt_mask = ((uint64_t)1 << lane) - 1;
-  for (int it = 0; it < p.unit / 64; it++) {
-    const long long i = (long long)unit * p.unit + it * 64 + lane;
-    const bool valid = unit < p.n_units && i < p.M;
+  for (int it = 0; it < per_wave; it += 64) {
+    const long long i = first + (long long)wave * per_wave + it + lane;
+    const bool valid = i < p.M;
     bool bad;
     const int key = valid ? sel_key(p, i, bad) : 0;
     uint64_t same = wave_ballot(valid);
@@ -261,7 +335,7 @@ __global__ __launch_bounds__(kThreads) void sel_scan_scatter_kernel(const SelPar
     if (valid) {
       p.sel_sorted[pos] = key;
       p.perm[pos] = (int)i;
-      p.in_index[pos] = (int)(i / p.k);
+      p.in_index[pos] = (int)((uint32_t)i / (uint32_t)p.k);
     }
   }
 }

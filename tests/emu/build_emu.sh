@@ -5,11 +5,25 @@ set -e
 here="$(cd "$(dirname "$0")" && pwd)"
 root="$(cd "$here/../.." && pwd)"
 CXX=/opt/rocm/llvm/bin/clang++
-flags="-x c++ -std=c++20 -O1 -g -fPIC -shared -pthread -Wno-psabi -I $here -I $root/include -I $root/analog_moe_amd/csrc"
+flags="-x c++ -std=c++20 -O1 -g -fPIC -pthread -Wno-psabi -I $here -I $root/include -I $root/analog_moe_amd/csrc"
+link="-shared -fPIC -pthread"
 out="$here/libamoe_emu.so"
 if [ "$1" = "asan" ]; then
   flags="$flags -fsanitize=address,undefined -fno-omit-frame-pointer -shared-libasan"
+  link="$link -fsanitize=address,undefined -shared-libasan"
   out="$here/libamoe_emu_asan.so"
 fi
-$CXX $flags "$root/analog_moe_amd/csrc/amoe.hip" -o "$out"
+objdir="$here/build${1:+_$1}"
+mkdir -p "$objdir"
+# one translation unit per source file, compiled side by side
+pids=""
+objs=""
+for src in "$root"/analog_moe_amd/csrc/*.hip; do
+  obj="$objdir/$(basename "$src" .hip).o"
+  objs="$objs $obj"
+  $CXX $flags -c "$src" -o "$obj" &
+  pids="$pids $!"
+done
+for pid in $pids; do wait "$pid"; done
+$CXX $link $objs -o "$out"
 echo "$out"

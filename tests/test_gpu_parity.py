@@ -318,3 +318,29 @@ def test_golden_fixture_parity(ops, name):
     # inherits it: the quantised stages are compared with the step allowance, what follows with a wider tolerance
     errs = util.compare_layer(got, want, 1e-4, adc_step=adc)
     print(errs)
+
+
+@pytest.mark.parametrize("M,E,k", [(1, 1, 1), (255, 3, 1), (4096, 256, 8), (4097, 5, 1), (8200, 256, 4),
+                                   (131072, 128, 4), (262144, 255, 8), (2 ** 21 + 7, 7, 1), (9000, 257, 4)])
+@pytest.mark.parametrize("dt", [torch.int32, torch.int64])
+def test_prepare_sel_at_the_edges_of_its_paths(ops, M, E, k, dt):
+    """One launch up to 4096 elements, two beyond, the general passes beyond 256 experts or 2^21 elements."""
+    rng = np.random.default_rng(M + E)
+    p = np.arange(1, E + 1) ** -1.2
+    sel = rng.choice(E, size=M, p=p / p.sum())
+    got = ops.prepare_sel(torch.from_numpy(sel).to(dt).cuda(), E, k)
+    want = O.prepare_sel(sel, E, k)
+    for g, w in zip(got, (want.sel_sorted, want.perm, want.in_index, want.offsets)):
+        assert np.array_equal(g.cpu().numpy(), w)
+
+
+@pytest.mark.parametrize("rows", [0, 1, 1023, 1024, 8193, 20001])
+def test_segment_sum_of_long_segments(ops, rows):
+    """One expert with `rows` rows beside short ones; fp32 sums of n values are within n * 2^-24 of the sum of |v|."""
+    off = np.array([0, 3, 3 + rows, 3 + rows, 10 + rows], dtype=np.int32)
+    v = np.random.default_rng(rows).standard_normal((int(off[-1]), 2)).astype(np.float32)
+    got = ops.segment_sum(torch.from_numpy(v).cuda(), torch.from_numpy(off).cuda(), 4).cpu().numpy()
+    for e in range(4):
+        part = v[off[e]:off[e + 1]].astype(np.float64)
+        bound = (len(part) + 1) * 2.0 ** -24 * np.abs(part).sum(0)
+        assert np.all(np.abs(got[e] - part.sum(0)) <= bound)
