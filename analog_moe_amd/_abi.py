@@ -6,6 +6,8 @@ integers (``tensor.data_ptr()``), NULL as 0/None.
 from __future__ import annotations
 
 import ctypes as C
+import functools
+import struct
 
 AMOE_MAX_TILES = 16
 AMOE_F32, AMOE_BF16, AMOE_F16 = 0, 1, 2
@@ -106,10 +108,35 @@ PROTOTYPES = {
     "amoe_weight_std_workspace": (SZ, [I32, I32, I32, I32]),
     "amoe_weight_std": (C.c_int, [I32, P, I32, I32, I32, I32, P, P, SZ, P]),
     "amoe_clamp_weights": (C.c_int, [I32, P, I32, I32, I32, P, I32, P]),
+    "amoe_ffn_args_bytes": (SZ, []),
+    "amoe_ffn_fwd_workspace": (SZ, [P]),
+    "amoe_ffn_bwd_workspace": (SZ, [P]),
+    "amoe_ffn_fwd": (C.c_int, [P, P, SZ, P, P]),
+    "amoe_ffn_bwd": (C.c_int, [P, P, SZ, P, P]),
+    "amoe_ffn_stage_name": (C.c_char_p, [I32, I32]),
     "amoe_select_workspace": (SZ, [I64, I32]),
     "amoe_select_fwd": (C.c_int, [I32, P, I64, I32, I32, P, P, P, P, P, SZ, P]),
     "amoe_select_bwd": (C.c_int, [I32, P, I64, I32, I32, P, P, P, P, P, P]),
 }
+
+
+# amoe_ffn_args: 8-byte fields in the header's order, packed in one call and handed over as bytes
+FFN_ARGS = struct.Struct("<"
+                         "7q"          # dtype T D E F V k
+                         "2q4q4q"      # x ldx, keys + 3 strides, values + 3 strides
+                         "3q2qq"       # input_range ir_dtype ir_cols, sel sel_is_i64, gate
+                         "4d"          # inp_res out_bound out_res noise_std
+                         "4qQ2q"       # n_up bounds_up n_dn bounds_dn, noise_seed, noise_seed_dev noise_per_channel
+                         "4q2q"        # noise_up noise_dn wmax_up wmax_dn, seed_bump down_ready
+                         "10q"         # y p1 z z_is_codes z_scale perm in_index offsets ir_up ir_dn
+                         "6qq3d"       # dy grad_x grad_keys grad_values grad_gate grad_ir, gradient_relative, 3 scalars
+                         "q")          # stage_events
+
+
+@functools.lru_cache(maxsize=256)
+def bounds_array(bounds):
+    """A tuple of K-tile bounds as a C array (kept: callers pass its address)."""
+    return (C.c_int32 * len(bounds))(*bounds)
 
 
 def bind(path: str) -> C.CDLL:
@@ -119,6 +146,8 @@ def bind(path: str) -> C.CDLL:
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+    if lib.amoe_ffn_args_bytes() != FFN_ARGS.size:
+        raise RuntimeError(f"{path}: amoe_ffn_args has another layout than this package packs")
     return lib
 
 

@@ -8,12 +8,13 @@ and the noise draw into the epilogue.
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
-from typing import Optional, Sequence
+from typing import Callable, Optional, Sequence
 
 import torch
 
-from . import ops
+from . import _abi, ops, raw
 
 
 @dataclass
@@ -40,17 +41,8 @@ class FFNConfig:
     down_ready: Optional["torch.cuda.Event"] = None  # the down-projection's weights and wmax_down are made on another
                                                   # stream: the current one waits for this event before it reads them
                                                   # (eager calls only, as seed_bump)
-
-
-_SIDE_STREAMS = {}
-
-
-def _side_stream(device: torch.device) -> "torch.cuda.Stream":
-    """One extra stream per device (default priority), for the bandwidth-bound companions."""
-    key = torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device()
-    if key not in _SIDE_STREAMS:
-        _SIDE_STREAMS[key] = torch.cuda.Stream(device=key)
-    return _SIDE_STREAMS[key]
+    stage_events: Optional[Callable[[bool], int]] = None  # profiling: address of the hipEvent_t pairs recorded around the
+                                                  # stages of a direction (argument: backward); eager calls only
 
 
 CFG_FIELDS = ("inp_res", "bounds_up", "bounds_down", "out_bound", "out_res", "noise_std", "noise_seed",
@@ -75,68 +67,93 @@ def ir_tables(input_range: Optional[torch.Tensor], E: int, cfg: FFNConfig):
     return ir3[0, :, :_n_tiles(cfg.bounds_up)].contiguous(), ir3[1, :, :_n_tiles(cfg.bounds_down)].contiguous()
 
 
+def _p(t: Optional[torch.Tensor]) -> int:
+    return 0 if t is None else t.data_ptr()
+
+
+def _dense(t: torch.Tensor) -> torch.Tensor:
+    t = t.detach()
+    return t if t.is_contiguous() else t.contiguous()
+
+
+def _bounds(bounds, K: int):
+    b = (0, K) if bounds is None else tuple(bounds)
+    if not 2 <= len(b) <= _abi.AMOE_MAX_TILES + 1:
+        raise ValueError(f"number of K-tiles must be in [1, {_abi.AMOE_MAX_TILES}]")
+    return len(b) - 1, ctypes.addressof(_abi.bounds_array(b))
+
+
+def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype, sel, gate, y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn,
+          grads=(0, 0, 0, 0, 0, 0)) -> bytes:
+    """The argument structure of ``amoe_ffn_fwd`` / ``amoe_ffn_bwd``.  All tensors rows-contiguous, x [T, D]."""
+    E, D, F = keys.shape
+    V = values.shape[2]
+    for t in (cfg.noise_up, cfg.noise_down, cfg.wmax_up, cfg.wmax_down):
+        if t is not None and (t.dtype != torch.float32 or not t.is_contiguous()):
+            raise TypeError("injected noise and max |W| tables must be contiguous float32 tensors")
+    if keys.dtype != x.dtype or values.dtype != x.dtype or gate.dtype != x.dtype:
+        raise TypeError("x, keys, values and gate must share one dtype")
+    if x.shape[1] != D or values.shape[0] != E or values.shape[1] != F:
+        raise ValueError("x / keys / values shapes do not match")
+    if x.dtype != torch.float32 and cfg.inp_res > 0:
+        raw.check_codes_fit(x.dtype, cfg.inp_res)
+    return _abi.FFN_ARGS.pack(
+        raw.dtype_code(x), x.shape[0], D, E, F, V, gate.shape[-1],
+        x.data_ptr(), x.stride(0), keys.data_ptr(), *keys.stride(), values.data_ptr(), *values.stride(),
+        _p(input_range), raw.DTYPE_CODES.get(ir_dtype, 0), 0 if input_range is None else input_range.numel() // (2 * E), sel.data_ptr(), sel.dtype == torch.int64, gate.data_ptr(),
+        cfg.inp_res, cfg.out_bound, cfg.out_res, cfg.noise_std,
+        *_bounds(cfg.bounds_up, D), *_bounds(cfg.bounds_down, F), cfg.noise_seed & 0xFFFFFFFFFFFFFFFF, _p(cfg.noise_seed_dev),
+        cfg.noise_per_channel, _p(cfg.noise_up), _p(cfg.noise_down), _p(cfg.wmax_up), _p(cfg.wmax_down),
+        cfg.seed_bump if cfg.noise_seed_dev is not None else 0, 0 if cfg.down_ready is None else cfg.down_ready.cuda_event,
+        _p(y), p1.data_ptr(), z.data_ptr(), z.dtype == torch.uint8, _p(z_scale), perm.data_ptr(), in_index.data_ptr(),
+        offsets.data_ptr(), _p(ir_up), _p(ir_dn),
+        *grads, cfg.gradient_relative, cfg.gradient_scale, cfg.decay, cfg.input_min_percentage,
+        0 if cfg.stage_events is None else cfg.stage_events(backward))
+
+
+def _int_ids(sel_idx: torch.Tensor) -> torch.Tensor:
+    sel = sel_idx.detach()
+    if sel.dtype not in (torch.int32, torch.int64):
+        sel = sel.to(torch.int64)
+    return sel if sel.is_contiguous() else sel.contiguous()
+
+
 def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
-    """Sort, both projections and the gate reduction.  Returns (y, p1, z, perm, in_index, offsets, z_scale, ir_up,
-    ir_dn): the result and what the backward pass reads again.  z is the down-projection's k-head result
+    """Sort, both projections and the gate reduction (``amoe_ffn_fwd``).  Returns (y, p1, z, perm, in_index, offsets,
+    z_scale, ir_up, ir_dn): the result and what the backward pass reads again.  z is the down-projection's k-head result
     [T*k, D], either as values (z_scale empty) or as uint8 ADC codes with z_scale [E, 2] (``ops.dequant_codes``)."""
-    T, D = x.shape
-    E, _, F = keys.shape
-    k = sel_idx.shape[-1]
+    ops._need_gpu(x, keys, values, input_range, gate, sel_idx)
+    lib = ops.get_lib()
+    x, keys, values, gate = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(gate)
+    sel = _int_ids(sel_idx)
+    dev, dt = x.device, x.dtype
+    (E, D, F), V = keys.shape, values.shape[2]
+    T, k = x.shape[0], sel.shape[-1]
     M = T * k
-    gen = cfg.noise_std > 0 and cfg.noise_up is None
-    wu = wd = ir_up = ir_dn = None
-    main = torch.cuda.current_stream()
-    if cfg.wmax_up is not None:
-        wu, wd = cfg.wmax_up, cfg.wmax_down
-        ir_up, ir_dn = ir_tables(input_range, E, cfg)
-    elif cfg.out_bound > 0 or gen:
-        # max |W| per expert and the fp32 input-range tables only read parameters: they run next to the expert
-        # sort on a second stream
-        side = _side_stream(x.device)
-        side.wait_stream(main)
-        with torch.cuda.stream(side):
-            if cfg.noise_per_channel:
-                ir_up, ir_dn = ir_tables(input_range, E, cfg)
-                wu = ops.weight_abs_max(keys, True)
-                wd = ops.weight_abs_max(values, True)
-            elif input_range is None:
-                wu, wd = ops.weight_abs_max_pair(keys, values)
-            else:                                # both max |W| tables and both fp32 range tables from two launches
-                wu, wd, ir_up, ir_dn = ops.layer_tables(keys, values, input_range.reshape(2, E, -1),
-                                                        _n_tiles(cfg.bounds_up), _n_tiles(cfg.bounds_down))
-        for t in (wu, wd, ir_up, ir_dn):
-            if t is not None:
-                t.record_stream(main)
-    else:
-        ir_up, ir_dn = ir_tables(input_range, E, cfg)
-    sel_sorted, perm, in_index, offsets = ops.prepare_sel(sel_idx, E, k)
-    if wu is not None and cfg.wmax_up is None:
-        main.wait_stream(side)
-    common = dict(inp_res=cfg.inp_res, out_bound=cfg.out_bound, out_res=cfg.out_res,
-                  noise_std=cfg.noise_std if gen else 0.0, ir_by_expert=ir_up is not None)
-    # the up-projection also emits the down-projection's DAC image of its result (each row belongs
-    # to one expert, so the image is made once instead of once per block of output columns)
-    chain = ir_dn is not None and cfg.inp_res > 0 and _n_tiles(cfg.bounds_down) == 1
-    p1 = ops.cvmm_fwd(x, keys, sel_sorted, offsets, in_index, perm, M, ir=ir_up, bounds=cfg.bounds_up,
-                      noise=cfg.noise_up, noise_seed=cfg.noise_seed, wmax=wu, relu=True,
-                      noise_seed_dev=cfg.noise_seed_dev, xq_ir=ir_dn[:, 0].contiguous() if chain else None,
-                      xq_inp_res=cfg.inp_res, **common)
-    p1, p1q = p1 if chain else (p1, None)
-    if cfg.down_ready is not None:
-        main.wait_event(cfg.down_ready)
-    down = dict(ir=ir_dn, bounds=cfg.bounds_down, noise=cfg.noise_down, noise_seed=cfg.noise_seed + 1, wmax=wd,
-                noise_seed_dev=cfg.noise_seed_dev, x_is_quantized=chain, **common)
-    # the gate reduction follows the last launch that draws noise: it moves the device seed word on
-    bump = (cfg.noise_seed_dev, cfg.seed_bump) if cfg.seed_bump and cfg.noise_seed_dev is not None else ()
-    if chain and z_as_codes(p1q, values, cfg):
-        # the down-projection's result is read twice more and never as a matrix operand (gate reduction now, gate
-        # gradient in the backward pass): it is kept as its ADC codes, one byte per value, with two factors per expert
-        z, z_scale = ops.cvmm_fwd(p1q, values, sel_sorted, offsets, perm, None, M, want_codes=True, **down)
-        y = ops.gate_reduce_codes(z, z_scale, sel_idx, gate, *bump)
-    else:
-        z = ops.cvmm_fwd(p1q if chain else p1, values, sel_sorted, offsets, perm, None, M, **down)
-        z_scale = torch.empty(0, dtype=torch.float32, device=x.device)
-        y = ops.gate_reduce(z, gate, *bump)
+    if sel.numel() != M or gate.numel() != M:
+        raise ValueError("sel_idx and gate must hold k values per token")
+    y, p1 = x.new_empty((T, V)), x.new_empty((M, F))
+    perm, in_index = (torch.empty(M, dtype=torch.int32, device=dev) for _ in range(2))
+    offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
+    ir_up = ir_dn = None
+    if input_range is not None:
+        input_range = _dense(input_range)
+        ir_up, ir_dn = (torch.empty((E, _n_tiles(b)), dtype=torch.float32, device=dev)
+                        for b in (cfg.bounds_up, cfg.bounds_down))
+    chain = input_range is not None and cfg.inp_res > 0 and _n_tiles(cfg.bounds_down) == 1
+    codes = chain and z_as_codes(p1, values, cfg)
+    z = torch.empty((M, V), dtype=torch.uint8 if codes else dt, device=dev)
+    z_scale = torch.empty((E, 2) if codes else 0, dtype=torch.float32, device=dev)
+    if M == 0:                                       # no tokens: nothing to launch but the step counter
+        if cfg.seed_bump and cfg.noise_seed_dev is not None:
+            cfg.noise_seed_dev.add_(cfg.seed_bump)
+        if input_range is not None:
+            ir_up, ir_dn = ir_tables(input_range, E, cfg)
+        return y, p1, z, perm, in_index, offsets.zero_(), z_scale, ir_up, ir_dn
+    args = _pack(cfg, False, x, keys, values, input_range, None if input_range is None else input_range.dtype, sel, gate,
+                 y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn)
+    ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8, device=dev)
+    _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_fwd")
     return y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn
 
 
@@ -149,62 +166,29 @@ def z_as_codes(p1q: torch.Tensor, values: torch.Tensor, cfg: FFNConfig) -> bool:
 
 def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn,
                  cfg: FFNConfig, want_ir_grad: bool, ir_dtype: torch.dtype = torch.float32):
-    """Returns (grad_x, grad_keys, grad_values, grad_ir [2, E, n_tiles] of type ir_dtype or None, grad_gate)."""
+    """Returns (grad_x, grad_keys, grad_values, grad_ir [2, E, n_tiles] of type ir_dtype or None, grad_gate)
+    (``amoe_ffn_bwd``)."""
+    lib = ops.get_lib()
+    x, keys, values, dy = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(dy)
+    gate_c, sel = _dense(gate), _int_ids(sel_idx)
     E = keys.shape[0]
-    k = gate.shape[-1]
-    M = perm.numel()
-    dy = dy.contiguous()
-    by = dict(ir_by_expert=ir_up is not None)
-    irkw = dict(gradient_relative=cfg.gradient_relative, gradient_scale=cfg.gradient_scale, decay=cfg.decay,
-                input_min_percentage=cfg.input_min_percentage)
-    tok = in_index                               # token of each sorted position: perm // k, as the sort left it
-    # the input gradient reads p1 for its masks anyway; it also leaves gate * clamp(p1), which is the
-    # x operand of the weight gradient (otherwise every block of its output columns clips and scales)
-    gp1, irg_dn, p1c = ops.cvmm_bwd_x(dy, values, offsets, tok, perm, M, x=p1, xf_index=perm, gate=gate,
-                                      ir=ir_dn, bounds=cfg.bounds_down, relu_mask=True, want_xc=True,
-                                      **irkw, **by)
-    # the clip mask of the up-projection's input gradient depends on the token's input row, which its k heads
-    # share: where the sum over the heads can apply it, the GEMM runs without a mask tile and x is read once per
-    # token instead of once per head
-    late_clip = ir_up is not None and ops.ksum_clip_supported(x, k, cfg.bounds_up)
-    if late_clip:
-        full, irg_up = ops.cvmm_bwd_x(gp1, keys, offsets, perm, perm, M)
-    else:
-        full, irg_up = ops.cvmm_bwd_x(gp1, keys, offsets, perm, perm, M, x=x, xf_index=in_index, ir=ir_up,
-                                      bounds=cfg.bounds_up, **irkw, **by)
-    # the gate gradient and the sum over the k heads only stream z, dy and the per-head input gradient
-    # through HBM; they run on a second stream next to the two weight gradients.  With evenly loaded experts the
-    # four launches take as long side by side as one after the other (together they are bound by memory traffic);
-    # with uneven loads the streaming kernels fill the CUs that the weight gradients' last tiles leave idle
-    # (2 - 3 % of the step)
-    main, side = torch.cuda.current_stream(), _side_stream(x.device)
-    side.wait_stream(main)
-    with torch.cuda.stream(side):
-        if z.dtype == torch.uint8:
-            grad_gate = ops.gate_grad_codes(z, z_scale, sel_idx, dy, k).view(gate.shape)
-        else:
-            grad_gate = ops.gate_grad(z, dy, k).view(gate.shape)
-        if late_clip:
-            grad_x, irg_up = ops.ksum_clip(full, x, sel_idx, perm, offsets, ir_up, k, bounds=cfg.bounds_up, **irkw)
-            irg_up.record_stream(main)
-        else:
-            grad_x = ops.ksum(full, k) if k > 1 else full
-    grad_gate.record_stream(main)
-    grad_x.record_stream(main)
+    grad_x = x.new_empty(x.shape)
+    grad_keys, grad_values, grad_gate = torch.empty_like(keys), torch.empty_like(values), torch.empty_like(gate_c)
     grad_ir = None
     if ir_up is not None and want_ir_grad:
-        ntu, ntd = ir_up.shape[1], ir_dn.shape[1]
-        # the two tables of per-expert sums are written where they belong, in the parameter's type, and each launch
-        # clears the columns its projection does not have.  The down-projection's sums are issued here, where the
-        # second stream keeps the GPU busy, instead of after the join at the end of the step
-        nt = max(ntu, ntd)
-        grad_ir = torch.empty((2, E, nt), dtype=ir_dtype, device=x.device)
-        ops.segment_sum(irg_dn, offsets, E, out=grad_ir[1, :, :ntd], zero_cols=nt - ntd)
-    grad_values = ops.cvmm_bwd_w(p1c, dy, E, offsets, perm, tok)
-    grad_keys = ops.cvmm_bwd_w(x, gp1, E, offsets, in_index, perm, ir=ir_up, bounds=cfg.bounds_up, **by)
-    main.wait_stream(side)
-    if grad_ir is not None:
-        ops.segment_sum(irg_up, offsets, E, out=grad_ir[0, :, :ntu], zero_cols=nt - ntu)
+        grad_ir = torch.empty((2, E, max(ir_up.shape[1], ir_dn.shape[1])), dtype=ir_dtype, device=x.device)
+    if perm.numel() == 0:
+        for g in (grad_x, grad_keys, grad_values, grad_gate, grad_ir):
+            if g is not None:
+                g.zero_()
+        return grad_x, grad_keys, grad_values, grad_ir, grad_gate
+    if dy.dtype != x.dtype:
+        raise TypeError("dy and x must share one dtype")
+    args = _pack(cfg, True, x, keys, values, None, ir_dtype, sel, gate_c, None, p1, z, z_scale, perm, in_index, offsets,
+                 ir_up, ir_dn, (dy.data_ptr(), grad_x.data_ptr(), grad_keys.data_ptr(), grad_values.data_ptr(),
+                                grad_gate.data_ptr(), _p(grad_ir)))
+    ws = torch.empty(lib.amoe_ffn_bwd_workspace(args), dtype=torch.uint8, device=x.device)
+    _abi.check(lib, lib.amoe_ffn_bwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_bwd")
     return grad_x, grad_keys, grad_values, grad_ir, grad_gate
 
 
@@ -239,4 +223,6 @@ def moe_ffn(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig) -> torc
     (their side streams and ctypes calls are nothing a tracer can follow)."""
     if torch.compiler.is_compiling():
         return torch.ops.amoe.ffn_fwd(x, keys, values, input_range, gate, sel_idx, *cfg_astuple(cfg))[0]
+    if not torch.is_grad_enabled():
+        return ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg)[0]
     return AnalogMoEFFN.apply(x, keys, values, input_range, gate, sel_idx, cfg)

@@ -30,7 +30,7 @@ from .config import (AIHWKITTorchInferenceRPUConfig, TorchInferenceRPUConfig, en
 from .cvmm import CVMM, AnalogExt, CVMMSel, cvmm_prepare_sel2, cvmm_std
 from . import library  # noqa: F401  (registers the amoe:: operators)
 from . import ops
-from .ffn import FFNConfig, _side_stream, moe_ffn
+from .ffn import FFNConfig, moe_ffn
 
 
 class MoEConifgError(Exception):
@@ -669,7 +669,7 @@ class AnalogSigmaMoELayer(SigmaMoELayer):
             want_wmax = noisy or cfg.out_bound > 0
             fork = x.is_cuda and not torch.compiler.is_compiling()
             main = torch.cuda.current_stream() if fork else None
-            side = _side_stream(x.device) if fork else None
+            side = ops.side_stream(x.device) if fork else None
             if fork:
                 side.wait_stream(main)
             with (torch.cuda.stream(side) if fork else contextlib.nullcontext()):

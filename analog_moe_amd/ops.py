@@ -6,6 +6,7 @@ There is no CPU path and no fallback: the library must have been built
 """
 from __future__ import annotations
 
+import functools
 import os
 from typing import Optional, Sequence, Tuple
 
@@ -34,7 +35,23 @@ def get_lib():
 
 
 def _stream(t: torch.Tensor):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
+
+
+_SIDE_STREAMS = {}
+
+
+def side_stream(device: torch.device) -> "torch.cuda.Stream":
+    """One extra stream per device (default priority), for launches that can run beside the current stream's."""
+    key = torch.device(device).index if torch.device(device).index is not None else torch.cuda.current_device()
+    if key not in _SIDE_STREAMS:
+        _SIDE_STREAMS[key] = torch.cuda.Stream(device=key)
+    return _SIDE_STREAMS[key]
+
+
+def _side(t: torch.Tensor):
+    """Handle of the device's extra stream (None where there are no streams)."""
+    return side_stream(t.device).cuda_stream if t.is_cuda else None
 
 
 def _need_gpu(*tensors) -> None:
@@ -135,25 +152,33 @@ def codes_supported(x: torch.Tensor, w: torch.Tensor, *, ir_by_expert: bool, inp
     ``cvmm_fwd`` would hand them over (freshly allocated tensors are 16-byte aligned, which is all that is left)."""
     if x.dtype not in (torch.bfloat16, torch.float16) or w.dtype != x.dtype or w.dim() != 3:
         return False
-    E, K, N = w.shape
+    K = w.shape[1]
     if x.dim() < 2 or x.shape[-1] != K or x.stride(-1) != 1 or (w.stride(2) != 1 and w.stride(1) != 1):
         return False
+    return _codes_supported(get_lib(), raw.dtype_code(x), x.numel() // K, x.stride(-2), tuple(w.shape), w.stride(), ir_by_expert,
+                            float(inp_res), n_tiles, float(out_bound), float(out_res), noise is not None, per_channel)
+
+
+@functools.lru_cache(maxsize=1024)
+def _codes_supported(lib, dtype, rows, ldx, w_shape, w_stride, ir_by_expert, inp_res, n_tiles, out_bound, out_res,
+                     injected_noise, per_channel) -> bool:
+    E, K, N = w_shape
     a = _abi.FwdArgs()
-    a.dtype = raw.dtype_code(x)
+    a.dtype = dtype
     a.M, a.N, a.K, a.E = 1, N, K, E
-    a.n_in_rows = x.numel() // K
-    a.ldx = x.stride(-2)
-    a.w_stride_e, a.w_stride_k, a.w_stride_n = w.stride(0), w.stride(1), w.stride(2)
+    a.n_in_rows = rows
+    a.ldx = ldx
+    a.w_stride_e, a.w_stride_k, a.w_stride_n = w_stride
     _abi.set_bounds(a, [0, K])
     a.n_tiles = n_tiles
     flag = 1                       # pointer fields are read as present / absent only
     a.ir, a.ir_by_expert = (flag if ir_by_expert else None), int(bool(ir_by_expert))
-    a.inp_res = float(inp_res)
-    a.noise = flag if noise is not None else None
+    a.inp_res = inp_res
+    a.noise = flag if injected_noise else None
     a.wmax, a.wmax_cols = flag, (N if per_channel else 1)
-    a.out_bound, a.out_res = float(out_bound), float(out_res)
+    a.out_bound, a.out_res = out_bound, out_res
     a.code_out, a.ldcode, a.code_scale_out = flag, N, flag
-    return bool(get_lib().amoe_fwd_codes_supported(a))
+    return bool(lib.amoe_fwd_codes_supported(a))
 
 
 def cvmm_bwd_w(x: torch.Tensor, g: torch.Tensor, n_experts: int, offsets: torch.Tensor, in_index: torch.Tensor,

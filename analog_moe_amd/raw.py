@@ -15,14 +15,23 @@ from . import _abi
 from ._abi import AMOE_BF16, AMOE_F16, AMOE_F32, BwdWArgs, BwdXArgs, FwdArgs, KsumClipArgs, check, set_bounds
 
 
+DTYPE_CODES = {torch.float32: AMOE_F32, torch.bfloat16: AMOE_BF16, torch.float16: AMOE_F16}
+
+
 def dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return AMOE_F32
-    if t.dtype == torch.bfloat16:
-        return AMOE_BF16
-    if t.dtype == torch.float16:
-        return AMOE_F16
-    raise TypeError(f"unsupported dtype {t.dtype}: the CVMM kernels take float32, bfloat16 or float16")
+    code = DTYPE_CODES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"unsupported dtype {t.dtype}: the CVMM kernels take float32, bfloat16 or float16")
+    return code
+
+
+def check_codes_fit(dtype: torch.dtype, res: float, name: str = "inp_res") -> None:
+    """The 16-bit kernels feed the DAC codes themselves to the matrix unit: integers are exact up to 256 in bf16 and
+    2048 in fp16 (the library returns AMOE_EUNSUPPORTED beyond that; this says why)."""
+    most = 256 if dtype == torch.bfloat16 else 2048
+    if res > 0 and 1.0 / res > most * (1 + 1e-6):
+        raise ValueError(f"{name}={res}: an input quantiser with more than {2 * most} steps needs fp32 tensors "
+                         f"({dtype} holds the codes exactly only up to +-{most})")
 
 
 def _p(t: Optional[torch.Tensor]):
@@ -123,13 +132,9 @@ def cvmm_fwd(lib, stream, x, w, out, sel_sorted, offsets, in_index, out_index=No
         a.xq_out, a.ldxq, a.xq_ir, a.xq_inp_res = _p(xq_out), xq_out.stride(0), _p(_f32(xq_ir, "xq_ir")), float(xq_inp_res)
     a.x_is_quantized = int(bool(x_is_quantized))
     if x.dtype != torch.float32:
-        # the 16-bit kernels feed the DAC codes themselves to the matrix unit: integers are exact up to 256 in
-        # bf16 and 2048 in fp16 (the library returns AMOE_EUNSUPPORTED beyond that; say why here)
-        most = 256 if x.dtype == torch.bfloat16 else 2048
-        for name, res in (("inp_res", inp_res), ("xq_inp_res", xq_inp_res if xq_out is not None else -1.0)):
-            if res > 0 and 1.0 / res > most * (1 + 1e-6):
-                raise ValueError(f"{name}={res}: an input quantiser with more than {2 * most} steps needs fp32 tensors "
-                                 f"({x.dtype} holds the codes exactly only up to +-{most})")
+        check_codes_fit(x.dtype, float(inp_res))
+        if xq_out is not None:
+            check_codes_fit(x.dtype, float(xq_inp_res), "xq_inp_res")
     check(lib, lib.amoe_cvmm_fwd(C.byref(a), stream), "amoe_cvmm_fwd")
 
 

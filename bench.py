@@ -11,6 +11,8 @@ The default workload is BASELINE.json's 64-expert tile-split layer,
 metric's MFMA-peak target is quoted on.  Only one GPU is used; --gpus N > 1 exits.
 """
 import argparse
+import ctypes
+import functools
 import json
 import os
 import sys
@@ -273,31 +275,33 @@ def main():
         for p in params:
             p.grad = None
 
-    # HIP events around every launch, on the stream the kernels are launched on; a launch is named
-    # by its op and its position among that op's calls within one step
-    ROLES = {"cvmm_fwd": ["fwd_up (up-projection forward)", "fwd_down (down-projection forward)"],
-             "cvmm_bwd_w": ["wgrad_down (weight gradient of the down-projection)",
-                            "wgrad_up (weight gradient of the up-projection)"],
-             "cvmm_bwd_x": ["xgrad_down (input gradient of the down-projection)",
-                            "xgrad_up (input gradient of the up-projection)"]}
+    # HIP events around every stage of the layer's two calls, on the stream its launches go to
+    from analog_moe_amd import ffn, moe_layer
+    ROLES = {"fwd_up": "fwd_up (up-projection forward)", "fwd_down": "fwd_down (down-projection forward)",
+             "wgrad_down": "wgrad_down (weight gradient of the down-projection)",
+             "wgrad_up": "wgrad_up (weight gradient of the up-projection)",
+             "xgrad_down": "xgrad_down (input gradient of the down-projection)",
+             "xgrad_up": "xgrad_up (input gradient of the up-projection)"}
+    lib = ops.get_lib()
+    stages = {}
+    for backward in (False, True):
+        names = []
+        while lib.amoe_ffn_stage_name(int(backward), len(names)) is not None:
+            names.append(lib.amoe_ffn_stage_name(int(backward), len(names)).decode())
+        stages[backward] = names
     events = {}
-    counter = {}
+    arrays = []                                   # the C arrays of event handles live as long as the timed steps
 
-    def timed(name):
-        fn = getattr(ops, name)
-
-        def wrapper(*a, **kw):
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            r = fn(*a, **kw)
-            e.record()
-            i = counter.get(name, 0)
-            counter[name] = i + 1
-            roles = ROLES.get(name)
-            key = roles[i % len(roles)] if roles else name
-            events.setdefault(key, []).append((s, e))
-            return r
-        return fn, wrapper
+    def stage_events(backward):
+        arr = (ctypes.c_void_p * (2 * len(stages[backward])))()
+        for i, name in enumerate(stages[backward]):
+            pair = tuple(torch.cuda.Event(enable_timing=True) for _ in range(2))
+            for j, ev in enumerate(pair):
+                ev.record()                       # (makes the handle; the call records it again where it belongs)
+                arr[2 * i + j] = ev.cuda_event
+            events.setdefault(ROLES.get(name, name), []).append(pair)
+        arrays.append(arr)
+        return ctypes.addressof(arr)
 
     if args.copy_calibration:
         # a plain device copy of known size: the scale for FETCH_SIZE / WRITE_SIZE readings of this run
@@ -324,20 +328,15 @@ def main():
         e0.record()
         torch.cuda.synchronize()
         spin_cycles = int(2.0 / max(s0.elapsed_time(e0), 1e-3) * 1_000_000)
-    saved = {}
-    for name in ("cvmm_fwd", "cvmm_bwd_w", "cvmm_bwd_x", "prepare_sel", "gate_reduce", "gate_grad", "ksum",
-                 "ksum_clip", "weight_abs_max", "weight_abs_max_pair", "segment_sum", "gate_reduce_codes",
-                 "gate_grad_codes"):
-        saved[name], w = timed(name)
-        setattr(ops, name, w)
+    plain_config = moe_layer.FFNConfig
+    moe_layer.FFNConfig = functools.partial(ffn.FFNConfig, stage_events=stage_events)
     torch.cuda.synchronize()
     for _ in range(args.steps):
         if spin_cycles:
             spin(spin_cycles)
         step()
     torch.cuda.synchronize()
-    for name, fn in saved.items():
-        setattr(ops, name, fn)
+    moe_layer.FFNConfig = plain_config
     # the same steps without events and spin kernels: the eager step time
     t0 = time.perf_counter()
     for _ in range(args.steps):
@@ -374,12 +373,12 @@ def main():
     kern = {n: sum(s.elapsed_time(e) for s, e in ev) / len(ev) for n, ev in events.items()}
     calls = {n: len(ev) // args.steps for n, ev in events.items()}
     per_step = {n: kern[n] * calls[n] for n in kern}
-    gemms = [r for rs in ROLES.values() for r in rs if r in kern]
+    gemms = [r for r in ROLES.values() if r in kern]
     # The dominant kernel is the GEMM kernel with the most time per step.  The two weight-gradient launches run one
     # kernel (a kernel trace lists them as one line with one average), so they count together and the figure is the
     # average over both; the forward and input-gradient launches may be different kernels and count alone.
-    groups = {r: [r] for r in gemms if r not in ROLES["cvmm_bwd_w"]}
-    wg = [r for r in ROLES["cvmm_bwd_w"] if r in kern]
+    wg = [r for r in gemms if r.startswith("wgrad")]
+    groups = {r: [r] for r in gemms if r not in wg}
     if wg:
         groups["wgrad (both weight-gradient launches, one kernel)"] = wg
     dom = max(groups, key=lambda g: sum(kern[r] for r in groups[g]))

@@ -383,6 +383,61 @@ int amoe_select_bwd(int32_t dtype, const void* logits, int64_t T, int32_t E, int
                     const int64_t* sel_idx, const void* grad_val, const float* reg_c,
                     const float* grad_reg, void* grad_logits, void* stream);
 
+/* ---------------------------------------------------------------------------------------
+ * The whole expert feed-forward of a layer, one call per direction: everything between a routing decision and the
+ * layer's output (moe_layer_aihwkit_lightning.py:384-410, 494-506: sort, up-projection, ReLU, down-projection, gate
+ * reduction), and everything between the output's gradient and the gradients of the inputs and parameters
+ * (cvmm.py:772-897 twice).  Each makes the calls above in their order, so the arithmetic is theirs; what it saves is
+ * the host time of a dozen separate calls and their argument structures.
+ * Every field is 8 bytes wide (pointers, int64, double), so that a binding can fill the struct with one pack call.
+ * A pointer that is NULL switches its feature off, as in the single calls. */
+typedef struct amoe_ffn_args {
+  /* sizes: T tokens of D features, E experts of F hidden features, V output features, k experts per token */
+  int64_t dtype, T, D, E, F, V, k;
+  const void* x;  int64_t ldx;                                  /* [T, D] rows */
+  const void* keys;  int64_t keys_se, keys_sk, keys_sn;         /* [E, D, F], strides in elements */
+  const void* values;  int64_t values_se, values_sk, values_sn; /* [E, F, V] */
+  const void* input_range;  int64_t ir_dtype, ir_cols;          /* parameter [2, E, ir_cols] (forward) */
+  const void* sel;  int64_t sel_is_i64;                         /* [T, k] expert ids */
+  const void* gate;                                             /* [T, k] dtype */
+  /* analog settings (amoe_fwd_args) */
+  double inp_res, out_bound, out_res, noise_std;
+  int64_t n_up;  const int32_t* bounds_up;                      /* K-tiles of the up-projection: n_up + 1 bounds */
+  int64_t n_dn;  const int32_t* bounds_dn;
+  int64_t noise_seed;  const uint64_t* noise_seed_dev;          /* the projections draw from seed and seed + 1 */
+  int64_t noise_per_channel;
+  const float* noise_up;  const float* noise_dn;                /* injected noise, or NULL */
+  const float* wmax_up;  const float* wmax_dn;                  /* max |W| made by the caller (modified weights), or NULL */
+  int64_t seed_bump;                                            /* added to *noise_seed_dev by the last launch */
+  void* down_ready;                                             /* hipEvent_t the down-projection waits for, or NULL */
+  /* what the forward call leaves and the backward call reads */
+  void* y;                                                      /* [T, V] */
+  void* p1;                                                     /* [T*k, F] hidden activation */
+  void* z;  int64_t z_is_codes;  float* z_scale;                /* [T*k, V] values, or ADC codes with scale [E, 2] */
+  int32_t* perm;  int32_t* in_index;  int32_t* offsets;         /* amoe_prepare_sel */
+  float* ir_up;  float* ir_dn;                                  /* fp32 input-range tables [E, n_up], [E, n_dn], NULL: no ranges */
+  /* backward only */
+  const void* dy;                                               /* [T, V] */
+  void* grad_x;  void* grad_keys;  void* grad_values;  void* grad_gate;
+  void* grad_ir;                                                /* [2, E, max(n_up, n_dn)] ir_dtype, or NULL */
+  int64_t gradient_relative;
+  double gradient_scale, decay, input_min_percentage;
+  /* profiling: if not NULL, hipEvent_t pairs recorded around the launches of each stage, in the order of
+   * amoe_ffn_stage_name(backward, i) */
+  void* const* stage_events;
+} amoe_ffn_args;
+
+/* Bytes of scratch memory the call needs (reads sizes and settings only).  Nothing in it outlives the call. */
+size_t amoe_ffn_fwd_workspace(const amoe_ffn_args* args);
+size_t amoe_ffn_bwd_workspace(const amoe_ffn_args* args);
+/* Launches on `stream`; launches that can run beside them go to `side_stream` (NULL: none do), which is joined with
+ * `stream` before the call returns, so that memory order on `stream` alone is enough for the caller. */
+int amoe_ffn_fwd(const amoe_ffn_args* args, void* workspace, size_t workspace_bytes, void* stream, void* side_stream);
+int amoe_ffn_bwd(const amoe_ffn_args* args, void* workspace, size_t workspace_bytes, void* stream, void* side_stream);
+/* Name of stage i of a direction, NULL past the last. */
+const char* amoe_ffn_stage_name(int32_t backward, int32_t i);
+size_t amoe_ffn_args_bytes(void);
+
 #ifdef __cplusplus
 }
 #endif

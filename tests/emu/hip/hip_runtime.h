@@ -33,6 +33,13 @@ typedef int hipError_t;
 typedef void* hipStream_t;
 enum { hipSuccess = 0 };
 inline hipError_t hipGetLastError() { return hipSuccess; }
+// launches run at once and in order, so streams and events order nothing here
+typedef void* hipEvent_t;
+enum { hipEventDisableTiming = 2 };
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = nullptr; return hipSuccess; }
+inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 inline const char* hipGetErrorString(hipError_t) { return "emu"; }
 enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount = 0 };
 inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }

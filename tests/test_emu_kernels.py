@@ -345,3 +345,9 @@ def test_chained_projections(emu_ops, dtype, D, F, T):
                                          (torch.bfloat16, 72, 40, 60), (torch.bfloat16, 256, 256, 200)])
 def test_clipped_input_for_the_weight_gradient(emu_ops, dtype, D, F, T):
     util.check_clipped_input_output(emu_ops, dtype=dtype, T=T, D=D, F=F)
+
+
+@pytest.mark.parametrize("case", util.LAYER_CALLS, ids=lambda c: f"{c[0]}x{c[1]}_{c[5]}")
+def test_layer_calls_equal_the_single_calls(emu_ops, case):
+    util.check_layer_calls(emu_ops, case, "cpu")
+

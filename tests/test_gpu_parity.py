@@ -344,3 +344,12 @@ def test_segment_sum_of_long_segments(ops, rows):
         part = v[off[e]:off[e + 1]].astype(np.float64)
         bound = (len(part) + 1) * 2.0 ** -24 * np.abs(part).sum(0)
         assert np.all(np.abs(got[e] - part.sum(0)) <= bound)
+
+
+# (the last two are large enough for the second stream in both directions)
+@pytest.mark.parametrize("case", util.LAYER_CALLS + [
+    (4096, 512, 64, 256, 4, "bf16", None, True, True, 0.04),
+    (2500, 1024, 16, 448, 8, "f16", [0, 512, 1024], True, False, 0.04)], ids=lambda c: f"{c[0]}x{c[1]}_{c[5]}")
+def test_layer_calls_equal_the_single_calls(ops, case):
+    util.check_layer_calls(ops, case, "cuda")
+

@@ -640,3 +640,44 @@ def check_gate_reduce_counter(ops, device="cpu"):
                        ops.gate_reduce_codes(codes, scale, sel, gate)) and int(counter) == 10
     assert ops.gate_reduce(z[:0], gate[:0], counter, 1).shape == (0, D) and int(counter) == 11
     assert ops.gate_reduce_codes(codes[:0], scale, sel[:0], gate[:0], counter, 1).shape == (0, D) and int(counter) == 12
+
+
+# ---- the layer calls (amoe_ffn_fwd / amoe_ffn_bwd) against the single calls ---------------------------------------
+LAYER_CALLS = [
+    # T, D, E, F, k, dtype, bounds of the up-projection, input ranges, ADC, noise
+    (1, 64, 4, 64, 2, "bf16", None, True, True, 0.0),
+    (37, 76, 3, 36, 2, "f32", [0, 40, 76], True, True, 0.04),       # clip not on 16-byte pieces: masks in the GEMM
+    (40, 128, 4, 64, 1, "f16", None, True, False, 0.04),            # one head: no sum over the heads
+    (33, 96, 5, 48, 3, "f32", None, False, False, 0.0),             # no input ranges
+    (60, 256, 3, 256, 2, "bf16", [0, 128, 256], True, True, 0.04),  # the result kept as ADC codes
+]
+
+
+def check_layer_calls(ops, case, device):
+    """Every output equals that of the single calls on the same inputs, bit for bit (the input-range sums, which the
+    layer makes per expert, to rounding)."""
+    from analog_moe_amd import ffn
+    T, D, E, F, k, dt, bounds, ranges, adc, noise = case
+    pr = {n: t.to(device) for n, t in make_problem(11, T=T, D=D, E=E, F=F, k=k, dtype=TORCH_DTYPE[dt]).items()}
+    nt = 1 if bounds is None else len(bounds) - 1
+    ir = (torch.rand(2, E, nt) + 1.0).to(device) if ranges else None
+    kw = dict(inp_res=1 / 127 if ranges else -1.0, out_bound=12.0 if adc else -1.0, out_res=254.0 if adc else -1.0)
+    cfg = ffn.FFNConfig(bounds_up=bounds, noise_std=noise, noise_seed=5, decay=0.01, input_min_percentage=0.5, **kw)
+    fwd = ffn.ffn_forward(pr["x"], pr["keys"], pr["values"], ir, pr["gate"], pr["idx"], cfg)
+    y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn = fwd
+    want = layer_ops_fwd_bwd(ops, pr, ir, bounds_up=bounds, noise_std=noise, noise_seed=5 if noise else None, decay=0.01,
+                             input_min_percentage=0.5, by_expert=True, **kw)
+    assert torch.equal(p1, want["scores"]) and torch.equal(perm, want["perm"]) and torch.equal(offsets, want["offsets"])
+    if z.dtype == torch.uint8:
+        assert torch.equal(ops.dequant_codes(z, z_scale, pr["idx"]).to(p1.dtype), want["z"])
+    else:
+        assert torch.equal(z, want["z"]) and torch.equal(y, want["y"])
+    gx, gk, gv, gir, gg = ffn.ffn_backward(pr["dy"], pr["x"], pr["keys"], pr["values"], pr["gate"], pr["idx"], *fwd[1:3],
+                                           z_scale, perm, in_index, offsets, ir_up, ir_dn, cfg, ranges)
+    assert torch.equal(gx, want["grad_x"]) and torch.equal(gk, want["grad_keys"]) and torch.equal(gv, want["grad_values"])
+    if z.dtype != torch.uint8:
+        assert torch.equal(gg, want["grad_gate"])
+    if ranges:      # sums of n fp32 values in another order: n * 2^-24 of their absolute sum
+        bound = (T * k * max(D, F)) * 2.0 ** -24 * float(want["grad_ir"].abs().max() + 1.0)
+        assert float((gir - want["grad_ir"]).abs().max()) <= bound
+
