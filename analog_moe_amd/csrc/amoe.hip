@@ -870,7 +870,10 @@ int amoe_clamp_weights(int32_t dtype, void* w, int32_t E, int32_t K, int32_t N, 
   return launch_rc();
 }
 
-static long long select_blocks(long long T) { return (T + 4 * kSelRowsPerWave - 1) / (4 * kSelRowsPerWave); }
+static long long select_blocks(long long T) {
+  const int per_block = 4 * select_rows_per_wave(T);
+  return (T + per_block - 1) / per_block;
+}
 
 size_t amoe_select_workspace(int64_t T, int32_t E) {
   if (T < 1 || E < 1) return 0;
@@ -898,20 +901,21 @@ int amoe_select_fwd(int32_t dtype, const void* logits, int64_t T, int32_t E, int
     partial = static_cast<float*>(workspace);
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const int rpw = select_rows_per_wave(T);
 #define AMOE_SELECT_FWD(PER)                                                                                           \
   do {                                                                                                                 \
     if (dtype == AMOE_F32) {                                                                                           \
       auto kf = &select_fwd_kernel<float, PER>;                                                                        \
       hipLaunchKernelGGL(kf, dim3((unsigned)blocks), dim3(kThreads), 0, st, static_cast<const float*>(logits),         \
-                         (long long)T, (int)E, (int)k, static_cast<float*>(sel_val), sel_idx, partial);                \
+                         (long long)T, (int)E, (int)k, rpw, static_cast<float*>(sel_val), sel_idx, partial);           \
     } else if (dtype == AMOE_BF16) {                                                                                   \
       auto kf = &select_fwd_kernel<uint16_t, PER>;                                                                     \
       hipLaunchKernelGGL(kf, dim3((unsigned)blocks), dim3(kThreads), 0, st, static_cast<const uint16_t*>(logits),      \
-                         (long long)T, (int)E, (int)k, static_cast<uint16_t*>(sel_val), sel_idx, partial);             \
+                         (long long)T, (int)E, (int)k, rpw, static_cast<uint16_t*>(sel_val), sel_idx, partial);        \
     } else {                                                                                                           \
       auto kf = &select_fwd_kernel<f16_t, PER>;                                                                        \
       hipLaunchKernelGGL(kf, dim3((unsigned)blocks), dim3(kThreads), 0, st, static_cast<const f16_t*>(logits),         \
-                         (long long)T, (int)E, (int)k, static_cast<f16_t*>(sel_val), sel_idx, partial);                \
+                         (long long)T, (int)E, (int)k, rpw, static_cast<f16_t*>(sel_val), sel_idx, partial);           \
     }                                                                                                                  \
   } while (0)
   if (E <= 64) AMOE_SELECT_FWD(1);

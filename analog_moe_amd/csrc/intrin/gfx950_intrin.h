@@ -68,8 +68,11 @@ __device__ __forceinline__ BufRsrc make_rsrc(const void* base) {
 __device__ __forceinline__ u32x4 buffer_load_b128(BufRsrc r, uint32_t lane_off, uint32_t uniform_off) {
   return __builtin_amdgcn_raw_buffer_load_b128(r, lane_off, uniform_off, 0);
 }
-__device__ __forceinline__ uint32_t buffer_load_b32(BufRsrc r, uint32_t lane_off) {
-  return __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, 0, 0);
+__device__ __forceinline__ uint32_t buffer_load_b32(BufRsrc r, uint32_t lane_off, uint32_t uniform_off = 0) {
+  return __builtin_amdgcn_raw_buffer_load_b32(r, lane_off, uniform_off, 0);
+}
+__device__ __forceinline__ u32x2 buffer_load_b64(BufRsrc r, uint32_t lane_off, uint32_t uniform_off) {
+  return __builtin_amdgcn_raw_buffer_load_b64(r, lane_off, uniform_off, 0);
 }
 // Resource over [base, base + bytes): an access at a byte offset >= bytes is out of range; out-of-range stores are
 // dropped by the hardware, which makes a store conditional without a branch around it.
@@ -89,8 +92,15 @@ __device__ __forceinline__ uint32_t pack_high_halves(uint32_t hi, uint32_t lo) {
   return __builtin_amdgcn_perm(hi, lo, 0x07060302u);
 }
 
+// the low halves likewise
+__device__ __forceinline__ uint32_t pack_low_halves(uint32_t hi, uint32_t lo) {
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
+
 // value held by the first active lane, as a scalar
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+// value held by lane `src` (the same for the whole wave), as a scalar
+__device__ __forceinline__ uint32_t wave_read(uint32_t v, int src) { return (uint32_t)__builtin_amdgcn_readlane((int)v, src); }
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
 template <typename V>

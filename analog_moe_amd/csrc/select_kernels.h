@@ -7,7 +7,10 @@
 namespace amoe {
 
 constexpr int kSelPerLane = 8;            // experts per lane: E <= 512
-constexpr int kSelRowsPerWave = 8;        // rows a wave walks through; its usage sums stay in registers meanwhile
+// Rows a wave walks through (its usage sums stay in registers meanwhile).  A row is a serial chain of about a
+// microsecond, so few rows take a wave each -- 1717 rows of 64 experts: 35.4 us with eight rows per wave -- and only
+// where two waves per SIMD are there anyway do they take more, for fewer partial usage sums to add.
+__host__ __device__ inline int select_rows_per_wave(long long rows) { return rows <= 2048 ? 1 : rows <= 16384 ? 2 : 8; }
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
@@ -26,11 +29,61 @@ __device__ __forceinline__ float gate_value(float x) {
   return Elem<T>::to_f32(Elem<T>::cvt(1.0f / (1.0f + expf(-x))));
 }
 
+// The k largest of a row's gate values s (lane owns the experts lane, lane + 64, ...; NaN: never chosen): an expert's
+// place is the number of experts with a larger value, or with the same value and a lower id.  Gate values are not
+// negative, so their bit patterns order as they do; 0 marks what cannot be chosen.
+template <typename T, int PER>
+__device__ __forceinline__ void select_by_rank(const float (&s)[PER], int lane, int E, int k, T* __restrict__ val,
+                                               int64_t* __restrict__ idx) {
+  uint32_t key[PER];
+  int place[PER], n = 0;
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    key[j] = s[j] >= 0.f ? as_u32(s[j]) + 1u : 0u;
+    place[j] = 0;
+    n += popc64(wave_ballot(key[j] != 0u));
+  }
+#pragma unroll
+  for (int jj = 0; jj < PER; jj++) {
+    const int here = E - 64 * jj < 64 ? E - 64 * jj : 64;
+#pragma unroll 8
+    for (int l = 0; l < here; l++) {
+      const uint32_t other = wave_read(key[jj], l);
+#pragma unroll
+      for (int j = 0; j < PER; j++) {
+        const bool lower_id = jj < j || (jj == j && l < lane);
+        place[j] += other > key[j] - (lower_id ? 1u : 0u) ? 1 : 0;
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < PER; j++)
+    if (key[j] != 0u && place[j] < k) {
+      val[place[j]] = Elem<T>::cvt(s[j]);
+      idx[place[j]] = lane + 64 * j;
+    }
+  if (lane >= n && lane < k) {                    // fewer than k experts can be chosen
+    val[lane] = Elem<T>::cvt(-__builtin_inff());
+    idx[lane] = 0x7fffffff;
+  }
+  for (int t = 64 + lane; t < k; t += 64)
+    if (t >= n) {
+      val[t] = Elem<T>::cvt(-__builtin_inff());
+      idx[t] = 0x7fffffff;
+    }
+}
+
 // sel_val / sel_idx [rows, k]: the k largest gate values of each row in descending order, ties to the lower
 // expert id.  prob_partial [gridDim.x, E] (optional): per workgroup, sum over its rows of softmax(logits[row]).
+//
+// Up to 128 experts every expert counts the experts ahead of it: one scalar broadcast and a compare-and-add per
+// expert, independent of each other, where k rounds of a wave-wide maximum are 12 * k dependent lane exchanges
+// (64 experts, k = 8: 4.4 us a row against 0.6).  The count costs E * PER compares whatever k is, so two experts per
+// lane need k >= 2 to gain and more than two keep the rounds.
 template <typename T, int PER>
 __global__ __launch_bounds__(kThreads) void select_fwd_kernel(const T* __restrict__ logits, long long rows, int E, int k,
-                                                               T* __restrict__ sel_val, int64_t* __restrict__ sel_idx,
+                                                               int rows_per_wave, T* __restrict__ sel_val,
+                                                               int64_t* __restrict__ sel_idx,
                                                                float* __restrict__ prob_partial) {
   __shared__ float sProb[4][64 * PER];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -38,8 +91,8 @@ __global__ __launch_bounds__(kThreads) void select_fwd_kernel(const T* __restric
   float usage[PER];
 #pragma unroll
   for (int j = 0; j < PER; j++) usage[j] = 0.f;
-  const long long first = ((long long)blockIdx.x * 4 + wave) * kSelRowsPerWave;
-  for (int rr = 0; rr < kSelRowsPerWave; rr++) {
+  const long long first = ((long long)blockIdx.x * 4 + wave) * rows_per_wave;
+  for (int rr = 0; rr < rows_per_wave; rr++) {
     const long long row = first + rr;
     if (row >= rows) break;                       // the same for the whole wave
     const T* __restrict__ src = logits + row * (long long)E;
@@ -64,6 +117,10 @@ __global__ __launch_bounds__(kThreads) void select_fwd_kernel(const T* __restric
       const float inv = 1.0f / wave_sum(sum);
 #pragma unroll
       for (int j = 0; j < PER; j++) usage[j] += ex[j] * inv;
+    }
+    if (PER <= 2 && k >= PER) {
+      select_by_rank<T, PER>(s, lane, E, k, sel_val + row * k, sel_idx + row * k);
+      continue;
     }
     for (int t = 0; t < k; t++) {
       float bv = kNegInf;

@@ -19,9 +19,14 @@ inline u32x4 buffer_load_b128(BufRsrc r, uint32_t lane_off, uint32_t uniform_off
   std::memcpy(&v, r.base + (size_t)lane_off + (size_t)uniform_off, 16);
   return v;
 }
-inline uint32_t buffer_load_b32(BufRsrc r, uint32_t lane_off) {
+inline uint32_t buffer_load_b32(BufRsrc r, uint32_t lane_off, uint32_t uniform_off = 0) {
   uint32_t v;
-  std::memcpy(&v, r.base + (size_t)lane_off, 4);
+  std::memcpy(&v, r.base + (size_t)lane_off + (size_t)uniform_off, 4);
+  return v;
+}
+inline u32x2 buffer_load_b64(BufRsrc r, uint32_t lane_off, uint32_t uniform_off) {
+  u32x2 v;
+  std::memcpy(&v, r.base + (size_t)lane_off + (size_t)uniform_off, 8);
   return v;
 }
 // out-of-range stores are dropped, as the hardware's range check does
@@ -29,6 +34,7 @@ inline void buffer_store_b128_nt(BufRsrc r, u32x4 v, uint32_t lane_off) {
   if ((uint64_t)lane_off + 16 <= r.bytes) std::memcpy(const_cast<unsigned char*>(r.base) + lane_off, &v, 16);
 }
 inline uint32_t pack_high_halves(uint32_t hi, uint32_t lo) { return (hi & 0xffff0000u) | (lo >> 16); }
+inline uint32_t pack_low_halves(uint32_t hi, uint32_t lo) { return (hi << 16) | (lo & 0xffffu); }
 // scheduling fences mean nothing to a host compiler
 inline void sched_fence() {}
 
@@ -46,6 +52,7 @@ template <class V> inline V emu_exchange(V v, int src) {
 }
 template <class V> inline V wave_shfl_xor(V v, int mask) { return emu_exchange(v, lane_id() ^ mask); }
 template <class V> inline V wave_shfl(V v, int src) { return emu_exchange(v, src); }
+inline uint32_t wave_read(uint32_t v, int src) { return emu_exchange(v, src); }
 template <class V> inline V wave_shfl_up(V v, int d) {
   int l = lane_id();
   return emu_exchange(v, l >= d ? l - d : l);

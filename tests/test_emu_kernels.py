@@ -351,3 +351,8 @@ def test_clipped_input_for_the_weight_gradient(emu_ops, dtype, D, F, T):
 def test_layer_calls_equal_the_single_calls(emu_ops, case):
     util.check_layer_calls(emu_ops, case, "cpu")
 
+
+
+@pytest.mark.parametrize("T,E,k", [(5, 64, 64), (3, 65, 1), (3, 128, 2), (2, 128, 128), (3, 7, 3)])
+def test_select_rows(emu_ops, T, E, k):
+    util.check_select_rows(emu_ops, "cpu", torch.bfloat16, T, E, k)

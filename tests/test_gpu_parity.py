@@ -353,3 +353,8 @@ def test_segment_sum_of_long_segments(ops, rows):
 def test_layer_calls_equal_the_single_calls(ops, case):
     util.check_layer_calls(ops, case, "cuda")
 
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,E,k", [(1, 64, 8), (2047, 64, 64), (2051, 128, 1), (2051, 128, 2), (16389, 16, 4), (300, 65, 65)])
+def test_select_rows(ops, dtype, T, E, k):
+    util.check_select_rows(ops, "cuda", dtype, T, E, k)

@@ -681,3 +681,25 @@ def check_layer_calls(ops, case, device):
         bound = (T * k * max(D, F)) * 2.0 ** -24 * float(want["grad_ir"].abs().max() + 1.0)
         assert float((gir - want["grad_ir"]).abs().max()) <= bound
 
+
+
+def check_select_rows(ops, device, dtype, T, E, k):
+    """Every expert of a row whose gate value is a number, in order (ties to the lower id); the sentinel of a row that
+    has fewer than k such values."""
+    g = torch.Generator().manual_seed(T + E)
+    logits = (torch.randn(T, E, generator=g) * 2.0).to(dtype)
+    logits[:, 1::3] = logits[:, :1]                                  # ties in every row
+    logits[T - 1, : E // 2] = float("nan")
+    val, idx, _, _ = ops.select_fwd(logits.to(device), k, False)
+    # (fp32 gate values come from the device's exp: what must hold is the order of the values it chose)
+    gate = torch.sigmoid(logits.float()).to(dtype).double().numpy()
+    idx, val = idx.cpu().numpy(), val.cpu().double().numpy()
+    n = [int(np.isfinite(r).sum()) for r in gate]
+    tol = {torch.float32: 2.0 ** -22, torch.bfloat16: 2.0 ** -7, torch.float16: 2.0 ** -10}[dtype]
+    for t in range(T):
+        m = min(k, n[t])
+        assert len(set(idx[t, :m])) == m and np.all(idx[t, m:] == 0x7FFFFFFF) and np.all(np.isneginf(val[t, m:]))
+        np.testing.assert_allclose(val[t, :m], gate[t, idx[t, :m]], rtol=tol)
+        np.testing.assert_allclose(val[t, :m], -np.sort(-np.where(np.isnan(gate[t]), -1.0, gate[t]))[:m], rtol=tol)
+        tied = val[t, 1:m] == val[t, : max(m - 1, 0)]
+        assert np.all(val[t, 1:m] <= val[t, : max(m - 1, 0)]) and np.all(np.diff(idx[t, :m])[tied] > 0)
