@@ -30,6 +30,7 @@ inline bool dac_codes_fit(int dtype, float inp_res) {
   if (dtype == AMOE_F32 || !(inp_res > 0.f)) return true;
   return 1.0f / inp_res <= (dtype == AMOE_BF16 ? 256.f : 2048.f) * (1.0f + 1e-6f);
 }
+constexpr int kDirRows = 32, kDirCols = 64;   // output tile of gemm_direct.h
 inline int max_row_tiles(int64_t M, int E) { return (int)(M / kTileRows) + E; }
 
 // Compute units of the current device (read once; the value cannot change while the process lives).
@@ -108,6 +109,7 @@ inline int launch_rows(int dtype, const RowsParams& p, bool w_kc, int mode, int 
 // gemm_fwd256.hip, gemm_bwdx256.hip: the tiled kernels of the training shapes and the weights-in-registers kernel
 // (16-bit types).  AMOE_EUNSUPPORTED: not one of their launches, the general kernel runs it.
 int launch_fwd256(const RowsParams& p, int mode, const amoe_fwd_args* a, hipStream_t st);
+int launch_direct(const RowsParams& p, bool w_kc, const amoe_fwd_args* a, hipStream_t st);   // gemm_direct.hip
 int launch_bwdx256(const RowsParams& p, const amoe_bwd_x_args* a, hipStream_t st, int* n_count_blocks, int* block_cols);
 
 }  // namespace amoe

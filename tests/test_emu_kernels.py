@@ -353,6 +353,13 @@ def test_layer_calls_equal_the_single_calls(emu_ops, case):
 
 
 
+@pytest.mark.parametrize("dtype,K,N,kc,tiles,stages", [
+    (torch.bfloat16, 130, 66, False, 2, "noisy"), (torch.bfloat16, 576, 64, True, 1, "noisy"), (torch.float16, 64, 2, False, 1, "plain"),
+    (torch.float32, 301, 34, False, 1, "noisy"), (torch.float32, 36, 61, True, 2, "dac")])
+def test_forward_small_tiles(emu_ops, dtype, K, N, kc, tiles, stages):
+    util.check_forward_small_tiles(emu_ops, "cpu", dtype, K, N, kc, tiles, stages)
+
+
 @pytest.mark.parametrize("T,E,k", [(5, 64, 64), (3, 65, 1), (3, 128, 2), (2, 128, 128), (3, 7, 3)])
 def test_select_rows(emu_ops, T, E, k):
     util.check_select_rows(emu_ops, "cpu", torch.bfloat16, T, E, k)

@@ -354,6 +354,17 @@ def test_layer_calls_equal_the_single_calls(ops, case):
     util.check_layer_calls(ops, case, "cuda")
 
 
+# copies 1: the kernel for small launches; 400: the tiled ones, on the same edges
+@pytest.mark.parametrize("copies", [1, 400])
+@pytest.mark.parametrize("kc,tiles,stages", [(False, 1, "plain"), (False, 2, "noisy"), (True, 1, "noisy"), (True, 2, "dac")])
+@pytest.mark.parametrize("dtype,K,N", [(torch.bfloat16, 412, 64), (torch.bfloat16, 130, 66), (torch.float16, 1088, 2),
+                                       (torch.float32, 301, 34), (torch.float32, 576, 130), (torch.bfloat16, 128, 256)])
+def test_forward_small_tiles(ops, dtype, K, N, kc, tiles, stages, copies):
+    if copies > 1 and K > 512:
+        pytest.skip("the oracle takes the long contraction row by row: small launches only")
+    util.check_forward_small_tiles(ops, "cuda", dtype, K, N, kc, tiles, stages, copies)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,E,k", [(1, 64, 8), (2047, 64, 64), (2051, 128, 1), (2051, 128, 2), (16389, 16, 4), (300, 65, 65)])
 def test_select_rows(ops, dtype, T, E, k):

@@ -683,6 +683,51 @@ def check_layer_calls(ops, case, device):
 
 
 
+def check_forward_small_tiles(ops, device, dtype, K, N, kc, tiles, stages, copies=1):
+    """cvmm_fwd against the oracle on experts that end at the edges of 32-row tiles, with contractions and columns that
+    end inside a step of 128 bytes and a block of 64 columns.  copies > 1: as many times the rows, which is past the
+    number of tiles that the kernel for small launches takes.  Tolerances: one rounding of the result (2^-9 in bf16,
+    2^-12 in fp16) or a 32-bit sum in another order (K * 2^-24 of the sum of magnitudes, far under 1e-5), times the ADC's
+    steps where a sum lies on its boundary."""
+    name = dtype_name(dtype)
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    g = torch.Generator().manual_seed(K + N)
+    counts = torch.tensor([0, 1, 31, 32, 33, 65]) * copies
+    E, M = len(counts), int(counts.sum())
+    idx = torch.repeat_interleave(torch.arange(E), counts)[torch.randperm(M, generator=g)].reshape(M, 1)
+    ss, perm, in_index, offsets = ops.prepare_sel(idx.to(device), E, 1)
+    x = torch.randn(M, K, generator=g).to(dtype)
+    w = (torch.randn(E, N, K, generator=g).transpose(1, 2) if kc else torch.randn(E, K, N, generator=g)) / K ** 0.5
+    w = w.to(dtype)
+    sel_np, perm_np = ss.cpu().numpy(), perm.cpu().numpy()
+    kw, okw, step = {}, dict(dtype=name), 0.0
+    wm = w.float().abs().amax((1, 2)).reshape(E, 1)
+    bounds = None if tiles == 1 else (0, K // 4 * 2, K)
+    if stages != "plain":
+        ir = torch.linspace(0.7, 2.5, E * tiles).reshape(E, tiles)
+        kw = dict(ir=ir.to(device), ir_by_expert=True, inp_res=1.0 / 127.0, bounds=bounds, wmax=wm.to(device))
+        okw.update(inp_res=1.0 / 127.0, ir=ir.numpy()[sel_np], bounds=bounds, wmax=wm.numpy())
+    if stages == "noisy":
+        for d in (kw, okw):
+            d.update(out_bound=12.0, out_res=254.0, noise_std=0.04, noise_seed=17)
+        step = tiles * 12.0 * float(wm.max()) / 127.0 * 2.5
+    xq_ir = torch.linspace(0.4, 1.1, E)
+    if stages == "noisy":
+        kw.update(relu=True, xq_ir=xq_ir.to(device), xq_inp_res=1.0 / 127.0)
+        okw.update(relu=True)
+    got = ops.cvmm_fwd(x.to(device), w.to(device) if not kc else w.transpose(1, 2).contiguous().to(device).transpose(1, 2),
+                       ss, offsets, perm, None, M, **kw)
+    want = O.cvmm_fwd(np32(x), perm_np, sel_np, np32(w), **okw)
+    if stages != "noisy":
+        assert rel_err(np32(got), want) < tol
+        return
+    got, xq = got
+    adc_flip_check(np32(got), want, tol, step, max_fraction=2e-3)
+    e = idx.reshape(-1)
+    _, codes = O.dac(np32(got), xq_ir.numpy()[e.numpy()].reshape(-1, 1), None, 1.0 / 127.0)
+    assert np.array_equal(np32(xq) if dtype != torch.float32 else np.rint(np32(xq) * 127.0), codes)
+
+
 def check_select_rows(ops, device, dtype, T, E, k):
     """Every expert of a row whose gate value is a number, in order (ties to the lower id); the sentinel of a row that
     has fewer than k such values."""
