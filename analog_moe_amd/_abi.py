@@ -108,6 +108,7 @@ PROTOTYPES = {
     "amoe_weight_std_workspace": (SZ, [I32, I32, I32, I32]),
     "amoe_weight_std": (C.c_int, [I32, P, I32, I32, I32, I32, P, P, SZ, P]),
     "amoe_clamp_weights": (C.c_int, [I32, P, I32, I32, I32, P, I32, P]),
+    "amoe_router_fwd": (C.c_int, [I32, P, I64, I64, I32, P, I64, I32, I32, P, I32, P, F32, F32, F32, P, P, P]),
     "amoe_ffn_args_bytes": (SZ, []),
     "amoe_ffn_fwd_workspace": (SZ, [P]),
     "amoe_ffn_bwd_workspace": (SZ, [P]),

@@ -33,20 +33,23 @@ template <typename T> inline constexpr int kDirStep = 128 / (int)sizeof(T);
 //   W_KC                : words 4 * f .. 4 * f + 3 = column 32 * f + lane % 32
 //   16-bit, column pairs: word r = contraction index r of the piece, columns 2 * (lane % 32) (low half) and + 1 (high)
 //   32-bit, column pairs: words 2 * r, 2 * r + 1
+// NF: blocks of 32 columns (2, and with W_KC also 4).
+template <int NF = 2>
 struct DirectStep {
   Raw x[4];
-  uint32_t w[4][8];
+  uint32_t w[4][4 * NF];
 };
 
-template <typename T, bool W_KC>
+template <typename T, bool W_KC, int NF = 2>
 struct DirectLoader {
+  static_assert(W_KC || NF == 2, "column pairs cover 64 columns");
   const T* xrow;                // this lane's token row
-  const T* wcol[2];             // W_KC: its two columns
+  const T* wcol[NF];            // W_KC: its columns
   BufRsrc w_rsrc;               // otherwise: W[e], addressed with 32-bit byte offsets
   uint32_t w_lane, w_ks;        // byte offset of (contraction index 0, this lane's column pair), bytes per index
   int lh;
 
-  __device__ __forceinline__ void load(DirectStep& s, int k0, int khi) const {
+  __device__ __forceinline__ void load(DirectStep<NF>& s, int k0, int khi) const {
     constexpr int CH = Elem<T>::kChunk, STEP = kDirStep<T>;
     if (k0 + STEP <= khi) {                                  // (the same for the whole wave)
 #pragma unroll
@@ -55,7 +58,7 @@ struct DirectLoader {
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-          for (int f = 0; f < 2; f++) {
+          for (int f = 0; f < NF; f++) {
             const Raw v = load16_al4(wcol[f] + k0 + (2 * i + lh) * CH);
 #pragma unroll
             for (int d = 0; d < 4; d++) s.w[i][4 * f + d] = v[d];
@@ -87,7 +90,7 @@ struct DirectLoader {
       s.x[i] = raw_load<T>(xrow + kpos, nv, false);
       if constexpr (W_KC) {
 #pragma unroll
-        for (int f = 0; f < 2; f++) {
+        for (int f = 0; f < NF; f++) {
           const Raw v = raw_load<T>(wcol[f] + kpos, nv, false);
 #pragma unroll
           for (int d = 0; d < 4; d++) s.w[i][4 * f + d] = v[d];
@@ -143,44 +146,44 @@ struct DirectDac {
 };
 
 // acc[f] += step (f: W_KC columns 32 * f + i, otherwise columns 2 * i + f of the tile, i the instruction's row index)
-template <typename T, bool W_KC>
-__device__ __forceinline__ void direct_multiply(f32x16 (&acc)[2], DirectStep& s, const DirectDac& dac) {
+template <typename T, bool W_KC, int NF = 2>
+__device__ __forceinline__ void direct_multiply(f32x16 (&acc)[NF], DirectStep<NF>& s, const DirectDac& dac) {
 #pragma unroll
   for (int i = 0; i < 4; i++) {
     if (dac.on) dac.apply<T>(s.x[i]);
     if constexpr (sizeof(T) == 2) {
-      u32x4 wf[2];
+      u32x4 wf[NF];
 #pragma unroll
       for (int d = 0; d < 4; d++) {
         if constexpr (W_KC) {
-          wf[0][d] = s.w[i][d];
-          wf[1][d] = s.w[i][4 + d];
+#pragma unroll
+          for (int f = 0; f < NF; f++) wf[f][d] = s.w[i][4 * f + d];
         } else {
           wf[0][d] = pack_low_halves(s.w[i][2 * d + 1], s.w[i][2 * d]);
           wf[1][d] = pack_high_halves(s.w[i][2 * d + 1], s.w[i][2 * d]);
         }
       }
 #pragma unroll
-      for (int f = 0; f < 2; f++) acc[f] = mfma_32x32x16<T>(wf[f], s.x[i], acc[f]);
+      for (int f = 0; f < NF; f++) acc[f] = mfma_32x32x16<T>(wf[f], s.x[i], acc[f]);
     } else {
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
-        for (int f = 0; f < 2; f++)
+        for (int f = 0; f < NF; f++)
           acc[f] = mfma_32x32x2_f32(as_f32(W_KC ? s.w[i][4 * f + j] : s.w[i][2 * j + f]), as_f32(s.x[i][j]), acc[f]);
     }
   }
 }
 
 // A wave's partial tile -> LDS, [row][column]
-template <bool W_KC>
-__device__ __forceinline__ void direct_store_partial(float* __restrict__ tile, const f32x16 (&acc)[2], int l32, int lh) {
-  float* __restrict__ row = tile + l32 * kDirLd;
+template <bool W_KC, int NF = 2>
+__device__ __forceinline__ void direct_store_partial(float* __restrict__ tile, const f32x16 (&acc)[NF], int l32, int lh) {
+  float* __restrict__ row = tile + l32 * (32 * NF + 4);
 #pragma unroll
   for (int q = 0; q < 4; q++) {
     if constexpr (W_KC) {
 #pragma unroll
-      for (int f = 0; f < 2; f++)
+      for (int f = 0; f < NF; f++)
         *reinterpret_cast<f32x4*>(row + 32 * f + 8 * q + 4 * lh) =
             f32x4{acc[f][4 * q], acc[f][4 * q + 1], acc[f][4 * q + 2], acc[f][4 * q + 3]};
     } else {
@@ -303,7 +306,7 @@ __global__ __launch_bounds__(kDirThreads, 2) void direct_fwd_kernel(const RowsPa
 #pragma unroll
       for (int i = 0; i < 16; i++) acc[f][i] = 0.f;
     if (wave < nsteps) {                    // two steps in flight: the next one is fetched before this one is multiplied
-      DirectStep s0, s1;
+      DirectStep<> s0, s1;
       ld.load(s0, klo + wave * STEP, khi);
       for (int s = wave; s < nsteps; s += 2 * kDirWaves) {
         const int s_b = s + kDirWaves, s_c = s + 2 * kDirWaves;

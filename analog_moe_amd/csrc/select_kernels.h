@@ -2,7 +2,7 @@
 // entropy regulariser of the mean expert usage; and its backward pass.  One wave per token row, a lane owns the
 // experts lane, lane + 64, ...  (PER of them: 1, 2, 4 or 8, the kernels are instantiated per count).
 #pragma once
-#include "common.h"
+#include "select_rank.h"
 
 namespace amoe {
 
@@ -21,56 +21,6 @@ __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) v = fmaxf(v, wave_shfl_xor(v, d));
   return v;
-}
-
-// The gate value as the tensor expression sigmoid(logits) holds it: computed in fp32, stored in T.
-template <typename T>
-__device__ __forceinline__ float gate_value(float x) {
-  return Elem<T>::to_f32(Elem<T>::cvt(1.0f / (1.0f + expf(-x))));
-}
-
-// The k largest of a row's gate values s (lane owns the experts lane, lane + 64, ...; NaN: never chosen): an expert's
-// place is the number of experts with a larger value, or with the same value and a lower id.  Gate values are not
-// negative, so their bit patterns order as they do; 0 marks what cannot be chosen.
-template <typename T, int PER>
-__device__ __forceinline__ void select_by_rank(const float (&s)[PER], int lane, int E, int k, T* __restrict__ val,
-                                               int64_t* __restrict__ idx) {
-  uint32_t key[PER];
-  int place[PER], n = 0;
-#pragma unroll
-  for (int j = 0; j < PER; j++) {
-    key[j] = s[j] >= 0.f ? as_u32(s[j]) + 1u : 0u;
-    place[j] = 0;
-    n += popc64(wave_ballot(key[j] != 0u));
-  }
-#pragma unroll
-  for (int jj = 0; jj < PER; jj++) {
-    const int here = E - 64 * jj < 64 ? E - 64 * jj : 64;
-#pragma unroll 8
-    for (int l = 0; l < here; l++) {
-      const uint32_t other = wave_read(key[jj], l);
-#pragma unroll
-      for (int j = 0; j < PER; j++) {
-        const bool lower_id = jj < j || (jj == j && l < lane);
-        place[j] += other > key[j] - (lower_id ? 1u : 0u) ? 1 : 0;
-      }
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < PER; j++)
-    if (key[j] != 0u && place[j] < k) {
-      val[place[j]] = Elem<T>::cvt(s[j]);
-      idx[place[j]] = lane + 64 * j;
-    }
-  if (lane >= n && lane < k) {                    // fewer than k experts can be chosen
-    val[lane] = Elem<T>::cvt(-__builtin_inff());
-    idx[lane] = 0x7fffffff;
-  }
-  for (int t = 64 + lane; t < k; t += 64)
-    if (t >= n) {
-      val[t] = Elem<T>::cvt(-__builtin_inff());
-      idx[t] = 0x7fffffff;
-    }
 }
 
 // sel_val / sel_idx [rows, k]: the k largest gate values of each row in descending order, ties to the lower

@@ -27,7 +27,7 @@ import torch.nn.functional as F
 from torch import Tensor, nn
 
 from .config import (AIHWKITTorchInferenceRPUConfig, TorchInferenceRPUConfig, enum_name, kernel_inp_res)
-from .cvmm import CVMM, AnalogExt, CVMMSel, cvmm_prepare_sel2, cvmm_std
+from .cvmm import CVMM, AnalogExt, CVMMSel, _abs_max_wanted, cvmm_prepare_sel2, cvmm_std
 from . import library  # noqa: F401  (registers the amoe:: operators)
 from . import ops
 from .ffn import FFNConfig, moe_ffn
@@ -115,6 +115,9 @@ class SigmaMoELayer(nn.Module):
     # -- router ------------------------------------------------------------------------------------
     def select(self, x: Tensor) -> Tuple[Tensor, Tensor, Tensor]:
         """Gate values and expert ids [..., k] of the top-k experts, and the regularisation loss."""
+        fused = self._select_at_inference(x)
+        if fused is not None:
+            return fused
         logits = self.expert_sel(x)
         if self._fused_select(logits):
             # sigmoid, top-k and the regulariser in one pass over the logits (and one for their gradient)
@@ -135,6 +138,10 @@ class SigmaMoELayer(nn.Module):
         if self.activation_after_topk:
             sel_val = self._sel_activation(sel_val)
         return sel_val, sel_idx, reg_loss
+
+    def _select_at_inference(self, x: Tensor):
+        """``select`` of an analog layer in eval mode without gradients as one launch; None where it does not apply."""
+        return None
 
     def _fused_select(self, logits: Tensor) -> bool:
         """The plain router (sigmoid before top-k, no expert dropout) on the GPU takes the fused kernels."""
@@ -292,6 +299,20 @@ class AnalogLinear(nn.Module):
 
     def extra_repr(self) -> str:
         return f"in_features={self.in_features}, out_features={self.out_features}, tiles={self.n_tiles}"
+
+
+def _plain(t: Tensor) -> bool:
+    """A tensor whose memory a kernel may read behind torch's back: no subclass, no function transform around it, no
+    dispatch mode that wants to see the operators."""
+    return type(t) in (Tensor, nn.Parameter) and torch._C._functorch.peek_interpreter_stack() is None \
+        and torch._C._len_torch_dispatch_stack() == 0 and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+
+
+def _observed(m: nn.Module) -> bool:
+    """Whether somebody hooked the call of m."""
+    g = nn.modules.module
+    return bool(m._forward_hooks or m._forward_pre_hooks or g._global_forward_hooks or g._global_forward_pre_hooks
+                or "forward" in m.__dict__)
 
 
 _LIGHTNING_MODIFIERS = ("DISCRETIZE", "DISCRETIZE_PER_CHANNEL", "ADD_NORMAL", "ADD_NORMAL_PER_CHANNEL",
@@ -625,6 +646,33 @@ class AnalogSigmaMoELayer(SigmaMoELayer):
         return res
 
     # -- fused path ---------------------------------------------------------------------------------------
+    def _select_at_inference(self, x: Tensor):
+        router = self.expert_sel
+        # eval mode, eager, no gradient or function transform, nothing between the router's call and its result
+        if self.training or type(router) is not AnalogLinear or router.training or torch.is_grad_enabled() \
+                or torch.compiler.is_compiling() or torch.is_autocast_enabled() or _observed(router) or not _plain(x):
+            return None
+        cfg, w, ir = router.rpu_config, router.weight, router.input_range
+        fwd = cfg.forward
+        if ir is None or not x.is_cuda or not (w.dtype == ir.dtype == x.dtype) or not (w.is_cuda and ir.is_cuda) \
+                or not (_plain(w) and _plain(ir)) or w.stride(1) != 1 or not ir.is_contiguous() or x.numel() == 0 \
+                or x.shape[-1] != router.in_features or bool(getattr(fwd, "is_perfect", False)) \
+                or bool(getattr(fwd, "out_noise_per_channel", False)) \
+                or (cfg.modifier.enable_during_test and enum_name(cfg.modifier.type) not in ("NONE", "COPY")) \
+                or _abs_max_wanted(cfg.pre_post.input_range, fwd) or self.selection_mode != "sigmoid" or self.activation_after_topk \
+                or self.n_heads > self.n_experts or x.dtype not in (torch.float32, torch.bfloat16, torch.float16):
+            return None
+        res = kernel_inp_res(fwd.inp_res)
+        if not res > 0:
+            return None
+        x2 = ops._rows2d(x)
+        got = ops.router_fwd(x2, w, ir, self.n_heads, router.bounds, res, float(getattr(fwd, "out_bound", -1)),
+                             float(getattr(fwd, "out_res", -1)))
+        if got is None:
+            return None
+        lead = x.shape[:-1]
+        return got[0].view(*lead, self.n_heads), got[1].view(*lead, self.n_heads), x.new_zeros(())
+
     def _fusable(self) -> bool:
         return (self.activation is F.relu and self.bias is None and self.dropout == 0 and
                 self.input_range is not None and not self._row_abs_max_on() and

@@ -6,6 +6,7 @@ There is no CPU path and no fallback: the library must have been built
 """
 from __future__ import annotations
 
+import ctypes
 import functools
 import os
 from typing import Optional, Sequence, Tuple
@@ -459,6 +460,25 @@ def select_fwd(logits: torch.Tensor, k: int, want_reg: bool):
         reg = torch.empty(0, dtype=torch.float32, device=lg.device)
         reg_c = torch.empty(0, dtype=torch.float32, device=lg.device)
     return sel_val, sel_idx, reg, reg_c
+
+
+def router_fwd(x: torch.Tensor, w: torch.Tensor, ir: torch.Tensor, k: int, bounds, inp_res: float, out_bound: float,
+               out_res: float):
+    """The analog router without noise as one launch: gate values [T, k] and expert ids [T, k] of x [T, D] for the weight
+    w [E, D] and its input range per K-tile ir (of x's type).  None where the library has no such kernel for the call."""
+    _need_gpu(x, w, ir)
+    T, E = x.shape[0], w.shape[0]
+    sel_val = torch.empty((T, k), dtype=x.dtype, device=x.device)
+    sel_idx = torch.empty((T, k), dtype=torch.int64, device=x.device)
+    lib = get_lib()
+    b = (0, x.shape[1]) if bounds is None else tuple(bounds)
+    rc = lib.amoe_router_fwd(raw.dtype_code(x), x.data_ptr(), x.stride(0), T, x.shape[1], w.data_ptr(), w.stride(0), E, k,
+                             ir.data_ptr(), len(b) - 1, ctypes.addressof(_abi.bounds_array(b)), inp_res, out_bound, out_res,
+                             sel_val.data_ptr(), sel_idx.data_ptr(), _stream(x))
+    if rc == _abi.AMOE_EUNSUPPORTED:
+        return None
+    _abi.check(lib, rc, "amoe_router_fwd")
+    return sel_val, sel_idx
 
 
 def select_bwd(logits: torch.Tensor, sel_idx: torch.Tensor, grad_val: Optional[torch.Tensor],

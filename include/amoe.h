@@ -383,6 +383,15 @@ int amoe_select_bwd(int32_t dtype, const void* logits, int64_t T, int32_t E, int
                     const int64_t* sel_idx, const void* grad_val, const float* reg_c,
                     const float* grad_reg, void* grad_logits, void* stream);
 
+/* The whole analog router at inference, one launch: logits = x [T, D] @ w [E, D]^T through the stages of
+ * amoe_cvmm_fwd (input range ir [n_tiles] in the element type, DAC, ADC relative to max |w|, no noise), then sel_val /
+ * sel_idx as amoe_select_fwd gives them.  Up to 128 experts and 1, 2, 4 or 8 K-tiles, inp_res > 0, rows of x and w at
+ * 4-byte multiples; otherwise AMOE_EUNSUPPORTED (use the single calls). */
+int amoe_router_fwd(int32_t dtype, const void* x, int64_t ldx, int64_t T, int32_t D, const void* w,
+                    int64_t ldw, int32_t E, int32_t k, const void* ir, int32_t n_tiles,
+                    const int32_t* bounds, float inp_res, float out_bound, float out_res,
+                    void* sel_val, int64_t* sel_idx, void* stream);
+
 /* ---------------------------------------------------------------------------------------
  * The whole expert feed-forward of a layer, one call per direction: everything between a routing decision and the
  * layer's output (moe_layer_aihwkit_lightning.py:384-410, 494-506: sort, up-projection, ReLU, down-projection, gate

@@ -363,3 +363,9 @@ def test_forward_small_tiles(emu_ops, dtype, K, N, kc, tiles, stages):
 @pytest.mark.parametrize("T,E,k", [(5, 64, 64), (3, 65, 1), (3, 128, 2), (2, 128, 128), (3, 7, 3)])
 def test_select_rows(emu_ops, T, E, k):
     util.check_select_rows(emu_ops, "cpu", torch.bfloat16, T, E, k)
+
+
+@pytest.mark.parametrize("dtype,T,D,E,k,tiles,adc", [
+    (torch.bfloat16, 9, 76, 16, 4, 1, True), (torch.float32, 33, 130, 66, 8, 2, True), (torch.float16, 3, 520, 128, 2, 4, False)])
+def test_router_in_one_launch(emu_ops, dtype, T, D, E, k, tiles, adc):
+    util.check_router(emu_ops, "cpu", dtype, T, D, E, k, tiles, adc)

@@ -816,3 +816,33 @@ def test_fused_router_epilogue_equals_the_tensor_expression(dtype):
     assert torch.allclose(g1, g0, rtol=10 * tol, atol=10 * tol * g0.abs().max().item())
     layer.eval()
     assert float(layer.select(x)[2]) == 0.0
+
+
+def test_router_at_inference_takes_one_launch_where_nobody_watches(monkeypatch):
+    """Eval mode without gradients: the same decision as the router's single calls; hooks, gradients, training and a
+    weight modifier during tests keep those calls."""
+    from analog_moe_amd import config as cfgmod, ops
+    layer = _layer(cfgmod, {}, E=16, k=4, out_bound=12.0, out_res=254)
+    x = torch.randn(3, 50, layer.k_dim, device="cuda")
+    calls = []
+    real = ops.router_fwd
+    monkeypatch.setattr(ops, "router_fwd", lambda *a: calls.append(1) or real(*a))
+    layer.eval()
+    with torch.no_grad():
+        val, idx, reg = layer.select(x)
+        assert calls and val.shape == idx.shape == (3, 50, layer.n_heads) and reg.shape == ()
+        calls.clear()
+        seen = []
+        h = layer.expert_sel.register_forward_hook(lambda m, a, out: seen.append(out.shape))
+        v2, i2, _ = layer.select(x)
+        h.remove()
+        assert seen and not calls and (i2 == idx).float().mean() > 0.99 and torch.allclose(v2, val, atol=2e-2)
+        layer.rpu_config.modifier.enable_during_test = True
+        layer.rpu_config.modifier.type = cfgmod.WeightModifierType.ADD_NORMAL
+        layer.select(x)
+        layer.rpu_config.modifier.type = cfgmod.WeightModifierType.NONE
+        layer.train()
+        layer.select(x)
+        layer.eval()
+    layer.select(x)[0].sum().backward()
+    assert not calls and layer.expert_sel.weight.grad is not None

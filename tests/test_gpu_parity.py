@@ -369,3 +369,10 @@ def test_forward_small_tiles(ops, dtype, K, N, kc, tiles, stages, copies):
 @pytest.mark.parametrize("T,E,k", [(1, 64, 8), (2047, 64, 64), (2051, 128, 1), (2051, 128, 2), (16389, 16, 4), (300, 65, 65)])
 def test_select_rows(ops, dtype, T, E, k):
     util.check_select_rows(ops, "cuda", dtype, T, E, k)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,D,E,k,tiles,adc", [(1, 1024, 64, 8, 1, True), (2049, 412, 16, 4, 1, True), (4100, 1024, 64, 8, 2, True),
+                                               (8200, 520, 128, 128, 8, False), (77, 2050, 65, 1, 4, True), (31, 4, 1, 1, 1, True)])
+def test_router_in_one_launch(ops, dtype, T, D, E, k, tiles, adc):
+    util.check_router(ops, "cuda", dtype, T, D, E, k, tiles, adc)

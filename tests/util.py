@@ -748,3 +748,31 @@ def check_select_rows(ops, device, dtype, T, E, k):
         np.testing.assert_allclose(val[t, :m], -np.sort(-np.where(np.isnan(gate[t]), -1.0, gate[t]))[:m], rtol=tol)
         tied = val[t, 1:m] == val[t, : max(m - 1, 0)]
         assert np.all(val[t, 1:m] <= val[t, : max(m - 1, 0)]) and np.all(np.diff(idx[t, :m])[tied] > 0)
+
+
+def check_router(ops, device, dtype, T, D, E, k, tiles, adc=True):
+    """The router's single launch against the calls it stands for: product with max |W|, then top-k.  The partial sums
+    of a K-tile split are added in another order, so a logit may differ by an ulp of its type or, with the ADC, sit on
+    the other side of a step: the chosen experts must agree but for such logits."""
+    g = torch.Generator().manual_seed(T + D + E)
+    x = torch.randn(T, D, generator=g).to(dtype).to(device)
+    w = (torch.randn(E, D, generator=g) / D ** 0.5).to(dtype).to(device)
+    ir = torch.linspace(1.5, 2.5, tiles).to(dtype).to(device)
+    bounds = None if tiles == 1 else [D // (4 * tiles) * 4 * t for t in range(tiles)] + [D]
+    kw = dict(out_bound=12.0, out_res=254.0) if adc else {}
+    got = ops.router_fwd(x, w, ir, k, bounds, 1.0 / 127.0, kw.get("out_bound", -1.0), kw.get("out_res", -1.0))
+    zeros = torch.zeros(T, dtype=torch.int32, device=device)
+    rows = torch.arange(T, dtype=torch.int32, device=device)
+    wv = w.t().unsqueeze(0)
+    logits = ops.cvmm_fwd(x, wv, zeros, torch.tensor([0, T], dtype=torch.int32, device=device), rows, None, T,
+                          ir=ir.float().reshape(1, tiles), ir_by_expert=True, inp_res=1.0 / 127.0, bounds=bounds,
+                          wmax=ops.weight_abs_max(wv.contiguous(), False), **kw)
+    val, idx, _, _ = ops.select_fwd(logits, k, False)
+    assert got[0].shape == val.shape and got[1].dtype == idx.dtype
+    # two orders of a sum of D products differ by less than 1e-5 of its size: that carries one logit in 1e-5 / (half an
+    # ulp of the type) across a rounding boundary (0.5 % in bf16, 4 % in fp16), and each can move three places of its row
+    moved = (got[1] != idx).float().mean().item()
+    assert moved <= {torch.float32: 0.01, torch.bfloat16: 0.02, torch.float16: 0.12}[dtype] + 2.0 / idx.numel()
+    gap = (got[0].float() - val.float()).abs().max().item()
+    step = 12.0 * w.float().abs().max().item() / 127.0 * 2.5 * tiles if adc else 1e-5
+    assert gap <= 0.25 * step + {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
