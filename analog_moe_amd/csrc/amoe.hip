@@ -163,18 +163,29 @@ int amoe_fwd_codes_supported(const amoe_fwd_args* a) {
   return 1;
 }
 
-// Whether the launch is small enough for the kernel that splits a 32 x 64 tile's contraction over its waves
-// (gemm_direct.h).  It re-reads weights per 32 rows and rows per 64 columns, so what counts is how often the chip has to
-// be filled with such tiles.  Measured, this kernel against the tiled ones: up to one tile per CU 2 to 6 times faster
-// (64 columns of 1024 features, 2048 rows: 11.1 against 41.1 us; 48 tokens of 64 experts, 1024 x 256: 18.5 against 38.7);
-// at 640 tiles 29.7 against 41.0 us, at 1150 tiles 47.6 against 43.3 (16-bit); fp32, whose tiled kernel is farther from
-// the matrix rate: 544 tiles 36.9 against 52.8 us, 2100 tiles 105 against 85 - 104.
-// A contraction of 256 with columns in groups of 256 stays with the weights-in-registers kernel and its twins.
-static bool direct_pays(const amoe_fwd_args* a, bool w_kc) {
-  if (a->dtype != AMOE_F32 && !w_kc && a->K == kWsK && a->N % 256 == 0) return false;
-  const int64_t rows = a->M / kDirRows + (a->E < a->M ? a->E : a->M) / 2;      // an expert's last tile is half full
-  const int64_t tiles = (rows + 1) * ((a->N + kDirCols - 1) / kDirCols);
-  return tiles <= (a->dtype == AMOE_F32 ? 6 : 4) * (int64_t)num_compute_units();
+// Which kernel of gemm_direct.h takes the launch: one wave per 32 x 64 tile, eight waves per tile, or none.
+//
+// Against the tiled kernels: these re-read weights per 32 rows and rows per 64 columns.  In fp32, and where the tiled kernel
+// would run its element-wise edge code, one wave per tile was faster wherever measured (fp32, 16 experts k = 4, 2048 tokens
+// 412 -> 128: 26.8 against 53.7 us, 32768 tokens 183 against 196; bf16, 8192 tokens 128 -> 412: 38 against 73, 1024 -> 320 in two K-tiles
+// 112 against 284).  Edge-free 16-bit launches go there only while they are small: 512 -> 128 with 544 tiles 18.7 against
+// 21.7 us, with 2176 tiles 39.5 against 28.1.  A contraction of 256 with columns in groups of 256 stays with the
+// weights-in-registers kernel and its twins.
+//
+// One wave or eight: a wave walks its contraction in 5 us + 45 ns (fp32) or 22 ns (16-bit) per element of K; eight waves
+// need 5 us + 12 ns or 6 ns, but fill a CU by themselves, so they do it once per 256 tiles (fp32 412 -> 128, 146 tiles 13.4
+// against 25.0 us, 544 tiles 37.1 against 26.8; bf16 1024 -> 320, 400 tiles 20.3 against 29.9, 1360 tiles 61 against 41.5).
+enum { DIRECT_NO = 0, DIRECT_WAVE = 1, DIRECT_SPLIT = 2 };
+static int direct_choice(const amoe_fwd_args* a, const RowsParams& p, bool w_kc, int mode) {
+  const bool f32 = a->dtype == AMOE_F32;
+  if (!f32 && !w_kc && a->K == kWsK && a->N % 256 == 0) return DIRECT_NO;
+  const int64_t rows = a->M / kDirRows + (a->E < a->M ? a->E : a->M) / 2 + 1;     // an expert's last tile is half full
+  const int64_t tiles = rows * ((a->N + kDirCols - 1) / kDirCols), cus = num_compute_units();
+  const bool edge_free = !f32 && rows_all_interior(p, mode, a->N % kFCols == 0 && !w_kc ? kFBK : Elem<uint16_t>::kBK);
+  if (edge_free && tiles > 3 * cus) return DIRECT_NO;
+  const int64_t rounds = (tiles + cus - 1) / cus, K = a->K;
+  const bool split = f32 ? rounds * (400 + K) * 5 < 2000 + 18 * K : rounds * (900 + K) < 800 + 4 * K;
+  return split ? DIRECT_SPLIT : DIRECT_WAVE;
 }
 
 int amoe_cvmm_fwd(const amoe_fwd_args* a, void* stream) {
@@ -243,8 +254,8 @@ int amoe_cvmm_fwd(const amoe_fwd_args* a, void* stream) {
              ((long long)a->K * a->w_stride_k + (long long)a->N * a->w_stride_n) * (long long)es < lim;
   const int mode = a->n_tiles > 1 ? MODE_FWD_SPLIT : MODE_FWD;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (direct_pays(a, w_kc)) {
-    const int rc = launch_direct(p, w_kc, a, st);
+  if (const int direct = direct_choice(a, p, w_kc, mode)) {
+    const int rc = launch_direct(p, w_kc, a, direct == DIRECT_SPLIT, st);
     if (rc != AMOE_EUNSUPPORTED) return rc;
   }
   if (a->dtype != AMOE_F32 && !w_kc) {

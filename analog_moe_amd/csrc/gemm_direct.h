@@ -379,4 +379,200 @@ __global__ __launch_bounds__(kDirThreads, 2) void direct_fwd_kernel(const RowsPa
   }
 }
 
+// The same tile and operand path with the whole contraction in ONE wave and nothing shared between waves: for launches
+// of many rows whose contraction or width is short or ends raggedly.  There a 128-row tiled kernel has one workgroup
+// per CU (a wave per SIMD, which waits for its own loads, input stage and matrix instructions in turn) and twice that
+// on the CUs that get the experts' last tiles; 32-row tiles of single waves fill two waves per SIMD and even out.
+// (The tile's operands pass the L1 once per wave: 12 KB per 128-byte step, a third of the 16-bit matrix rate, twice the
+// fp32 one.)  Wave w of the launch takes (row tile w / column blocks, column block w % column blocks).
+constexpr int kDirWaveThreads = 256;
+
+// This wave's row tile: (expert, first sorted position, end position); expert -1: there is none.  No barriers.
+__device__ __forceinline__ void direct_find_wave_tile(const int32_t* __restrict__ offsets, int E, int tile, int& e, int& row0,
+                                                      int& row_end) {
+  const int lane = lane_id();
+  e = -1;
+  row0 = row_end = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {          // 64 experts at a time
+    const int ee = e0 + lane;
+    const int lo = ee < E ? offsets[ee] : 0, hi = ee < E ? offsets[ee + 1] : 0;
+    const int nt = (hi - lo + kDirRows - 1) / kDirRows;
+    int incl = nt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = wave_shfl_up(incl, d);
+      if (lane >= d) incl += up;
+    }
+    const uint64_t past = wave_ballot(incl > tile);
+    if (past != 0) {                            // the first expert whose tiles reach past `tile`
+      const int src = ctz64(past);
+      const int before = (int)wave_read((uint32_t)(incl - nt), src);
+      e = e0 + src;
+      row0 = (int)wave_read((uint32_t)lo, src) + (tile - before) * kDirRows;
+      const int end = (int)wave_read((uint32_t)hi, src);
+      row_end = row0 + kDirRows < end ? row0 + kDirRows : end;
+      return;
+    }
+    tile -= (int)wave_read((uint32_t)incl, 63);
+  }
+}
+
+template <typename T, bool W_KC, bool SPLIT>
+__global__ __launch_bounds__(kDirWaveThreads, 2) void direct_wave_kernel(const RowsParams p) {
+  constexpr bool B16 = sizeof(T) == 2;
+  constexpr int STEP = kDirStep<T>;
+  const int lane = lane_id(), l32 = lane & 31, lh = lane >> 5;
+  const int ncb = p.n_col_blocks;
+  const int id = xcd_contiguous_id(blockIdx.x, gridDim.x) * (kDirWaveThreads / 64) + wave_uniform((int)threadIdx.x >> 6);
+  const int cb = id % ncb;
+  int e, row0, row_end;
+  direct_find_wave_tile(p.offsets, p.E, id / ncb, e, row0, row_end);
+  if (e < 0) return;                            // the same for the whole wave
+  const int c0 = cb * kDirCols, N = p.ND;
+  const bool valid = row0 + l32 < row_end;
+  const int r = valid ? row0 + l32 : row0;
+  const bool has_ir = p.ir != nullptr;
+  const bool quant = p.inp_res > 0.f;
+  const bool codes_mode = B16 && quant;
+  const bool adc_clip = p.out_bound > 0.f, adc_quant = adc_clip && p.out_half_states > 0.f;
+  const bool gen_noise = p.noise_std > 0.f;
+  const uint64_t seed = p.seed + ((gen_noise && p.seed_dev != nullptr) ? *p.seed_dev : 0);
+  const int64_t ir_row = (int64_t)(p.ir_by_expert ? e : r) * p.ir_cols;
+
+  DirectLoader<T, W_KC> ld;
+  ld.lh = lh;
+  ld.xrow = static_cast<const T*>(p.a) + (int64_t)p.a_index[r] * p.lda;
+  const T* __restrict__ W = static_cast<const T*>(p.w) + (int64_t)e * p.w_se;
+  if constexpr (W_KC) {
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+      const int col = c0 + 32 * f + l32;
+      ld.wcol[f] = W + (int64_t)(col < N ? col : N - 1) * p.w_snd;
+    }
+  } else {
+    const int col = c0 + 2 * l32;
+    ld.w_rsrc = make_rsrc(W);
+    ld.w_ks = (uint32_t)(p.w_skd * (int64_t)sizeof(T));
+    ld.w_lane = (uint32_t)(col + 1 < N ? col : N - 2) * (uint32_t)sizeof(T);
+  }
+  DirectDac dac;
+  dac.on = quant && p.a_prequant == 0;
+  dac.res = p.inp_res;
+  dac.resinv = quant ? 1.0f / p.inp_res : 0.f;
+  dac.margin = dac_tie_margin(dac.resinv);
+  const int orow = p.out_index != nullptr ? p.out_index[r] : p.a_index[r];
+  const float wm = p.wmax != nullptr ? p.wmax[e] : 1.f;
+  const float u_nzs = p.noise_std * wm * kNoiseScale, u_bound = p.out_bound * wm;
+  const float u_q = adc_quant ? p.out_half_states / u_bound : 0.f;
+  const float u_qinv = adc_quant ? u_bound / p.out_half_states : 0.f;
+
+  f32x16 acc[2], total[2];
+  for (int t = 0; t < (SPLIT ? p.n_kd_tiles : 1); t++) {
+    const int klo = p.kd_bounds[t], khi = p.kd_bounds[t + 1];
+    const float ir_r = has_ir ? p.ir[ir_row + t] : 1.f;
+    if (dac.on) dac.set_range(ir_r);
+#pragma unroll
+    for (int f = 0; f < 2; f++)
+#pragma unroll
+      for (int i = 0; i < 16; i++) acc[f][i] = 0.f;
+    DirectStep<> s0, s1;
+    ld.load(s0, klo, khi);
+    for (int k0 = klo; k0 < khi; k0 += 2 * STEP) {
+      if (k0 + STEP < khi) ld.load(s1, k0 + STEP, khi);
+      direct_multiply<T, W_KC>(acc, s0, dac);
+      if (k0 + STEP < khi) {
+        if (k0 + 2 * STEP < khi) ld.load(s0, k0 + 2 * STEP, khi);
+        direct_multiply<T, W_KC>(acc, s1, dac);
+      }
+    }
+    // slot (f, 4 * q + j): column 32 * f + i (W_KC) or 2 * i + f of the tile, i = 8 * q + 4 * lh + j
+#pragma unroll
+    for (int f = 0; f < 2; f++) {
+      if (codes_mode) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[f][i] *= p.inp_res;
+      }
+      if (gen_noise) {
+        // The noise of a 32-column block of the output is one product; the columns 2 * i + f of the tile are the even
+        // or odd ones of both blocks: two products, and each slot takes the one of its column's block.
+        const NoiseKey key = noise_key(seed, t);
+        const uint32_t row_key = noise_row_key(key, (uint32_t)orow);
+        const uint32_t col_key = noise_col_key(key, (uint32_t)(c0 + (W_KC ? 32 * f + l32 : 2 * l32 + f)));
+        const uint32_t block = (uint32_t)(c0 >> 5) + (W_KC ? (uint32_t)f : 0u);
+        const i32x16 z = noise_block(row_key, col_key, block, (uint32_t)row0, lh);
+#pragma unroll
+        for (int i = 0; i < (W_KC ? 16 : 8); i++) acc[f][i] = fmaf((float)z[i], u_nzs, acc[f][i]);
+        if constexpr (!W_KC) {
+          const i32x16 z1 = noise_block(row_key, col_key, block + 1u, (uint32_t)row0, lh);
+#pragma unroll
+          for (int i = 8; i < 16; i++) acc[f][i] = fmaf((float)z1[i], u_nzs, acc[f][i]);
+        }
+      }
+      if (adc_clip) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+          float v = clamp_sym(acc[f][i], u_bound);
+          if (adc_quant) v = rintf(v * u_q) * u_qinv;
+          acc[f][i] = v;
+        }
+      }
+      if (has_ir) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) acc[f][i] *= ir_r;
+      }
+      if constexpr (SPLIT) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) total[f][i] = t == 0 ? acc[f][i] : total[f][i] + acc[f][i];
+      }
+    }
+  }
+  if constexpr (SPLIT) {
+    acc[0] = total[0];
+    acc[1] = total[1];
+  }
+  if (!valid) return;                           // nothing of a whole wave follows
+
+  // eight runs of four consecutive columns
+  const float qr = p.xq_out != nullptr ? p.xq_ir[e] : 1.f;
+  const float qrinv = 1.0f / qr, qresinv = 1.0f / p.xq_inp_res, qkq = qrinv * qresinv, qmargin = dac_tie_margin(qresinv);
+#pragma unroll
+  for (int run = 0; run < 8; run++) {
+    float v[4];
+    int oc;
+    if constexpr (W_KC) {
+      const int f = run >> 2, q = run & 3;
+      oc = 32 * f + 8 * q + 4 * lh;
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[j] = acc[f][4 * q + j];
+    } else {
+      const int q = run >> 1, h = run & 1;
+      oc = 16 * q + 8 * lh + 4 * h;
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[j] = acc[j & 1][4 * q + 2 * h + (j >> 1)];
+    }
+    const int col = c0 + oc;
+    int nv = N - col;
+    nv = nv < 0 ? 0 : (nv > 4 ? 4 : nv);
+    if (p.relu) {
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[j] = fmaxf(v[j], 0.f);
+    }
+    if (nv > 0) store4<T>(static_cast<T*>(p.out) + (int64_t)orow * p.ldo + col, v, nv, p.out_vec != 0);
+    if (p.xq_out != nullptr) {                  // the DAC image of the value as stored
+      float tie = 0.f, xc[4], c[4];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        xc[j] = clamp_sym(B16 ? Elem<T>::to_f32(Elem<T>::cvt(v[j])) : v[j], qr);
+        c[j] = dac_code<B16>(xc[j], qr, qrinv, p.xq_inp_res, qresinv, qkq, tie);
+        if (!B16) c[j] *= p.xq_inp_res;
+      }
+      if (B16 && tie > qmargin) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) c[j] = dac_code_exact(xc[j], qr, qrinv, p.xq_inp_res, qresinv);
+      }
+      if (nv > 0) store4<T>(static_cast<T*>(p.xq_out) + (int64_t)orow * p.ldxq + col, c, nv, p.xq_vec != 0);
+    }
+  }
+}
+
 }  // namespace amoe

@@ -4,7 +4,7 @@
 
 namespace amoe {
 
-int launch_direct(const RowsParams& p0, bool w_kc, const amoe_fwd_args* a, hipStream_t st) {
+int launch_direct(const RowsParams& p0, bool w_kc, const amoe_fwd_args* a, bool split_waves, hipStream_t st) {
   RowsParams p = p0;
   const int64_t es = (int64_t)esize(a->dtype);
   // the stages the kernel has: ranges with the input quantiser or neither, one max |W| per expert, generated noise
@@ -20,15 +20,36 @@ int launch_direct(const RowsParams& p0, bool w_kc, const amoe_fwd_args* a, hipSt
   // (a tile for every 32 rows and one more per expert that can have any)
   const int64_t tiles = (int64_t)a->M / kDirRows + (a->E < a->M ? a->E : a->M);
   if (tiles * p.n_col_blocks > 0x7fffffffLL) return AMOE_EUNSUPPORTED;
-  const dim3 grid((unsigned)(tiles * p.n_col_blocks)), block(kDirThreads);
+  const int64_t work = tiles * p.n_col_blocks;
+  if (split_waves) {
+    const dim3 grid((unsigned)work), block(kDirThreads);
 #define AMOE_DIRECT(T)                                                                  \
   do {                                                                                  \
     if (w_kc) hipLaunchKernelGGL((&direct_fwd_kernel<T, true>), grid, block, 0, st, p); \
     else hipLaunchKernelGGL((&direct_fwd_kernel<T, false>), grid, block, 0, st, p);     \
   } while (0)
-  if (a->dtype == AMOE_F32) AMOE_DIRECT(float);
-  else if (a->dtype == AMOE_F16) AMOE_DIRECT(f16_t);
-  else AMOE_DIRECT(uint16_t);
+    if (a->dtype == AMOE_F32) AMOE_DIRECT(float);
+    else if (a->dtype == AMOE_F16) AMOE_DIRECT(f16_t);
+    else AMOE_DIRECT(uint16_t);
+#undef AMOE_DIRECT
+    return launch_rc();
+  }
+  constexpr int kWaves = kDirWaveThreads / 64;
+  const dim3 grid((unsigned)((work + kWaves - 1) / kWaves)), block(kDirWaveThreads);
+#define AMOE_DIRECT(T, SPLIT)                                                                   \
+  do {                                                                                          \
+    if (w_kc) hipLaunchKernelGGL((&direct_wave_kernel<T, true, SPLIT>), grid, block, 0, st, p); \
+    else hipLaunchKernelGGL((&direct_wave_kernel<T, false, SPLIT>), grid, block, 0, st, p);     \
+  } while (0)
+#define AMOE_DIRECT_T(T)                    \
+  do {                                      \
+    if (a->n_tiles > 1) AMOE_DIRECT(T, true); \
+    else AMOE_DIRECT(T, false);             \
+  } while (0)
+  if (a->dtype == AMOE_F32) AMOE_DIRECT_T(float);
+  else if (a->dtype == AMOE_F16) AMOE_DIRECT_T(f16_t);
+  else AMOE_DIRECT_T(uint16_t);
+#undef AMOE_DIRECT_T
 #undef AMOE_DIRECT
   return launch_rc();
 }

@@ -109,7 +109,8 @@ inline int launch_rows(int dtype, const RowsParams& p, bool w_kc, int mode, int 
 // gemm_fwd256.hip, gemm_bwdx256.hip: the tiled kernels of the training shapes and the weights-in-registers kernel
 // (16-bit types).  AMOE_EUNSUPPORTED: not one of their launches, the general kernel runs it.
 int launch_fwd256(const RowsParams& p, int mode, const amoe_fwd_args* a, hipStream_t st);
-int launch_direct(const RowsParams& p, bool w_kc, const amoe_fwd_args* a, hipStream_t st);   // gemm_direct.hip
+// gemm_direct.hip: small tiles; split_waves: a tile's contraction over the waves of a workgroup, else one wave per tile
+int launch_direct(const RowsParams& p, bool w_kc, const amoe_fwd_args* a, bool split_waves, hipStream_t st);
 int launch_bwdx256(const RowsParams& p, const amoe_bwd_x_args* a, hipStream_t st, int* n_count_blocks, int* block_cols);
 
 }  // namespace amoe

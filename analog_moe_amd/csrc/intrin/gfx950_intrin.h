@@ -110,6 +110,7 @@ __device__ __forceinline__ V wave_shfl(V v, int src) { return __shfl(v, src, 64)
 template <typename V>
 __device__ __forceinline__ V wave_shfl_up(V v, int d) { return __shfl_up(v, d, 64); }
 __device__ __forceinline__ uint64_t wave_ballot(bool p) { return __ballot(p); }
+__device__ __forceinline__ int ctz64(uint64_t v) { return __builtin_ctzll(v); }
 __device__ __forceinline__ int popc64(uint64_t v) { return __popcll(v); }
 // Orders this wave's LDS accesses before the barrier against those after it.
 __device__ __forceinline__ void wave_sync() {

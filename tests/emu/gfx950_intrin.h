@@ -66,6 +66,7 @@ inline uint64_t wave_ballot(bool p) {
   w->bar.arrive_and_wait();
   return m;
 }
+inline int ctz64(uint64_t v) { return __builtin_ctzll(v); }
 inline int popc64(uint64_t v) { return __builtin_popcountll(v); }
 inline void wave_sync() { emu_wave->bar.arrive_and_wait(); }
 

@@ -358,6 +358,7 @@ def test_layer_calls_equal_the_single_calls(emu_ops, case):
     (torch.float32, 301, 34, False, 1, "noisy"), (torch.float32, 36, 61, True, 2, "dac")])
 def test_forward_small_tiles(emu_ops, dtype, K, N, kc, tiles, stages):
     util.check_forward_small_tiles(emu_ops, "cpu", dtype, K, N, kc, tiles, stages)
+    util.check_forward_small_tiles(emu_ops, "cpu", dtype, K, N, kc, tiles, stages, copies=3)     # one wave per tile
 
 
 @pytest.mark.parametrize("T,E,k", [(5, 64, 64), (3, 65, 1), (3, 128, 2), (2, 128, 128), (3, 7, 3)])

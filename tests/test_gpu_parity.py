@@ -354,7 +354,7 @@ def test_layer_calls_equal_the_single_calls(ops, case):
     util.check_layer_calls(ops, case, "cuda")
 
 
-# copies 1: the kernel for small launches; 400: the tiled ones, on the same edges
+# copies 1: a tile's contraction over eight waves; 400: one wave per tile, or the tiled kernels where they are edge-free
 @pytest.mark.parametrize("copies", [1, 400])
 @pytest.mark.parametrize("kc,tiles,stages", [(False, 1, "plain"), (False, 2, "noisy"), (True, 1, "noisy"), (True, 2, "dac")])
 @pytest.mark.parametrize("dtype,K,N", [(torch.bfloat16, 412, 64), (torch.bfloat16, 130, 66), (torch.float16, 1088, 2),
