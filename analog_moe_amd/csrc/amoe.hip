@@ -276,6 +276,32 @@ size_t amoe_bwd_x_workspace(int64_t M, int32_t K, int32_t n_tiles) {
   return (size_t)(col_blocks * (M > 0 ? M : 1)) * sizeof(float) + (size_t)(row_tiles * col_blocks) * sizeof(int32_t);
 }
 
+// Plain input gradients (no mask, gate or range) in fp32 or with edges, up to a wave per SIMD: the forward product with
+// contraction-contiguous weights, one wave per 32 x 64 tile.  Always one wave: it adds in the tiled kernel's order, so
+// that the clip applied by the sum over the heads gives the masked launch's result bit for bit.  With more tiles the
+// tiled kernel's shared operands win.  us per launch, tiled and direct, contraction -> columns:
+//   fp32  64 -> 132, 963 tiles 16.5 / 13.0; 128 -> 412, 483 tiles 16.4 / 12.1; 256 -> 1028, 629 tiles 28.4 / 19.5;
+//         516 -> 2044, 672 tiles 51.5 / 31.8; but 128 -> 412, 2247 tiles 27.5 / 29.1; 516 -> 2044, 1184 tiles 53.2 / 53.8
+//   bf16  64 -> 132, 579 tiles 7.0 / 6.1; 516 -> 2044, 672 tiles 24.8 / 16.6; 256 -> 1028, 629 tiles 11.0 / 10.8; but
+//         1173 tiles 12.0 / 17.3; 128 -> 412, 1351 tiles 11.1 / 12.7
+static bool bwdx_direct(const amoe_bwd_x_args* a, const RowsParams& p) {
+  if (bwdx_reads_x(a) || a->ir || a->relu_mask || a->gate || a->xc_out) return false;
+  const int64_t rows = a->M / kDirRows + (a->E < a->M ? a->E : a->M) / 2 + 1;     // an expert's last tile is half full
+  if (rows * ((a->K + kDirCols - 1) / kDirCols) > 4 * num_compute_units()) return false;
+  return a->dtype == AMOE_F32 || !rows_all_interior(p, MODE_BWDX, Elem<uint16_t>::kBK);
+}
+
+static int launch_bwdx_direct(const amoe_bwd_x_args* a, const RowsParams& p, hipStream_t st) {
+  amoe_fwd_args f{};
+  f.dtype = a->dtype;
+  f.M = a->M; f.K = a->N; f.N = a->K; f.E = a->E;
+  f.x = a->g; f.ldx = a->ldg;
+  f.w = a->w; f.w_stride_e = a->w_stride_e; f.w_stride_k = 1; f.w_stride_n = a->w_stride_k;
+  f.n_tiles = 1; f.tile_bounds[1] = a->N;
+  f.inp_res = -1.f;
+  return launch_direct(p, true, &f, false, st);
+}
+
 int amoe_cvmm_bwd_x(const amoe_bwd_x_args* a, void* stream) {
   if (!a) return AMOE_ENULL;
   if (a->dtype != AMOE_F32 && a->dtype != AMOE_BF16 && a->dtype != AMOE_F16) return AMOE_EINVAL;
@@ -327,8 +353,8 @@ int amoe_cvmm_bwd_x(const amoe_bwd_x_args* a, void* stream) {
   p.xf_vec = a->x && aligned(a->x, 16) && (a->ldx % 4 == 0) && bounds_multiple_of(a->n_tiles, a->tile_bounds, 4);
   hipStream_t st = static_cast<hipStream_t>(stream);
   int block_cols = kTileCols, n_count_blocks = grid;
-  int rc = AMOE_EUNSUPPORTED;
-  if (a->dtype != AMOE_F32) {
+  int rc = bwdx_direct(a, p) ? launch_bwdx_direct(a, p, st) : AMOE_EUNSUPPORTED;
+  if (rc == AMOE_EUNSUPPORTED && a->dtype != AMOE_F32) {
     int cols = kTileCols;
     rc = launch_bwdx256(p, a, st, &n_count_blocks, &cols);
     if (rc == AMOE_OK) block_cols = cols;

@@ -165,12 +165,29 @@ __device__ __forceinline__ void direct_multiply(f32x16 (&acc)[NF], DirectStep<NF
       }
 #pragma unroll
       for (int f = 0; f < NF; f++) acc[f] = mfma_32x32x16<T>(wf[f], s.x[i], acc[f]);
+    } else if constexpr (W_KC) {
+      // A half wave holds four consecutive indices; with the halves' odd and even words exchanged an instruction takes
+      // two consecutive ones, in order: the sums come out as the tiled kernel's, bit for bit.
+      uint32_t x[4] = {s.x[i][0], s.x[i][1], s.x[i][2], s.x[i][3]};
+      swap_half_waves(x[0], x[1]);
+      swap_half_waves(x[2], x[3]);
+#pragma unroll
+      for (int f = 0; f < NF; f++) {
+        swap_half_waves(s.w[i][4 * f], s.w[i][4 * f + 1]);
+        swap_half_waves(s.w[i][4 * f + 2], s.w[i][4 * f + 3]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int d = j == 0 ? 0 : j == 1 ? 2 : j == 2 ? 1 : 3;      // words of indices 2 * j and 2 * j + 1
+#pragma unroll
+        for (int f = 0; f < NF; f++) acc[f] = mfma_32x32x2_f32(as_f32(s.w[i][4 * f + d]), as_f32(x[d]), acc[f]);
+      }
     } else {
 #pragma unroll
       for (int j = 0; j < 4; j++)
 #pragma unroll
         for (int f = 0; f < NF; f++)
-          acc[f] = mfma_32x32x2_f32(as_f32(W_KC ? s.w[i][4 * f + j] : s.w[i][2 * j + f]), as_f32(s.x[i][j]), acc[f]);
+          acc[f] = mfma_32x32x2_f32(as_f32(s.w[i][2 * j + f]), as_f32(s.x[i][j]), acc[f]);
     }
   }
 }

@@ -101,6 +101,12 @@ __device__ __forceinline__ uint32_t pack_low_halves(uint32_t hi, uint32_t lo) {
 __device__ __forceinline__ int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 // value held by lane `src` (the same for the whole wave), as a scalar
 __device__ __forceinline__ uint32_t wave_read(uint32_t v, int src) { return (uint32_t)__builtin_amdgcn_readlane((int)v, src); }
+// The upper half wave's a and the lower half wave's b change places.
+__device__ __forceinline__ void swap_half_waves(uint32_t& a, uint32_t& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
 __device__ __forceinline__ int lane_id() { return threadIdx.x & 63; }
 
 template <typename V>

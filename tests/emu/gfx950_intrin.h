@@ -53,6 +53,11 @@ template <class V> inline V emu_exchange(V v, int src) {
 template <class V> inline V wave_shfl_xor(V v, int mask) { return emu_exchange(v, lane_id() ^ mask); }
 template <class V> inline V wave_shfl(V v, int src) { return emu_exchange(v, src); }
 inline uint32_t wave_read(uint32_t v, int src) { return emu_exchange(v, src); }
+inline void swap_half_waves(uint32_t& a, uint32_t& b) {
+  const bool upper = lane_id() >= 32;
+  const uint32_t got = emu_exchange(upper ? a : b, lane_id() ^ 32);
+  (upper ? a : b) = got;
+}
 template <class V> inline V wave_shfl_up(V v, int d) {
   int l = lane_id();
   return emu_exchange(v, l >= d ? l - d : l);

@@ -361,6 +361,11 @@ def test_forward_small_tiles(emu_ops, dtype, K, N, kc, tiles, stages):
     util.check_forward_small_tiles(emu_ops, "cpu", dtype, K, N, kc, tiles, stages, copies=3)     # one wave per tile
 
 
+@pytest.mark.parametrize("dtype,K,N", util.PLAIN_BWDX[:5])
+def test_plain_input_gradient(emu_ops, dtype, K, N):
+    util.check_plain_input_gradient(emu_ops, "cpu", dtype, K, N)
+
+
 @pytest.mark.parametrize("T,E,k", [(5, 64, 64), (3, 65, 1), (3, 128, 2), (2, 128, 128), (3, 7, 3)])
 def test_select_rows(emu_ops, T, E, k):
     util.check_select_rows(emu_ops, "cpu", torch.bfloat16, T, E, k)

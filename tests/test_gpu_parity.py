@@ -365,6 +365,12 @@ def test_forward_small_tiles(ops, dtype, K, N, kc, tiles, stages, copies):
     util.check_forward_small_tiles(ops, "cuda", dtype, K, N, kc, tiles, stages, copies)
 
 
+@pytest.mark.parametrize("copies", [1, 12])
+@pytest.mark.parametrize("dtype,K,N", util.PLAIN_BWDX)
+def test_plain_input_gradient(ops, dtype, K, N, copies):
+    util.check_plain_input_gradient(ops, "cuda", dtype, K, N, copies)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,E,k", [(1, 64, 8), (2047, 64, 64), (2051, 128, 1), (2051, 128, 2), (16389, 16, 4), (300, 65, 65)])
 def test_select_rows(ops, dtype, T, E, k):

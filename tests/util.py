@@ -728,6 +728,35 @@ def check_forward_small_tiles(ops, device, dtype, K, N, kc, tiles, stages, copie
     assert np.array_equal(np32(xq) if dtype != torch.float32 else np.rint(np32(xq) * 127.0), codes)
 
 
+# output columns and contraction of a plain input gradient: ends inside a 64-column block, a 128-byte step, a 4-byte word
+PLAIN_BWDX = [(torch.float32, 65, 37), (torch.float32, 128, 64), (torch.bfloat16, 70, 66), (torch.float16, 412, 34), (torch.bfloat16, 66, 33),
+              (torch.float32, 412, 128), (torch.float32, 256, 516), (torch.bfloat16, 412, 128), (torch.float16, 1, 2)]
+
+
+def check_plain_input_gradient(ops, device, dtype, K, N, copies=1):
+    """g @ W[e]^T without masks on experts that end at the edges of 32-row tiles: against float64, and bit for bit what
+    the launch with an input-range mask gives when nothing is clipped.  Tolerances: one rounding of the result, or N
+    fp32 additions."""
+    g = torch.Generator().manual_seed(K + N)
+    counts = torch.tensor([0, 1, 31, 32, 33, 65]) * copies
+    E, M = len(counts), int(counts.sum())
+    idx = torch.repeat_interleave(torch.arange(E), counts)[torch.randperm(M, generator=g)].reshape(M, 1)
+    _, perm, in_index, offsets = ops.prepare_sel(idx.to(device), E, 1)
+    dy = torch.randn(M, N, generator=g).to(dtype)
+    w = (torch.randn(E, K, N, generator=g) / N ** 0.5).to(dtype)
+    x = torch.rand(M, K, generator=g).to(dtype)
+    got, none = ops.cvmm_bwd_x(dy.to(device), w.to(device), offsets, perm, perm, M)
+    masked, _ = ops.cvmm_bwd_x(dy.to(device), w.to(device), offsets, perm, perm, M, x=x.to(device), xf_index=in_index,
+                               ir=torch.full((E, 1), 2.0, device=device), ir_by_expert=True)
+    assert none is None and torch.equal(got, masked)
+    want = torch.empty(M, K, dtype=torch.float64)
+    for e in range(E):
+        rows = idx[:, 0] == e
+        want[rows] = dy[rows].double() @ w[e].double().t()
+    tol = {torch.float32: N * 2.0 ** -24, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert rel_err(np32(got), want.numpy()) < tol
+
+
 def check_select_rows(ops, device, dtype, T, E, k):
     """Every expert of a row whose gate value is a number, in order (ties to the lower id); the sentinel of a row that
     has fewer than k such values."""
