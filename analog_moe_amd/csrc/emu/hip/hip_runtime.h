@@ -1,5 +1,5 @@
 // CPU stand-in for <hip/hip_runtime.h>, used ONLY by the host-compiled test build of the
-// kernels (tests/emu).  One std::thread per GPU thread, blocks run one after another, so the
+// kernels.  One std::thread per GPU thread, blocks run one after another, so the
 // kernels' own index arithmetic, masking and LDS traffic run unchanged under the host
 // AddressSanitizer.  Nothing in the shipped library includes this file.
 #pragma once

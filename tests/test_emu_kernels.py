@@ -1,5 +1,5 @@
 """CPU parity tests of the HIP kernels' own source, compiled for the host with the stand-in
-headers of tests/emu (one thread per GPU thread).  They check index arithmetic, masking, tile
+headers of csrc/emu (one thread per GPU thread).  They check index arithmetic, masking, tile
 scheduling and the analog pro/epilogues against the oracle without a GPU; the matrix
 instruction and LDS-transpose stand-ins reproduce the operand layouts measured on MI355X.
 The product path is untouched: these tests point analog_moe_amd.ops at the host build by
@@ -16,16 +16,16 @@ from oracle import cvmm_oracle as O
 from tests import util
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-EMU_SO = os.path.join(HERE, "emu", "libamoe_emu.so")
+CSRC = os.path.join(HERE, "..", "analog_moe_amd", "csrc")
+EMU_SO = os.path.join(CSRC, "emu", "libamoe_emu.so")
 
 
 @pytest.fixture(scope="module")
 def emu_ops():
-    src = [os.path.join(HERE, "..", "analog_moe_amd", "csrc", f) for f in os.listdir(
-        os.path.join(HERE, "..", "analog_moe_amd", "csrc")) if f.endswith((".h", ".hip"))]
-    src += [os.path.join(HERE, "emu", "gfx950_intrin.h"), os.path.join(HERE, "emu", "hip", "hip_runtime.h")]
+    src = [os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".h", ".hip"))]
+    src += [os.path.join(CSRC, "emu", "gfx950_intrin.h"), os.path.join(CSRC, "emu", "hip", "hip_runtime.h")]
     if not os.path.exists(EMU_SO) or any(os.path.getmtime(s) > os.path.getmtime(EMU_SO) for s in src):
-        subprocess.run([os.path.join(HERE, "emu", "build_emu.sh")], check=True, capture_output=True)
+        subprocess.run([os.path.join(CSRC, "emu", "build.sh")], check=True, capture_output=True)
     lib = _abi.bind(EMU_SO)
     saved = (ops._LIB, ops._stream, ops._need_gpu)
     ops._LIB, ops._stream, ops._need_gpu = lib, (lambda t: None), (lambda *a: None)

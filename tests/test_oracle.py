@@ -719,7 +719,7 @@ def test_div_by_is_the_correctly_rounded_quotient(tmp_path):
     here = os.path.dirname(os.path.abspath(__file__))
     so = str(tmp_path / "libdivcheck.so")
     subprocess.run(["/opt/rocm/llvm/bin/clang++", "-x", "c++", "-std=c++20", "-O2", "-fPIC", "-shared",
-                    "-ffp-contract=off", "-Wno-psabi", "-I", os.path.join(here, "emu"),
+                    "-ffp-contract=off", "-Wno-psabi", "-I", os.path.join(here, "..", "analog_moe_amd", "csrc", "emu"),
                     "-I", os.path.join(here, "..", "include"), "-I", os.path.join(here, "..", "analog_moe_amd", "csrc"),
                     os.path.join(here, "emu", "div_by_check.cpp"), "-o", so], check=True)
     lib = ctypes.CDLL(so)
