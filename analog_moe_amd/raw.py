@@ -18,11 +18,15 @@ from ._abi import AMOE_BF16, AMOE_F16, AMOE_F32, BwdWArgs, BwdXArgs, FwdArgs, Ks
 DTYPE_CODES = {torch.float32: AMOE_F32, torch.bfloat16: AMOE_BF16, torch.float16: AMOE_F16}
 
 
-def dtype_code(t: torch.Tensor) -> int:
-    code = DTYPE_CODES.get(t.dtype)
+def code_of(dtype: torch.dtype) -> int:
+    code = DTYPE_CODES.get(dtype)
     if code is None:
-        raise TypeError(f"unsupported dtype {t.dtype}: the CVMM kernels take float32, bfloat16 or float16")
+        raise TypeError(f"unsupported dtype {dtype}: the CVMM kernels take float32, bfloat16 or float16")
     return code
+
+
+def dtype_code(t: torch.Tensor) -> int:
+    return code_of(t.dtype)
 
 
 def check_codes_fit(dtype: torch.dtype, res: float, name: str = "inp_res") -> None:

@@ -1,0 +1,49 @@
+"""What the layer calls (``ffn.ffn_forward`` / ``ffn_backward``, and the operators in front of them) do with arguments that
+do not fit: converted where that is exact, refused where the kernels would read something else than the tensor."""
+import dataclasses
+
+import pytest
+import torch
+
+from analog_moe_amd import _abi, ffn
+from tests import util
+from tests.test_emu_kernels import emu_ops  # noqa: F401  (the host build behind analog_moe_amd.ops)
+
+E, D, F, T, K = 3, 32, 24, 10, 2
+
+
+def problem(dtype=torch.float32, **kw):
+    pr = util.make_problem(7, **{**dict(T=T, D=D, E=E, F=F, k=K, dtype=dtype), **kw})
+    pr["ir"] = torch.linspace(1.0, 2.0, 2 * E).reshape(2, E, 1)
+    return pr
+
+
+def forward(pr, cfg, **swap):
+    a = {**pr, **swap}
+    return ffn.ffn_forward(a["x"], a["keys"], a["values"], a["ir"], a["gate"], a["idx"], cfg)
+
+
+def backward(pr, cfg, saved, want_ir_grad=True, ir_dtype=torch.float32, **swap):
+    a = {**pr, **dict(zip(("p1", "z", "perm", "in_index", "offsets", "z_scale", "ir_up", "ir_dn"), saved[1:])), **swap}
+    return ffn.ffn_backward(a["dy"], a["x"], a["keys"], a["values"], a["gate"], a["idx"], a["p1"], a["z"], a["z_scale"],
+                            a["perm"], a["in_index"], a["offsets"], a["ir_up"], a["ir_dn"], cfg, want_ir_grad, ir_dtype)
+
+
+def same(a, b):
+    return all((p is None and q is None) or torch.equal(p, q) for p, q in zip(a, b))
+
+
+PLAIN = ffn.FFNConfig(inp_res=1 / 127)
+ADC = dataclasses.replace(PLAIN, out_bound=12.0, out_res=254.0)
+
+
+def test_input_range_of_another_type(emu_ops):
+    pr = problem()
+    want = forward(pr, PLAIN)
+    got = forward(pr, PLAIN, ir=pr["ir"].double())
+    assert same(got, want)
+    with pytest.raises(TypeError):              # the tables' launch reads the parameter itself
+        forward(pr, ADC, ir=pr["ir"].double())
+    with pytest.raises(TypeError):              # and the per-expert sums are written in its type
+        backward(pr, PLAIN, got, ir_dtype=torch.float64)
+    assert backward(pr, PLAIN, got, want_ir_grad=False, ir_dtype=torch.float64)[3] is None
