@@ -100,7 +100,7 @@ def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype
     return _abi.FFN_ARGS.pack(
         raw.dtype_code(x), x.shape[0], D, E, F, V, gate.shape[-1],
         x.data_ptr(), x.stride(0), keys.data_ptr(), *keys.stride(), values.data_ptr(), *values.stride(),
-        _p(input_range), 0 if ir_dtype is None else raw.code_of(ir_dtype), 0 if input_range is None else input_range.numel() // (2 * E), sel.data_ptr(), sel.dtype == torch.int64, gate.data_ptr(),
+        _p(input_range), 0 if ir_dtype is None else raw.code_of(ir_dtype), 0 if input_range is None else input_range.shape[2], sel.data_ptr(), sel.dtype == torch.int64, gate.data_ptr(),
         cfg.inp_res, cfg.out_bound, cfg.out_res, cfg.noise_std,
         *_bounds(cfg.bounds_up, D), *_bounds(cfg.bounds_down, F), cfg.noise_seed & 0xFFFFFFFFFFFFFFFF, _p(cfg.noise_seed_dev),
         cfg.noise_per_channel, _p(cfg.noise_up), _p(cfg.noise_down), _p(cfg.wmax_up), _p(cfg.wmax_down),
@@ -118,10 +118,11 @@ def _int_ids(sel_idx: torch.Tensor) -> torch.Tensor:
     return sel if sel.is_contiguous() else sel.contiguous()
 
 
-def _range_table(input_range: torch.Tensor, cfg: FFNConfig) -> torch.Tensor:
-    """The parameter as the library reads it.  Types it does not know are converted, but for the launch that makes the
+def _range_table(input_range: torch.Tensor, E: int, cfg: FFNConfig) -> torch.Tensor:
+    """The parameter as the library reads it, [2, E, columns].  Types it does not know are converted, but for the launch that makes the
     range tables together with max |W| and takes the parameter as it is (TypeError)."""
     with_wmax = (cfg.out_bound > 0 or (cfg.noise_std > 0 and cfg.noise_up is None)) and cfg.wmax_up is None
+    input_range = input_range.reshape(2, E, -1)
     if input_range.dtype in raw.DTYPE_CODES or (with_wmax and not cfg.noise_per_channel):
         raw.dtype_code(input_range)
         return _dense(input_range)
@@ -147,7 +148,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
     ir_up = ir_dn = None
     if input_range is not None:
-        input_range = _range_table(input_range, cfg)
+        input_range = _range_table(input_range, E, cfg)
         ir_up, ir_dn = (torch.empty((E, _n_tiles(b)), dtype=torch.float32, device=dev)
                         for b in (cfg.bounds_up, cfg.bounds_down))
     chain = input_range is not None and cfg.inp_res > 0 and _n_tiles(cfg.bounds_down) == 1

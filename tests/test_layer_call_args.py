@@ -47,3 +47,12 @@ def test_input_range_of_another_type(emu_ops):
     with pytest.raises(TypeError):              # and the per-expert sums are written in its type
         backward(pr, PLAIN, got, ir_dtype=torch.float64)
     assert backward(pr, PLAIN, got, want_ir_grad=False, ir_dtype=torch.float64)[3] is None
+
+
+@pytest.mark.parametrize("cfg", [PLAIN, ADC], ids=["plain", "adc"])
+def test_input_range_that_is_no_table_of_both_projections(emu_ops, cfg):
+    pr = problem()
+    with pytest.raises((RuntimeError, ValueError)):
+        forward(pr, cfg, ir=torch.ones(2 * E + 1))
+    with pytest.raises((RuntimeError, ValueError)):            # fewer columns than K-tiles
+        forward(pr, dataclasses.replace(cfg, bounds_up=(0, 16, D)))
