@@ -84,13 +84,13 @@ def _bounds(bounds, K: int):
 
 
 def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype, sel, gate, y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn,
-          grads=(0, 0, 0, 0, 0, 0)) -> bytes:
+          grads=(0, 0, 0, 0, 0, 0), noise=(None, None)) -> bytes:
     """The argument structure of ``amoe_ffn_fwd`` / ``amoe_ffn_bwd``.  All tensors rows-contiguous, x [T, D]."""
     E, D, F = keys.shape
     V = values.shape[2]
-    for t in (cfg.noise_up, cfg.noise_down, cfg.wmax_up, cfg.wmax_down):
+    for t in (cfg.wmax_up, cfg.wmax_down):
         if t is not None and (t.dtype != torch.float32 or not t.is_contiguous()):
-            raise TypeError("injected noise and max |W| tables must be contiguous float32 tensors")
+            raise TypeError("max |W| tables must be contiguous float32 tensors")
     if keys.dtype != x.dtype or values.dtype != x.dtype or gate.dtype != x.dtype:
         raise TypeError("x, keys, values and gate must share one dtype")
     if x.shape[1] != D or values.shape[0] != E or values.shape[1] != F:
@@ -103,7 +103,7 @@ def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype
         _p(input_range), 0 if ir_dtype is None else raw.code_of(ir_dtype), 0 if input_range is None else input_range.shape[2], sel.data_ptr(), sel.dtype == torch.int64, gate.data_ptr(),
         cfg.inp_res, cfg.out_bound, cfg.out_res, cfg.noise_std,
         *_bounds(cfg.bounds_up, D), *_bounds(cfg.bounds_down, F), cfg.noise_seed & 0xFFFFFFFFFFFFFFFF, _p(cfg.noise_seed_dev),
-        cfg.noise_per_channel, _p(cfg.noise_up), _p(cfg.noise_down), _p(cfg.wmax_up), _p(cfg.wmax_down),
+        cfg.noise_per_channel, *map(_p, noise), _p(cfg.wmax_up), _p(cfg.wmax_down),
         cfg.seed_bump if cfg.noise_seed_dev is not None else 0, 0 if cfg.down_ready is None else cfg.down_ready.cuda_event,
         _p(y), p1.data_ptr(), z.data_ptr(), z.dtype == torch.uint8, _p(z_scale), perm.data_ptr(), in_index.data_ptr(),
         offsets.data_ptr(), _p(ir_up), _p(ir_dn),
@@ -129,6 +129,15 @@ def _range_table(input_range: torch.Tensor, E: int, cfg: FFNConfig) -> torch.Ten
     return _dense(input_range.detach().float())
 
 
+def _noise(t: Optional[torch.Tensor], bounds, M: int, N: int) -> Optional[torch.Tensor]:
+    """Injected output noise of a projection, fp32 [K-tiles, M, N]."""
+    if t is None:
+        return None
+    if t.numel() != _n_tiles(bounds) * M * N:
+        raise ValueError(f"injected noise must be [{_n_tiles(bounds)}, {M}, {N}], not {tuple(t.shape)}")
+    return ops._f32c(t)
+
+
 def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     """Sort, both projections and the gate reduction (``amoe_ffn_fwd``).  Returns (y, p1, z, perm, in_index, offsets,
     z_scale, ir_up, ir_dn): the result and what the backward pass reads again.  z is the down-projection's k-head result
@@ -143,6 +152,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     M = T * k
     if sel.numel() != M or gate.numel() != M:
         raise ValueError("sel_idx and gate must hold k values per token")
+    noise = _noise(cfg.noise_up, cfg.bounds_up, M, F), _noise(cfg.noise_down, cfg.bounds_down, M, V)
     y, p1 = x.new_empty((T, V)), x.new_empty((M, F))
     perm, in_index = (torch.empty(M, dtype=torch.int32, device=dev) for _ in range(2))
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
@@ -162,7 +172,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
             ir_up, ir_dn = ir_tables(input_range, E, cfg)
         return y, p1, z, perm, in_index, offsets.zero_(), z_scale, ir_up, ir_dn
     args = _pack(cfg, False, x, keys, values, input_range, None if input_range is None else input_range.dtype, sel, gate,
-                 y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn)
+                 y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn, noise=noise)
     ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8, device=dev)
     _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_fwd")
     return y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn

@@ -56,3 +56,27 @@ def test_input_range_that_is_no_table_of_both_projections(emu_ops, cfg):
         forward(pr, cfg, ir=torch.ones(2 * E + 1))
     with pytest.raises((RuntimeError, ValueError)):            # fewer columns than K-tiles
         forward(pr, dataclasses.replace(cfg, bounds_up=(0, 16, D)))
+
+
+def injected(pr, dtype=torch.float32, nt=1):
+    g = torch.Generator().manual_seed(3)
+    return dict(noise_std=0.04, noise_up=(0.1 * torch.randn(nt, T * K, F, generator=g)).to(dtype),
+                noise_down=(0.1 * torch.randn(1, T * K, D, generator=g)).to(dtype))
+
+
+def test_injected_noise_of_another_type_or_layout(emu_ops):
+    pr = problem()
+    noise = injected(pr, torch.bfloat16)
+    want = forward(pr, dataclasses.replace(ADC, **{n: t.float() if n != "noise_std" else t for n, t in noise.items()}))
+    assert same(forward(pr, dataclasses.replace(ADC, **noise)), want)
+    turned = noise["noise_up"].float().transpose(1, 2).contiguous().transpose(1, 2)
+    assert not turned.is_contiguous() and same(forward(pr, dataclasses.replace(ADC, **{**noise, "noise_up": turned})), want)
+
+
+@pytest.mark.parametrize("which", ["noise_up", "noise_down"])
+def test_injected_noise_of_another_size(emu_ops, which):
+    pr = problem()
+    noise = injected(pr)
+    noise[which] = noise[which][:, 1:].contiguous()
+    with pytest.raises(ValueError):
+        forward(pr, dataclasses.replace(ADC, **noise))
