@@ -84,13 +84,10 @@ def _bounds(bounds, K: int):
 
 
 def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype, sel, gate, y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn,
-          grads=(0, 0, 0, 0, 0, 0), noise=(None, None)) -> bytes:
+          grads=(0, 0, 0, 0, 0, 0), noise=(None, None), wmax=(None, None), per_channel=False) -> bytes:
     """The argument structure of ``amoe_ffn_fwd`` / ``amoe_ffn_bwd``.  All tensors rows-contiguous, x [T, D]."""
     E, D, F = keys.shape
     V = values.shape[2]
-    for t in (cfg.wmax_up, cfg.wmax_down):
-        if t is not None and (t.dtype != torch.float32 or not t.is_contiguous()):
-            raise TypeError("max |W| tables must be contiguous float32 tensors")
     if keys.dtype != x.dtype or values.dtype != x.dtype or gate.dtype != x.dtype:
         raise TypeError("x, keys, values and gate must share one dtype")
     if x.shape[1] != D or values.shape[0] != E or values.shape[1] != F:
@@ -103,7 +100,7 @@ def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype
         _p(input_range), 0 if ir_dtype is None else raw.code_of(ir_dtype), 0 if input_range is None else input_range.shape[2], sel.data_ptr(), sel.dtype == torch.int64, gate.data_ptr(),
         cfg.inp_res, cfg.out_bound, cfg.out_res, cfg.noise_std,
         *_bounds(cfg.bounds_up, D), *_bounds(cfg.bounds_down, F), cfg.noise_seed & 0xFFFFFFFFFFFFFFFF, _p(cfg.noise_seed_dev),
-        cfg.noise_per_channel, *map(_p, noise), _p(cfg.wmax_up), _p(cfg.wmax_down),
+        per_channel, *map(_p, noise), *map(_p, wmax),
         cfg.seed_bump if cfg.noise_seed_dev is not None else 0, 0 if cfg.down_ready is None else cfg.down_ready.cuda_event,
         _p(y), p1.data_ptr(), z.data_ptr(), z.dtype == torch.uint8, _p(z_scale), perm.data_ptr(), in_index.data_ptr(),
         offsets.data_ptr(), _p(ir_up), _p(ir_dn),
@@ -138,6 +135,26 @@ def _noise(t: Optional[torch.Tensor], bounds, M: int, N: int) -> Optional[torch.
     return ops._f32c(t)
 
 
+def _wmax_tables(cfg: FFNConfig, E: int, F: int, V: int):
+    """The caller's max |W| tables as the library takes them (fp32; None: it makes them) and whether they have a column per
+    output channel.  Each table says for itself whether it is [E] or [E, N]; the library has one flag for both."""
+    if cfg.wmax_up is None:
+        return (None, None), cfg.noise_per_channel
+    if cfg.out_bound <= 0 and (cfg.noise_std <= 0 or cfg.noise_up is not None):
+        return (None, None), False                   # nothing reads them
+    given = ((cfg.wmax_up, F), (cfg.wmax_down, V))
+    if any(t is None or t.numel() // E not in (1, N) for t, N in given):
+        raise ValueError("max |W| tables must be [E] or [E, output channels]")
+    wide = [t.numel() // E == N != 1 for t, N in given]
+    late = cfg.wmax_down
+    if cfg.down_ready is not None and (late.dtype != torch.float32 or not late.is_contiguous() or wide[0] != wide[1]):
+        torch.cuda.current_stream().wait_event(cfg.down_ready)
+    tables = [ops._f32c(t) for t, _ in given]
+    if any(wide):
+        tables = [t if w else t.reshape(-1)[:E, None].expand(E, N).contiguous() for t, w, (_, N) in zip(tables, wide, given)]
+    return tuple(tables), any(wide)
+
+
 def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     """Sort, both projections and the gate reduction (``amoe_ffn_fwd``).  Returns (y, p1, z, perm, in_index, offsets,
     z_scale, ir_up, ir_dn): the result and what the backward pass reads again.  z is the down-projection's k-head result
@@ -153,6 +170,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     if sel.numel() != M or gate.numel() != M:
         raise ValueError("sel_idx and gate must hold k values per token")
     noise = _noise(cfg.noise_up, cfg.bounds_up, M, F), _noise(cfg.noise_down, cfg.bounds_down, M, V)
+    wmax, per_channel = _wmax_tables(cfg, E, F, V)
     y, p1 = x.new_empty((T, V)), x.new_empty((M, F))
     perm, in_index = (torch.empty(M, dtype=torch.int32, device=dev) for _ in range(2))
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
@@ -172,7 +190,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
             ir_up, ir_dn = ir_tables(input_range, E, cfg)
         return y, p1, z, perm, in_index, offsets.zero_(), z_scale, ir_up, ir_dn
     args = _pack(cfg, False, x, keys, values, input_range, None if input_range is None else input_range.dtype, sel, gate,
-                 y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn, noise=noise)
+                 y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn, noise=noise, wmax=wmax,
+                 per_channel=per_channel)
     ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8, device=dev)
     _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_fwd")
     return y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn

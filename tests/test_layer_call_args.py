@@ -80,3 +80,42 @@ def test_injected_noise_of_another_size(emu_ops, which):
     noise[which] = noise[which][:, 1:].contiguous()
     with pytest.raises(ValueError):
         forward(pr, dataclasses.replace(ADC, **noise))
+
+
+@pytest.mark.parametrize("per_channel", [False, True])
+def test_max_w_tables_say_their_own_columns(emu_ops, per_channel):
+    """[E] (or [E, 1]) and [E, N] tables of the caller, whatever noise_per_channel says of tables made here, one of each
+    kind among them, in any floating type; the down-projection's alone is not used."""
+    pr = problem()
+    cfg = dataclasses.replace(ADC, noise_std=0.04, noise_seed=5)
+    up, dn = (torch.rand(E, n, generator=torch.Generator().manual_seed(n)) + 1.0 for n in (F, D))
+    one_up, one_dn = up[:, :1].clone(), dn[:, :1].clone()
+
+    def run(u, d, pc=per_channel):
+        return forward(pr, dataclasses.replace(cfg, wmax_up=u, wmax_down=d, noise_per_channel=pc))
+    wide = run(up, dn, True)
+    narrow = run(one_up, one_dn, False)
+    assert same(run(up, dn), wide) and same(run(one_up, one_dn), narrow)
+    assert same(run(one_up[:, 0], one_dn[:, 0]), narrow)
+    assert same(run(one_up, dn)[1:2], narrow[1:2]) and same(run(up, one_dn)[1:2], wide[1:2])
+    assert same(run(one_up.expand(E, F), dn), run(one_up, dn))
+    assert same(run(up.double(), dn.double()), wide)
+    assert same(run(None, one_dn), forward(pr, dataclasses.replace(cfg, noise_per_channel=per_channel)))
+    for bad in ((up[:, :-1], dn), (up, dn[:, 1:])):
+        with pytest.raises((ValueError, _abi.AmoeError)):
+            run(*bad)
+    assert same(forward(pr, dataclasses.replace(PLAIN, wmax_up=up[:, :5], wmax_down=dn)), forward(pr, PLAIN))   # no reader
+
+
+def test_late_max_w_table_is_converted_after_its_event(emu_ops, monkeypatch):
+    """A table of the down-projection that another stream still makes: what converts it waits for its event first."""
+    pr, order = problem(), []
+    event = type("Event", (), {"cuda_event": 0})()
+    stream = type("Stream", (), {"wait_event": lambda self, e: order.append(e)})()
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: stream)
+    cfg = dataclasses.replace(ADC, wmax_up=torch.ones(E, 1), wmax_down=torch.ones(E, 1), down_ready=event)
+    forward(pr, cfg)
+    assert order == []                                         # (the library's own launch waits)
+    forward(pr, dataclasses.replace(cfg, wmax_down=cfg.wmax_down.double()))
+    forward(pr, dataclasses.replace(cfg, wmax_up=torch.ones(E, F)))
+    assert order == [event, event]
