@@ -169,6 +169,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     M = T * k
     if sel.numel() != M or gate.numel() != M:
         raise ValueError("sel_idx and gate must hold k values per token")
+    if cfg.noise_seed_dev is not None and (cfg.noise_seed_dev.dtype != torch.int64 or cfg.noise_seed_dev.numel() != 1):
+        raise ValueError("noise_seed_dev must be one int64 word")
     noise = _noise(cfg.noise_up, cfg.bounds_up, M, F), _noise(cfg.noise_down, cfg.bounds_down, M, V)
     wmax, per_channel = _wmax_tables(cfg, E, F, V)
     y, p1 = x.new_empty((T, V)), x.new_empty((M, F))

@@ -119,3 +119,12 @@ def test_late_max_w_table_is_converted_after_its_event(emu_ops, monkeypatch):
     forward(pr, dataclasses.replace(cfg, wmax_down=cfg.wmax_down.double()))
     forward(pr, dataclasses.replace(cfg, wmax_up=torch.ones(E, F)))
     assert order == [event, event]
+
+
+@pytest.mark.parametrize("word", [torch.zeros(1, dtype=torch.int32), torch.zeros(2, dtype=torch.int64), torch.zeros(1)])
+def test_seed_word_that_is_none(emu_ops, word):
+    pr = problem()
+    with pytest.raises(ValueError):
+        forward(pr, dataclasses.replace(ADC, noise_std=0.04, noise_seed_dev=word))
+    with pytest.raises(ValueError):
+        forward(pr, dataclasses.replace(PLAIN, noise_seed_dev=word))
