@@ -108,6 +108,15 @@ def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype
         0 if cfg.stage_events is None else cfg.stage_events(backward))
 
 
+def _rows_of(t: torch.Tensor, rows: int, cols: int, name: str) -> torch.Tensor:
+    """t as a contiguous [rows, cols]."""
+    if t.shape == (rows, cols) and t.is_contiguous():
+        return t
+    if t.shape[-1] != cols or t.numel() != rows * cols:
+        raise ValueError(f"{name} must be [{rows}, {cols}], not {tuple(t.shape)}")
+    return t.detach().reshape(rows, cols).contiguous()
+
+
 def _int_ids(sel_idx: torch.Tensor) -> torch.Tensor:
     sel = sel_idx.detach()
     if sel.dtype not in (torch.int32, torch.int64):
@@ -211,9 +220,27 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
     """Returns (grad_x, grad_keys, grad_values, grad_ir [2, E, n_tiles] of type ir_dtype or None, grad_gate)
     (``amoe_ffn_bwd``)."""
     lib = ops.get_lib()
-    x, keys, values, dy = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(dy)
+    x, keys, values = ops._rows2d(x.detach()), _dense(keys), _dense(values)
     gate_c, sel = _dense(gate), _int_ids(sel_idx)
-    E = keys.shape[0]
+    (E, D, F), V = keys.shape, values.shape[2]
+    T, k = x.shape[0], gate.shape[-1]
+    M = T * k
+    if sel.numel() != M or gate_c.numel() != M:
+        raise ValueError("sel_idx and gate must hold k values per token")
+    # what the forward call left may come back through hooks in another layout, and from a caller as anything
+    dy, p1, z = _rows_of(dy, T, V, "dy"), _rows_of(p1, M, F, "p1"), _rows_of(z, M, V, "z")
+    if dy.dtype != x.dtype or p1.dtype != x.dtype or z.dtype not in (x.dtype, torch.uint8):
+        raise TypeError("dy, p1 and x must share one dtype, z that or uint8 codes")
+    if z.dtype == torch.uint8 and (z_scale.dtype != torch.float32 or tuple(z_scale.shape) != (E, 2) or not z_scale.is_contiguous()):
+        raise ValueError("ADC codes come with their scale, fp32 [E, 2]")
+    for t, n, name in ((perm, M, "perm"), (in_index, M, "in_index"), (offsets, E + 1, "offsets")):
+        if raw._i32(t, name).numel() != n:
+            raise ValueError(f"{name} must hold {n} values")
+    if (ir_up is None) != (ir_dn is None):
+        raise ValueError("input ranges of both projections or of none")
+    ir_up, ir_dn = ops._f32c(ir_up), ops._f32c(ir_dn)
+    if ir_up is not None and (ir_up.shape != (E, _n_tiles(cfg.bounds_up)) or ir_dn.shape != (E, _n_tiles(cfg.bounds_down))):
+        raise ValueError("input ranges must be [E, K-tiles of the projection]")
     grad_x = x.new_empty(x.shape)
     grad_keys, grad_values, grad_gate = torch.empty_like(keys), torch.empty_like(values), torch.empty_like(gate_c)
     grad_ir = None
@@ -224,8 +251,6 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
             if g is not None:
                 g.zero_()
         return grad_x, grad_keys, grad_values, grad_ir, grad_gate
-    if dy.dtype != x.dtype:
-        raise TypeError("dy and x must share one dtype")
     args = _pack(cfg, True, x, keys, values, None, None if grad_ir is None else ir_dtype, sel, gate_c, None, p1, z, z_scale, perm, in_index, offsets,
                  ir_up, ir_dn, (dy.data_ptr(), grad_x.data_ptr(), grad_keys.data_ptr(), grad_values.data_ptr(),
                                 grad_gate.data_ptr(), _p(grad_ir)))

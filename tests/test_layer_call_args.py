@@ -128,3 +128,36 @@ def test_seed_word_that_is_none(emu_ops, word):
         forward(pr, dataclasses.replace(ADC, noise_std=0.04, noise_seed_dev=word))
     with pytest.raises(ValueError):
         forward(pr, dataclasses.replace(PLAIN, noise_seed_dev=word))
+
+
+def test_backward_of_another_gradient(emu_ops):
+    pr = problem()
+    saved = forward(pr, ADC)
+    want = backward(pr, ADC, saved)
+    assert same(backward(pr, ADC, saved, dy=pr["dy"].reshape(2, T // 2, D)), want)
+    assert same(backward(pr, ADC, saved, dy=pr["dy"].t().contiguous().t()), want)
+    for bad in (pr["dy"][1:], pr["dy"][:, 1:], torch.cat((pr["dy"], pr["dy"]))):
+        with pytest.raises((ValueError, RuntimeError)):
+            backward(pr, ADC, saved, dy=bad)
+    with pytest.raises(TypeError):
+        backward(pr, ADC, saved, dy=pr["dy"].double())
+
+
+def test_backward_of_other_saved_tensors(emu_ops):
+    """Hooks on saved tensors, and callers of the operators, may hand over copies in another layout, or anything."""
+    pr = problem()
+    saved = forward(pr, ADC)
+    want = backward(pr, ADC, saved)
+    y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn = saved
+
+    def turned(t):
+        return t.t().contiguous().t()
+    assert same(backward(pr, ADC, saved, p1=turned(p1), z=turned(z), idx=turned(pr["idx"]), gate=turned(pr["gate"]),
+                         ir_up=ir_up.double(), ir_dn=ir_dn.double()), want)
+    wrong = [dict(p1=p1[1:]), dict(z=z[1:]), dict(z=z[:, 1:]), dict(perm=perm[1:]), dict(in_index=in_index[1:]),
+             dict(offsets=offsets[1:]), dict(perm=perm.long()), dict(in_index=in_index.float()), dict(offsets=offsets.long()),
+             dict(ir_up=ir_up[1:]), dict(ir_dn=torch.ones(E, 3)), dict(idx=pr["idx"][1:]), dict(gate=pr["gate"][1:]), dict(p1=p1.double()),
+             dict(z=z.double()), dict(z=z.to(torch.uint8)), dict(perm=torch.stack((perm, perm), 1)[:, 0])]
+    for swap in wrong:
+        with pytest.raises((ValueError, TypeError)):
+            backward(pr, ADC, saved, **swap)
