@@ -168,7 +168,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     """Sort, both projections and the gate reduction (``amoe_ffn_fwd``).  Returns (y, p1, z, perm, in_index, offsets,
     z_scale, ir_up, ir_dn): the result and what the backward pass reads again.  z is the down-projection's k-head result
     [T*k, D], either as values (z_scale empty) or as uint8 ADC codes with z_scale [E, 2] (``ops.dequant_codes``)."""
-    ops._need_gpu(x, keys, values, input_range, gate, sel_idx)
+    ops._need_gpu(x, keys, values, input_range, gate, sel_idx, cfg.noise_up, cfg.noise_down, cfg.wmax_up, cfg.wmax_down,
+                  cfg.noise_seed_dev)
     lib = ops.get_lib()
     x, keys, values, gate = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(gate)
     sel = _int_ids(sel_idx)
@@ -219,6 +220,7 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
                  cfg: FFNConfig, want_ir_grad: bool, ir_dtype: torch.dtype = torch.float32):
     """Returns (grad_x, grad_keys, grad_values, grad_ir [2, E, n_tiles] of type ir_dtype or None, grad_gate)
     (``amoe_ffn_bwd``)."""
+    ops._need_gpu(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn)
     lib = ops.get_lib()
     x, keys, values = ops._rows2d(x.detach()), _dense(keys), _dense(values)
     gate_c, sel = _dense(gate), _int_ids(sel_idx)

@@ -161,3 +161,21 @@ def test_backward_of_other_saved_tensors(emu_ops):
     for swap in wrong:
         with pytest.raises((ValueError, TypeError)):
             backward(pr, ADC, saved, **swap)
+
+
+def test_every_tensor_must_lie_on_the_gpu(emu_ops, monkeypatch):
+    """A pointer to host memory in a kernel is a fault on the GPU: every tensor of a call passes the device check."""
+    pr = problem()
+    noise = injected(pr)
+    cfg = dataclasses.replace(ADC, **noise, wmax_up=torch.ones(E, 1), wmax_down=torch.ones(E, 1), noise_seed_dev=torch.zeros(1, dtype=torch.int64))
+    saved = forward(pr, cfg)
+    seen = []
+    monkeypatch.setattr(emu_ops, "_need_gpu", lambda *t: seen.extend(id(v) for v in t))
+    forward(pr, cfg)
+    for t in (*(pr[n] for n in ("x", "keys", "values", "ir", "gate", "idx")), cfg.noise_up, cfg.noise_down, cfg.wmax_up, cfg.wmax_down,
+              cfg.noise_seed_dev):
+        assert id(t) in seen
+    del seen[:]
+    backward(pr, cfg, saved)
+    for t in (*(pr[n] for n in ("dy", "x", "keys", "values", "gate", "idx")), *(t for t in saved[1:])):
+        assert id(t) in seen
