@@ -117,6 +117,12 @@ def _rows_of(t: torch.Tensor, rows: int, cols: int, name: str) -> torch.Tensor:
     return t.detach().reshape(rows, cols).contiguous()
 
 
+def _check_heads(sel: torch.Tensor, gate: torch.Tensor, M: int, k: int) -> None:
+    """The library counts the heads once for both."""
+    if sel.numel() != M or gate.numel() != M or sel.shape[-1] != k or gate.shape[-1] != k:
+        raise ValueError(f"sel_idx and gate must hold k values per token: {tuple(sel.shape)} and {tuple(gate.shape)}")
+
+
 def _int_ids(sel_idx: torch.Tensor) -> torch.Tensor:
     sel = sel_idx.detach()
     if sel.dtype not in (torch.int32, torch.int64):
@@ -170,6 +176,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     [T*k, D], either as values (z_scale empty) or as uint8 ADC codes with z_scale [E, 2] (``ops.dequant_codes``)."""
     ops._need_gpu(x, keys, values, input_range, gate, sel_idx, cfg.noise_up, cfg.noise_down, cfg.wmax_up, cfg.wmax_down,
                   cfg.noise_seed_dev)
+    if x.dim() != 2:
+        raise ValueError("x must be [tokens, features]")
     lib = ops.get_lib()
     x, keys, values, gate = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(gate)
     sel = _int_ids(sel_idx)
@@ -177,8 +185,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     (E, D, F), V = keys.shape, values.shape[2]
     T, k = x.shape[0], sel.shape[-1]
     M = T * k
-    if sel.numel() != M or gate.numel() != M:
-        raise ValueError("sel_idx and gate must hold k values per token")
+    _check_heads(sel, gate, M, k)
     if cfg.noise_seed_dev is not None and (cfg.noise_seed_dev.dtype != torch.int64 or cfg.noise_seed_dev.numel() != 1):
         raise ValueError("noise_seed_dev must be one int64 word")
     noise = _noise(cfg.noise_up, cfg.bounds_up, M, F), _noise(cfg.noise_down, cfg.bounds_down, M, V)
@@ -227,8 +234,7 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
     (E, D, F), V = keys.shape, values.shape[2]
     T, k = x.shape[0], gate.shape[-1]
     M = T * k
-    if sel.numel() != M or gate_c.numel() != M:
-        raise ValueError("sel_idx and gate must hold k values per token")
+    _check_heads(sel, gate, M, k)
     # what the forward call left may come back through hooks in another layout, and from a caller as anything
     dy, p1, z = _rows_of(dy, T, V, "dy"), _rows_of(p1, M, F, "p1"), _rows_of(z, M, V, "z")
     if dy.dtype != x.dtype or p1.dtype != x.dtype or z.dtype not in (x.dtype, torch.uint8):

@@ -179,3 +179,19 @@ def test_every_tensor_must_lie_on_the_gpu(emu_ops, monkeypatch):
     backward(pr, cfg, saved)
     for t in (*(pr[n] for n in ("dy", "x", "keys", "values", "gate", "idx")), *(t for t in saved[1:])):
         assert id(t) in seen
+
+
+def test_heads_of_gate_and_ids_agree(emu_ops):
+    pr = problem()
+    want = forward(pr, PLAIN)
+    lead = dict(gate=pr["gate"].reshape(2, T // 2, K), idx=pr["idx"].reshape(2, T // 2, K))
+    assert same(forward(pr, PLAIN, **lead), want)
+    g3 = backward(pr, PLAIN, want, **lead)
+    assert g3[4].shape == lead["gate"].shape and torch.equal(g3[4].reshape(T, K), backward(pr, PLAIN, want)[4])
+    for bad in (dict(gate=pr["gate"].reshape(-1)), dict(gate=pr["gate"].reshape(1, -1)), dict(gate=pr["gate"].reshape(-1, 1)),
+                dict(idx=pr["idx"].reshape(-1)), dict(x=pr["x"].reshape(2, T // 2, D))):
+        with pytest.raises(ValueError):
+            forward(pr, PLAIN, **bad)
+    for bad in (dict(gate=pr["gate"].reshape(-1)), dict(gate=pr["gate"].reshape(-1, 1)), dict(idx=pr["idx"].reshape(-1))):
+        with pytest.raises(ValueError):
+            backward(pr, PLAIN, want, **bad)
