@@ -179,7 +179,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     if x.dim() != 2:
         raise ValueError("x must be [tokens, features]")
     lib = ops.get_lib()
-    x, keys, values, gate = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(gate)
+    x, keys, values, own_gate = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(gate)
+    gate = own_gate if own_gate.dtype == x.dtype else own_gate.to(x.dtype)
     sel = _int_ids(sel_idx)
     dev, dt = x.device, x.dtype
     (E, D, F), V = keys.shape, values.shape[2]
@@ -200,6 +201,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
                         for b in (cfg.bounds_up, cfg.bounds_down))
     chain = input_range is not None and cfg.inp_res > 0 and _n_tiles(cfg.bounds_down) == 1
     codes = chain and z_as_codes(p1, values, cfg)
+    if codes and gate is not own_gate:               # (codes are weighted in the gate's type)
+        raw.dtype_code(own_gate)
     z = torch.empty((M, V), dtype=torch.uint8 if codes else dt, device=dev)
     z_scale = torch.empty((E, 2) if codes else 0, dtype=torch.float32, device=dev)
     if M == 0:                                       # no tokens: nothing to launch but the step counter
@@ -213,6 +216,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
                  per_channel=per_channel)
     ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8, device=dev)
     _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_fwd")
+    if codes and gate is not own_gate:
+        y = ops.gate_reduce_codes(z, z_scale, sel, own_gate)
     return y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn
 
 
@@ -230,7 +235,7 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
     ops._need_gpu(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn)
     lib = ops.get_lib()
     x, keys, values = ops._rows2d(x.detach()), _dense(keys), _dense(values)
-    gate_c, sel = _dense(gate), _int_ids(sel_idx)
+    gate_c, sel = _dense(gate).to(x.dtype), _int_ids(sel_idx)
     (E, D, F), V = keys.shape, values.shape[2]
     T, k = x.shape[0], gate.shape[-1]
     M = T * k

@@ -195,3 +195,21 @@ def test_heads_of_gate_and_ids_agree(emu_ops):
     for bad in (dict(gate=pr["gate"].reshape(-1)), dict(gate=pr["gate"].reshape(-1, 1)), dict(idx=pr["idx"].reshape(-1))):
         with pytest.raises(ValueError):
             backward(pr, PLAIN, want, **bad)
+
+
+def test_gate_of_another_type(emu_ops):
+    pr = problem(torch.bfloat16)
+    want = forward(pr, ADC)
+    assert want[2].dtype == torch.bfloat16
+    for dt in (torch.float32, torch.float64):
+        assert same(forward(pr, ADC, gate=pr["gate"].to(dt)), want)
+    assert same(backward(pr, ADC, want, gate=pr["gate"].float()), backward(pr, ADC, want))
+    # ADC codes are weighted in the gate's own type
+    big = dict(T=T, D=256, E=E, F=256, k=K)
+    pr = problem(torch.bfloat16, **big)
+    want = forward(pr, ADC)
+    got = forward(pr, ADC, gate=pr["gate"].float())
+    assert want[2].dtype == torch.uint8 and got[0].dtype == torch.float32 and same(got[1:], want[1:])
+    assert torch.equal(got[0].bfloat16(), want[0])
+    with pytest.raises(TypeError):
+        forward(pr, ADC, gate=pr["gate"].double())
