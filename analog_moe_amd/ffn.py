@@ -303,6 +303,6 @@ def moe_ffn(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig) -> torc
     (their side streams and ctypes calls are nothing a tracer can follow)."""
     if torch.compiler.is_compiling():
         return torch.ops.amoe.ffn_fwd(x, keys, values, input_range, gate, sel_idx, *cfg_astuple(cfg))[0]
-    if not torch.is_grad_enabled():
+    if not torch.is_grad_enabled() and ops.unwatched():
         return ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg)[0]
     return AnalogMoEFFN.apply(x, keys, values, input_range, gate, sel_idx, cfg)

@@ -302,10 +302,8 @@ class AnalogLinear(nn.Module):
 
 
 def _plain(t: Tensor) -> bool:
-    """A tensor whose memory a kernel may read behind torch's back: no subclass, no function transform around it, no
-    dispatch mode that wants to see the operators."""
-    return type(t) in (Tensor, nn.Parameter) and torch._C._functorch.peek_interpreter_stack() is None \
-        and torch._C._len_torch_dispatch_stack() == 0 and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+    """A tensor whose memory a kernel may read behind torch's back: no subclass, nobody who wants to see the operators."""
+    return type(t) in (Tensor, nn.Parameter) and ops.unwatched() and not torch._C._functorch.is_functorch_wrapped_tensor(t)
 
 
 def _observed(m: nn.Module) -> bool:

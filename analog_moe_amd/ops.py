@@ -12,6 +12,7 @@ import os
 from typing import Optional, Sequence, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _abi, raw
 
@@ -53,6 +54,13 @@ def side_stream(device: torch.device) -> "torch.cuda.Stream":
 def _side(t: torch.Tensor):
     """Handle of the device's extra stream (None where there are no streams)."""
     return side_stream(t.device).cuda_stream if t.is_cuda else None
+
+
+def unwatched() -> bool:
+    """Whether a call may go to the kernels behind torch's back: no forward-mode level, function transform, dispatch mode
+    or trace that wants to see the operators."""
+    return (forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None)
 
 
 def _need_gpu(*tensors) -> None:
