@@ -10,7 +10,9 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <memory>
+#include <mutex>
 #include <sched.h>
 #include <thread>
 #include <vector>
@@ -33,13 +35,54 @@ typedef int hipError_t;
 typedef void* hipStream_t;
 enum { hipSuccess = 0 };
 inline hipError_t hipGetLastError() { return hipSuccess; }
-// launches run at once and in order, so streams and events order nothing here
+// Launches run at once and in order, so streams and events order nothing here; what the calls would order is written down:
+// per stream the launches given to it, per event the stream and its count when it was recorded, per pair of streams how far
+// the first waits for the second.
 typedef void* hipEvent_t;
 enum { hipEventDisableTiming = 2 };
-inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = nullptr; return hipSuccess; }
-inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-inline hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-inline hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+struct EmuOrder {
+  std::mutex lock;
+  uintptr_t handles = 0;
+  std::map<hipStream_t, long long> given;
+  std::map<hipEvent_t, std::pair<hipStream_t, long long>> events;
+  std::map<std::pair<hipStream_t, hipStream_t>, long long> waited;
+};
+inline EmuOrder emu_order;
+inline void emu_note_launch(hipStream_t s) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  emu_order.given[s]++;
+}
+inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  *e = reinterpret_cast<hipEvent_t>(++emu_order.handles);
+  return hipSuccess;
+}
+inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  emu_order.events[e] = {s, emu_order.given[s]};
+  return hipSuccess;
+}
+inline hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  auto it = emu_order.events.find(e);
+  if (it != emu_order.events.end()) emu_order.waited[{s, it->second.first}] = it->second.second;
+  return hipSuccess;
+}
+inline hipError_t hipEventDestroy(hipEvent_t e) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  emu_order.events.erase(e);
+  return hipSuccess;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+// launches given to `other`, and how many of them stream s does not wait for
+extern "C" inline __attribute__((used)) long long amoe_emu_launches(hipStream_t other) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  return emu_order.given[other];
+}
+extern "C" inline __attribute__((used)) long long amoe_emu_not_waited_for(hipStream_t s, hipStream_t other) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  return emu_order.given[other] - emu_order.waited[{s, other}];
+}
 inline const char* hipGetErrorString(hipError_t) { return "emu"; }
 enum hipDeviceAttribute_t { hipDeviceAttributeMultiprocessorCount = 0 };
 inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
@@ -122,4 +165,5 @@ inline void emu_launch(K kernel, dim3 grid, dim3 block, A... args) {
     for (auto& x : th) x.join();
   }
 }
-#define hipLaunchKernelGGL(kernel, grid, block, shmem, stream, ...) emu_launch(kernel, grid, block, __VA_ARGS__)
+#define hipLaunchKernelGGL(kernel, grid, block, shmem, stream, ...) \
+  (emu_note_launch(stream), emu_launch(kernel, grid, block, __VA_ARGS__))

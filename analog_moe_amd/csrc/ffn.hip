@@ -106,6 +106,31 @@ int order_after(hipStream_t to, hipStream_t from) {
   return (int)rc;
 }
 
+// Launches on the second stream beside those on the first.  However the call ends, the first stream continues after both:
+// what a launch uses belongs to the caller again once the call has returned.
+struct Fork {
+  hipStream_t main, side;
+  bool open = false;
+  Fork(hipStream_t main_, void* side_stream, bool wanted)
+      : main(main_), side(wanted && side_stream ? static_cast<hipStream_t>(side_stream) : main_) {}
+  int begin() {
+    if (side == main) return AMOE_OK;
+    const int rc = order_after(side, main);
+    open = rc == AMOE_OK;
+    return rc;
+  }
+  int join() {
+    if (!open) return AMOE_OK;
+    open = false;
+    const int rc = order_after(main, side);
+    if (rc) (void)hipStreamSynchronize(side);        // no event to wait for: the host waits
+    return rc;
+  }
+  ~Fork() { (void)join(); }
+  Fork(const Fork&) = delete;
+  Fork& operator=(const Fork&) = delete;
+};
+
 const char* const kFwdStages[] = {"prepare_sel", "tables", "fwd_up", "fwd_down", "gate_reduce"};
 const char* const kBwdStages[] = {"xgrad_down", "xgrad_up", "gate_grad", "head_sum", "wgrad_down", "wgrad_up", "ir_sums"};
 
@@ -187,16 +212,15 @@ int amoe_ffn_fwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes
   if (workspace_bytes < amoe_ffn_fwd_workspace(a)) return AMOE_EWORKSPACE;
   Arena m{static_cast<char*>(workspace)};
   const FwdScratch s = fwd_scratch(a, m);
-  hipStream_t st = static_cast<hipStream_t>(stream), side = static_cast<hipStream_t>(side_stream);
+  hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t M = rows_of(a);
   const bool ranges = has_ranges(a), gen = generates_noise(a), chain = chained(a);
   // max |W| per expert and the fp32 input-range tables only read parameters: they can run next to the expert sort
-  const bool fork = side && s.wmax_up && overlap_tables(a);
-  if (fork)
-    if (int rc = order_after(side, st)) return rc;
+  Fork fork(st, side_stream, s.wmax_up && overlap_tables(a));
+  if (int rc = fork.begin()) return rc;
   if (s.wmax_up || ranges) {
-    Stage t(a, 1, fork ? side : st);
-    if (int rc = tables(a, s, fork ? side : st)) return rc;
+    Stage t(a, 1, fork.side);
+    if (int rc = tables(a, s, fork.side)) return rc;
   }
   {
     Stage t(a, 0, st);
@@ -204,8 +228,7 @@ int amoe_ffn_fwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes
                                   a->in_index, a->offsets, nullptr, s.sort, amoe_prepare_sel_workspace(M, (int32_t)a->E), st))
       return rc;
   }
-  if (fork)
-    if (int rc = order_after(st, side)) return rc;
+  if (int rc = fork.join()) return rc;
   const float* wmax_up = a->wmax_up ? a->wmax_up : s.wmax_up;
   const float* wmax_dn = a->wmax_dn ? a->wmax_dn : s.wmax_dn;
 
@@ -321,10 +344,9 @@ int amoe_ffn_bwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes
   // the two weight gradients.  With evenly loaded experts the launches take as long side by side as one after the other
   // (together they are bound by memory traffic); with uneven loads the streaming kernels fill the CUs that the weight
   // gradients' last tiles leave idle (2 - 3 % of the step).
-  const bool fork = side_stream && overlap_companions(a);
-  hipStream_t side = fork ? static_cast<hipStream_t>(side_stream) : st;
-  if (fork)
-    if (int rc = order_after(side, st)) return rc;
+  Fork fork(st, side_stream, overlap_companions(a));
+  hipStream_t side = fork.side;
+  if (int rc = fork.begin()) return rc;
   {
     Stage t(a, 2, side);
     const int rc = a->z_is_codes
@@ -380,8 +402,7 @@ int amoe_ffn_bwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes
     Stage t(a, 5, st);
     if (int rc = amoe_cvmm_bwd_w(&w, st)) return rc;
   }
-  if (fork)
-    if (int rc = order_after(st, side)) return rc;
+  if (int rc = fork.join()) return rc;
   if (ranges && gir) {
     Stage t(a, 6, st);
     return amoe_segment_sum(s.irg_up, a->offsets, E, (int32_t)a->n_up, (int32_t)a->ir_dtype, gir, nt, nt - (int32_t)a->n_up, st);

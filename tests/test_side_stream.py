@@ -1,0 +1,70 @@
+"""The layer calls' second stream is joined however a call ends: what its launches read and write belongs to the caller again
+once the call has returned, with an error as without one."""
+import ctypes
+
+import pytest
+import torch
+
+from analog_moe_amd import ffn
+from tests.test_emu_kernels import emu_ops  # noqa: F401
+
+MAIN, SIDE = 11, 12                      # stream handles: the host build only writes down what is given to them
+
+
+def arguments(T, D, E, F, k, cfg, grads=(0, 0, 0, 0, 0, 0)):
+    g = torch.Generator().manual_seed(1)
+    M = T * k
+    t = dict(x=torch.randn(T, D, generator=g), keys=torch.randn(E, D, F, generator=g), values=torch.randn(E, F, D, generator=g),
+             gate=torch.rand(T, k, generator=g), sel=torch.randint(0, E, (M + 1,), generator=g, dtype=torch.int64), y=torch.zeros(T, D),
+             p1=torch.rand(M, F, generator=g), z=torch.rand(M, D, generator=g), perm=torch.arange(M, dtype=torch.int32),
+             in_index=(torch.arange(M) // k).int(), offsets=(torch.arange(E + 1) * M // E).int())
+    args = ffn._pack(cfg, any(grads), t["x"], t["keys"], t["values"], None, None, t["sel"], t["gate"], t["y"], t["p1"], t["z"], None,
+                     t["perm"], t["in_index"], t["offsets"], None, None, grads)
+    return t, args
+
+
+def streams(lib):
+    count = {}
+    for name, n in (("amoe_emu_launches", 1), ("amoe_emu_not_waited_for", 2)):
+        fn = getattr(lib, name)
+        fn.restype, fn.argtypes = ctypes.c_longlong, [ctypes.c_void_p] * n
+        count[name] = fn
+    return count["amoe_emu_launches"], count["amoe_emu_not_waited_for"]
+
+
+def shifted(args, ptr, by):
+    """The packed arguments with a pointer moved."""
+    at = args.index(ptr.to_bytes(8, "little"))
+    return args[:at] + (ptr + by).to_bytes(8, "little") + args[at + 8:]
+
+
+@pytest.mark.parametrize("fails", [False, True])
+def test_forward(emu_ops, fails):
+    """max |W| of 24 MB of weights beside the sort, which refuses ids that are not 8-byte aligned"""
+    lib = emu_ops.get_lib()
+    launches, not_waited = streams(lib)
+    t, args = arguments(1, 6144, 1, 512, 1, ffn.FFNConfig(inp_res=-1.0, out_bound=12.0, out_res=254.0))
+    if fails:
+        args = shifted(args, t["sel"].data_ptr(), 4)
+    ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8)
+    before = launches(SIDE)
+    rc = lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), MAIN, SIDE)
+    assert (rc != 0) == fails and launches(SIDE) > before and not_waited(MAIN, SIDE) == 0
+
+
+@pytest.mark.parametrize("fails", [False, True])
+def test_backward(emu_ops, fails):
+    """the streaming companions beside the weight gradients, which refuse an output that is not aligned to its elements"""
+    lib = emu_ops.get_lib()
+    launches, not_waited = streams(lib)
+    T, D, E, F, k = 64, 24704, 1, 4, 2
+    out = [torch.zeros(n) for n in (T * D, E * D * F, E * F * D + 1, T * k)]
+    dy = torch.randn(T, D)
+    ptrs = [t.data_ptr() for t in (dy, *out)] + [0]
+    t, args = arguments(T, D, E, F, k, ffn.FFNConfig(inp_res=-1.0), ptrs)
+    if fails:
+        args = shifted(args, out[2].data_ptr(), 2)
+    ws = torch.empty(lib.amoe_ffn_bwd_workspace(args), dtype=torch.uint8)
+    before = launches(SIDE)
+    rc = lib.amoe_ffn_bwd(args, ws.data_ptr(), ws.numel(), MAIN, SIDE)
+    assert (rc != 0) == fails and launches(SIDE) == before + 2 and not_waited(MAIN, SIDE) == 0
