@@ -52,19 +52,17 @@ def test_forward(emu_ops, fails):
     assert (rc != 0) == fails and launches(SIDE) > before and not_waited(MAIN, SIDE) == 0
 
 
-@pytest.mark.parametrize("fails", [False, True])
-def test_backward(emu_ops, fails):
+def test_backward(emu_ops):
     """the streaming companions beside the weight gradients, which refuse an output that is not aligned to its elements"""
     lib = emu_ops.get_lib()
     launches, not_waited = streams(lib)
-    T, D, E, F, k = 64, 24704, 1, 4, 2
+    T, D, E, F, k = 260, 6144, 1, 4, 2
     out = [torch.zeros(n) for n in (T * D, E * D * F, E * F * D + 1, T * k)]
     dy = torch.randn(T, D)
     ptrs = [t.data_ptr() for t in (dy, *out)] + [0]
     t, args = arguments(T, D, E, F, k, ffn.FFNConfig(inp_res=-1.0), ptrs)
-    if fails:
-        args = shifted(args, out[2].data_ptr(), 2)
+    args = shifted(args, out[2].data_ptr(), 2)
     ws = torch.empty(lib.amoe_ffn_bwd_workspace(args), dtype=torch.uint8)
     before = launches(SIDE)
     rc = lib.amoe_ffn_bwd(args, ws.data_ptr(), ws.numel(), MAIN, SIDE)
-    assert (rc != 0) == fails and launches(SIDE) == before + 2 and not_waited(MAIN, SIDE) == 0
+    assert rc != 0 and launches(SIDE) == before + 2 and not_waited(MAIN, SIDE) == 0
