@@ -136,7 +136,8 @@ FFN_ARGS = struct.Struct("<"
 
 @functools.lru_cache(maxsize=256)
 def bounds_array(bounds):
-    """A tuple of K-tile bounds as a C array (kept: callers pass its address)."""
+    """A tuple of K-tile bounds as a C array.  A caller that passes its address holds the array itself until its call
+    returns: the cache may forget it."""
     return (C.c_int32 * len(bounds))(*bounds)
 
 

@@ -77,15 +77,17 @@ def _dense(t: torch.Tensor) -> torch.Tensor:
 
 
 def _bounds(bounds, K: int):
-    b = (0, K) if bounds is None else tuple(bounds)
+    """The bounds of a projection's K-tiles as a C array, to be held until the call that reads them returns."""
+    b = (0, K) if bounds is None else tuple(map(int, bounds))
     if not 2 <= len(b) <= _abi.AMOE_MAX_TILES + 1:
         raise ValueError(f"number of K-tiles must be in [1, {_abi.AMOE_MAX_TILES}]")
-    return len(b) - 1, ctypes.addressof(_abi.bounds_array(b))
+    return _abi.bounds_array(b)
 
 
 def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype, sel, gate, y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn,
-          grads=(0, 0, 0, 0, 0, 0), noise=(None, None), wmax=(None, None), per_channel=False) -> bytes:
-    """The argument structure of ``amoe_ffn_fwd`` / ``amoe_ffn_bwd``.  All tensors rows-contiguous, x [T, D]."""
+          grads=(0, 0, 0, 0, 0, 0), noise=(None, None), wmax=(None, None), per_channel=False):
+    """The argument structure of ``amoe_ffn_fwd`` / ``amoe_ffn_bwd``, and what it points at beside the tensors (to be held
+    until the call returns).  All tensors rows-contiguous, x [T, D]."""
     E, D, F = keys.shape
     V = values.shape[2]
     if keys.dtype != x.dtype or values.dtype != x.dtype or gate.dtype != x.dtype:
@@ -94,18 +96,20 @@ def _pack(cfg: FFNConfig, backward: bool, x, keys, values, input_range, ir_dtype
         raise ValueError("x / keys / values shapes do not match")
     if x.dtype != torch.float32 and cfg.inp_res > 0:
         raw.check_codes_fit(x.dtype, cfg.inp_res)
-    return _abi.FFN_ARGS.pack(
+    up, down = _bounds(cfg.bounds_up, D), _bounds(cfg.bounds_down, F)
+    packed = _abi.FFN_ARGS.pack(
         raw.dtype_code(x), x.shape[0], D, E, F, V, gate.shape[-1],
         x.data_ptr(), x.stride(0), keys.data_ptr(), *keys.stride(), values.data_ptr(), *values.stride(),
         _p(input_range), 0 if ir_dtype is None else raw.code_of(ir_dtype), 0 if input_range is None else input_range.shape[2], sel.data_ptr(), sel.dtype == torch.int64, gate.data_ptr(),
         cfg.inp_res, cfg.out_bound, cfg.out_res, cfg.noise_std,
-        *_bounds(cfg.bounds_up, D), *_bounds(cfg.bounds_down, F), cfg.noise_seed & 0xFFFFFFFFFFFFFFFF, _p(cfg.noise_seed_dev),
+        len(up) - 1, ctypes.addressof(up), len(down) - 1, ctypes.addressof(down), cfg.noise_seed & 0xFFFFFFFFFFFFFFFF, _p(cfg.noise_seed_dev),
         per_channel, *map(_p, noise), *map(_p, wmax),
         cfg.seed_bump if cfg.noise_seed_dev is not None else 0, 0 if cfg.down_ready is None else cfg.down_ready.cuda_event,
         _p(y), p1.data_ptr(), z.data_ptr(), z.dtype == torch.uint8, _p(z_scale), perm.data_ptr(), in_index.data_ptr(),
         offsets.data_ptr(), _p(ir_up), _p(ir_dn),
         *grads, cfg.gradient_relative, cfg.gradient_scale, cfg.decay, cfg.input_min_percentage,
         0 if cfg.stage_events is None else cfg.stage_events(backward))
+    return packed, (up, down)
 
 
 def _rows_of(t: torch.Tensor, rows: int, cols: int, name: str) -> torch.Tensor:
@@ -211,11 +215,12 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
         if input_range is not None:
             ir_up, ir_dn = ir_tables(input_range, E, cfg)
         return y, p1, z, perm, in_index, offsets.zero_(), z_scale, ir_up, ir_dn
-    args = _pack(cfg, False, x, keys, values, input_range, None if input_range is None else input_range.dtype, sel, gate,
+    args, held = _pack(cfg, False, x, keys, values, input_range, None if input_range is None else input_range.dtype, sel, gate,
                  y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn, noise=noise, wmax=wmax,
                  per_channel=per_channel)
     ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8, device=dev)
     _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_fwd")
+    del held
     if codes and gate is not own_gate:
         y = ops.gate_reduce_codes(z, z_scale, sel, own_gate)
     return y, p1, z, perm, in_index, offsets, z_scale, ir_up, ir_dn
@@ -264,11 +269,12 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
             if g is not None:
                 g.zero_()
         return grad_x, grad_keys, grad_values, grad_ir, grad_gate
-    args = _pack(cfg, True, x, keys, values, None, None if grad_ir is None else ir_dtype, sel, gate_c, None, p1, z, z_scale, perm, in_index, offsets,
+    args, held = _pack(cfg, True, x, keys, values, None, None if grad_ir is None else ir_dtype, sel, gate_c, None, p1, z, z_scale, perm, in_index, offsets,
                  ir_up, ir_dn, (dy.data_ptr(), grad_x.data_ptr(), grad_keys.data_ptr(), grad_values.data_ptr(),
                                 grad_gate.data_ptr(), _p(grad_ir)))
     ws = torch.empty(lib.amoe_ffn_bwd_workspace(args), dtype=torch.uint8, device=x.device)
     _abi.check(lib, lib.amoe_ffn_bwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_bwd")
+    del held
     return grad_x, grad_keys, grad_values, grad_ir, grad_gate
 
 

@@ -479,9 +479,9 @@ def router_fwd(x: torch.Tensor, w: torch.Tensor, ir: torch.Tensor, k: int, bound
     sel_val = torch.empty((T, k), dtype=x.dtype, device=x.device)
     sel_idx = torch.empty((T, k), dtype=torch.int64, device=x.device)
     lib = get_lib()
-    b = (0, x.shape[1]) if bounds is None else tuple(bounds)
+    b = _abi.bounds_array((0, x.shape[1]) if bounds is None else tuple(map(int, bounds)))
     rc = lib.amoe_router_fwd(raw.dtype_code(x), x.data_ptr(), x.stride(0), T, x.shape[1], w.data_ptr(), w.stride(0), E, k,
-                             ir.data_ptr(), len(b) - 1, ctypes.addressof(_abi.bounds_array(b)), inp_res, out_bound, out_res,
+                             ir.data_ptr(), len(b) - 1, ctypes.addressof(b), inp_res, out_bound, out_res,
                              sel_val.data_ptr(), sel_idx.data_ptr(), _stream(x))
     if rc == _abi.AMOE_EUNSUPPORTED:
         return None

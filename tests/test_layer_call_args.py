@@ -1,6 +1,8 @@
 """What the layer calls (``ffn.ffn_forward`` / ``ffn_backward``, and the operators in front of them) do with arguments that
 do not fit: converted where that is exact, refused where the kernels would read something else than the tensor."""
 import dataclasses
+import types
+import weakref
 
 import pytest
 import torch
@@ -213,3 +215,32 @@ def test_gate_of_another_type(emu_ops):
     assert torch.equal(got[0].bfloat16(), want[0])
     with pytest.raises(TypeError):
         forward(pr, ADC, gate=pr["gate"].double())
+
+
+def test_k_tile_bounds_live_until_the_call_returns(emu_ops, monkeypatch):
+    """The library reads the bounds through addresses in the packed arguments: a cache that forgets them meanwhile (other
+    layers, other threads) must not free them."""
+    pr = problem()
+    made, alive = [], []
+    real, lib = _abi.bounds_array, emu_ops.get_lib()
+
+    def recorded(bounds):
+        made.append(weakref.ref(real(bounds)))
+        return made[-1]()
+
+    def during(name):
+        def call(*args):
+            for n in range(1000):
+                real((0, n + 1))
+            alive.extend(r() is not None for r in made)
+            del made[:]
+            return getattr(lib, name)(*args)
+        return call
+    monkeypatch.setattr(_abi, "bounds_array", recorded)
+    monkeypatch.setattr(emu_ops, "_LIB", types.SimpleNamespace(
+        **{n: during(n) if n in ("amoe_ffn_fwd", "amoe_ffn_bwd", "amoe_router_fwd") else getattr(lib, n) for n in _abi.PROTOTYPES}))
+    pr["ir"] = pr["ir"].expand(2, E, 2).contiguous()
+    cfg = dataclasses.replace(PLAIN, bounds_up=[0, 16, D])
+    backward(pr, cfg, forward(pr, cfg))
+    emu_ops.router_fwd(pr["x"], torch.randn(E, D), torch.ones(2), K, [0, 16, D], 1 / 127, -1.0, -1.0)
+    assert len(alive) >= 5 and all(alive)

@@ -18,7 +18,7 @@ def arguments(T, D, E, F, k, cfg, grads=(0, 0, 0, 0, 0, 0)):
              gate=torch.rand(T, k, generator=g), sel=torch.randint(0, E, (M + 1,), generator=g, dtype=torch.int64), y=torch.zeros(T, D),
              p1=torch.rand(M, F, generator=g), z=torch.rand(M, D, generator=g), perm=torch.arange(M, dtype=torch.int32),
              in_index=(torch.arange(M) // k).int(), offsets=(torch.arange(E + 1) * M // E).int())
-    args = ffn._pack(cfg, any(grads), t["x"], t["keys"], t["values"], None, None, t["sel"], t["gate"], t["y"], t["p1"], t["z"], None,
+    args, t["held"] = ffn._pack(cfg, any(grads), t["x"], t["keys"], t["values"], None, None, t["sel"], t["gate"], t["y"], t["p1"], t["z"], None,
                      t["perm"], t["in_index"], t["offsets"], None, None, grads)
     return t, args
 
