@@ -76,6 +76,12 @@ def _dense(t: torch.Tensor) -> torch.Tensor:
     return t if t.is_contiguous() else t.contiguous()
 
 
+def _operand(w: torch.Tensor) -> torch.Tensor:
+    """Weights of a forward product: the kernels take any strides as long as one of the two dimensions is adjacent."""
+    w = w.detach()
+    return w if w.stride(2) == 1 or w.stride(1) == 1 else w.contiguous()
+
+
 def _bounds(bounds, K: int):
     """The bounds of a projection's K-tiles as a C array, to be held until the call that reads them returns."""
     b = (0, K) if bounds is None else tuple(map(int, bounds))
@@ -137,7 +143,7 @@ def _int_ids(sel_idx: torch.Tensor) -> torch.Tensor:
 def _range_table(input_range: torch.Tensor, E: int, cfg: FFNConfig) -> torch.Tensor:
     """The parameter as the library reads it, [2, E, columns].  Types it does not know are converted, but for the launch that makes the
     range tables together with max |W| and takes the parameter as it is (TypeError)."""
-    with_wmax = (cfg.out_bound > 0 or (cfg.noise_std > 0 and cfg.noise_up is None)) and cfg.wmax_up is None
+    with_wmax = _reads_wmax(cfg) and cfg.wmax_up is None
     input_range = input_range.reshape(2, E, -1)
     if input_range.dtype in raw.DTYPE_CODES or (with_wmax and not cfg.noise_per_channel):
         raw.dtype_code(input_range)
@@ -154,13 +160,21 @@ def _noise(t: Optional[torch.Tensor], bounds, M: int, N: int) -> Optional[torch.
     return ops._f32c(t)
 
 
-def _wmax_tables(cfg: FFNConfig, E: int, F: int, V: int):
+def _reads_wmax(cfg: FFNConfig) -> bool:
+    return cfg.out_bound > 0 or (cfg.noise_std > 0 and cfg.noise_up is None)
+
+
+def _wmax_tables(cfg: FFNConfig, keys: torch.Tensor, values: torch.Tensor):
     """The caller's max |W| tables as the library takes them (fp32; None: it makes them) and whether they have a column per
     output channel.  Each table says for itself whether it is [E] or [E, N]; the library has one flag for both."""
+    E, F, V = *keys.shape[::2], values.shape[2]
+    if not _reads_wmax(cfg):
+        return (None, None), False
     if cfg.wmax_up is None:
-        return (None, None), cfg.noise_per_channel
-    if cfg.out_bound <= 0 and (cfg.noise_std <= 0 or cfg.noise_up is not None):
-        return (None, None), False                   # nothing reads them
+        if keys.is_contiguous() and values.is_contiguous():
+            return (None, None), cfg.noise_per_channel
+        # (the library's own reduction walks dense weights)
+        return tuple(ops.weight_abs_max(w, cfg.noise_per_channel) for w in (keys, values)), cfg.noise_per_channel
     given = ((cfg.wmax_up, F), (cfg.wmax_down, V))
     if any(t is None or t.numel() // E not in (1, N) for t, N in given):
         raise ValueError("max |W| tables must be [E] or [E, output channels]")
@@ -183,7 +197,9 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     if x.dim() != 2:
         raise ValueError("x must be [tokens, features]")
     lib = ops.get_lib()
-    x, keys, values, own_gate = ops._rows2d(x.detach()), _dense(keys), _dense(values), _dense(gate)
+    if cfg.down_ready is not None and not values.is_contiguous():    # (torch may read them below)
+        torch.cuda.current_stream().wait_event(cfg.down_ready)
+    x, keys, values, own_gate = ops._rows2d(x.detach()), _operand(keys), _operand(values), _dense(gate)
     gate = own_gate if own_gate.dtype == x.dtype else own_gate.to(x.dtype)
     sel = _int_ids(sel_idx)
     dev, dt = x.device, x.dtype
@@ -194,7 +210,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     if cfg.noise_seed_dev is not None and (cfg.noise_seed_dev.dtype != torch.int64 or cfg.noise_seed_dev.numel() != 1):
         raise ValueError("noise_seed_dev must be one int64 word")
     noise = _noise(cfg.noise_up, cfg.bounds_up, M, F), _noise(cfg.noise_down, cfg.bounds_down, M, V)
-    wmax, per_channel = _wmax_tables(cfg, E, F, V)
+    wmax, per_channel = _wmax_tables(cfg, keys, values)
     y, p1 = x.new_empty((T, V)), x.new_empty((M, F))
     perm, in_index = (torch.empty(M, dtype=torch.int32, device=dev) for _ in range(2))
     offsets = torch.empty(E + 1, dtype=torch.int32, device=dev)
@@ -239,7 +255,8 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
     (``amoe_ffn_bwd``)."""
     ops._need_gpu(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn)
     lib = ops.get_lib()
-    x, keys, values = ops._rows2d(x.detach()), _dense(keys), _dense(values)
+    x = ops._rows2d(x.detach())
+    keys, values = (w.detach() if w.stride(2) == 1 else w.detach().contiguous() for w in (keys, values))
     gate_c, sel = _dense(gate).to(x.dtype), _int_ids(sel_idx)
     (E, D, F), V = keys.shape, values.shape[2]
     T, k = x.shape[0], gate.shape[-1]
@@ -260,7 +277,7 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
     if ir_up is not None and (ir_up.shape != (E, _n_tiles(cfg.bounds_up)) or ir_dn.shape != (E, _n_tiles(cfg.bounds_down))):
         raise ValueError("input ranges must be [E, K-tiles of the projection]")
     grad_x = x.new_empty(x.shape)
-    grad_keys, grad_values, grad_gate = torch.empty_like(keys), torch.empty_like(values), torch.empty_like(gate_c)
+    grad_keys, grad_values, grad_gate = keys.new_empty((E, D, F)), values.new_empty((E, F, V)), torch.empty_like(gate_c)
     grad_ir = None
     if ir_up is not None and want_ir_grad:
         grad_ir = torch.empty((2, E, max(ir_up.shape[1], ir_dn.shape[1])), dtype=ir_dtype, device=x.device)

@@ -244,3 +244,26 @@ def test_k_tile_bounds_live_until_the_call_returns(emu_ops, monkeypatch):
     backward(pr, cfg, forward(pr, cfg))
     emu_ops.router_fwd(pr["x"], torch.randn(E, D), torch.ones(2), K, [0, 16, D], 1 / 127, -1.0, -1.0)
     assert len(alive) >= 5 and all(alive)
+
+
+@pytest.mark.parametrize("cfg", [PLAIN, ADC, dataclasses.replace(ADC, noise_std=0.04, noise_per_channel=True)], ids=["plain", "adc", "per_channel"])
+def test_weights_in_other_layouts_are_not_copied_where_the_kernels_take_strides(emu_ops, monkeypatch, cfg):
+    pr = problem()
+    want = forward(pr, cfg)
+    turned = {n: pr[n].transpose(1, 2).contiguous().transpose(1, 2) for n in ("keys", "values")}
+    wide = {n: torch.cat((pr[n], pr[n]), 2)[:, :, :pr[n].shape[2]] for n in ("keys", "values")}
+    packed = []
+    real = ffn._abi.FFN_ARGS
+    monkeypatch.setattr(ffn._abi, "FFN_ARGS", types.SimpleNamespace(pack=lambda *a: packed.append(a) or real.pack(*a)))
+    for layout in (turned, wide):
+        got = forward(pr, cfg, **layout)
+        for a, b in zip(got, want):
+            torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+        assert layout["keys"].data_ptr() in packed[-1] and layout["values"].data_ptr() in packed[-1]
+        back, ref = backward(pr, cfg, got, **layout), backward(pr, cfg, want)
+        for a, b in zip(back, ref):
+            assert a.is_contiguous()
+            torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-4)
+    assert wide["keys"].data_ptr() in packed[-2]                      # (the backward call before the reference's)
+    scattered = pr["keys"].permute(2, 1, 0).contiguous().permute(2, 1, 0)        # neither features nor outputs adjacent
+    assert same(forward(pr, cfg, keys=scattered), want)
