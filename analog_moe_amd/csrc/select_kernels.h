@@ -26,10 +26,14 @@ __device__ __forceinline__ float wave_max(float v) {
 // sel_val / sel_idx [rows, k]: the k largest gate values of each row in descending order, ties to the lower
 // expert id.  prob_partial [gridDim.x, E] (optional): per workgroup, sum over its rows of softmax(logits[row]).
 //
-// Up to 128 experts every expert counts the experts ahead of it: one scalar broadcast and a compare-and-add per
-// expert, independent of each other, where k rounds of a wave-wide maximum are 12 * k dependent lane exchanges
-// (64 experts, k = 8: 4.4 us a row against 0.6).  The count costs E * PER compares whatever k is, so two experts per
-// lane need k >= 2 to gain and more than two keep the rounds.
+// Two ways to choose: every expert counts the experts ahead of it (select_by_rank: a scalar broadcast and PER
+// compare-and-adds per expert, E * PER in all, independent of each other), or k rounds of a wave-wide maximum (a chain of 12
+// lane exchanges each).  With a wave per row the chains of many rows overlap, and both cost what they issue: 32768 rows of 64
+// experts take 7 + 27 us by count and 5.3 + 4.5 * k by rounds, of 128 experts 8 + 78 and 8 + 4.6 * k.  A round is worth 11
+// compares; more than two experts per lane keep the rounds.  (Counting wherever k >= PER, those 128 experts took 86.3 us
+// for k = 2, where rounds take 16.8.)
+__host__ __device__ inline bool select_by_count(int E, int per, int k) { return per <= 2 && E * per <= 11 * k; }
+
 template <typename T, int PER>
 __global__ __launch_bounds__(kThreads) void select_fwd_kernel(const T* __restrict__ logits, long long rows, int E, int k,
                                                                int rows_per_wave, T* __restrict__ sel_val,
@@ -68,9 +72,11 @@ __global__ __launch_bounds__(kThreads) void select_fwd_kernel(const T* __restric
 #pragma unroll
       for (int j = 0; j < PER; j++) usage[j] += ex[j] * inv;
     }
-    if (PER <= 2 && k >= PER) {
-      select_by_rank<T, PER>(s, lane, E, k, sel_val + row * k, sel_idx + row * k);
-      continue;
+    if constexpr (PER <= 2) {
+      if (select_by_count(E, PER, k)) {
+        select_by_rank<T, PER>(s, lane, E, k, sel_val + row * k, sel_idx + row * k);
+        continue;
+      }
     }
     for (int t = 0; t < k; t++) {
       float bv = kNegInf;

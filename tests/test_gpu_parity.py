@@ -372,7 +372,8 @@ def test_plain_input_gradient(ops, dtype, K, N, copies):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("T,E,k", [(1, 64, 8), (2047, 64, 64), (2051, 128, 1), (2051, 128, 2), (16389, 16, 4), (300, 65, 65)])
+@pytest.mark.parametrize("T,E,k", [(1, 64, 8), (2047, 64, 64), (2051, 128, 1), (2051, 128, 2), (16389, 16, 4), (300, 65, 65),
+                                   (2051, 64, 5), (2051, 64, 6), (300, 128, 23), (300, 128, 24), (16389, 100, 8)])
 def test_select_rows(ops, dtype, T, E, k):
     util.check_select_rows(ops, "cuda", dtype, T, E, k)
 
