@@ -756,19 +756,19 @@ int amoe_segment_sum(const float* v, const int32_t* offsets, int32_t E, int32_t 
     return AMOE_EINVAL;
   if (!v || !offsets || !out) return AMOE_ENULL;
   if (!aligned(v, 4) || !aligned(offsets, 4) || !aligned(out, esize(out_dtype))) return AMOE_EALIGN;
-  const dim3 grid(E, n_tiles + zero_cols);
+  const dim3 grid(E, n_tiles + zero_cols), block(seg_threads((long long)E * (n_tiles + zero_cols)));
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (out_dtype == AMOE_F32) {
     auto kf = &segment_sum_kernel<float>;
-    hipLaunchKernelGGL(kf, grid, dim3(kSegThreads), 0, st, v, offsets, (int)n_tiles, static_cast<float*>(out),
+    hipLaunchKernelGGL(kf, grid, block, 0, st, v, offsets, (int)n_tiles, static_cast<float*>(out),
                        (long long)ldout);
   } else if (out_dtype == AMOE_BF16) {
     auto kf = &segment_sum_kernel<uint16_t>;
-    hipLaunchKernelGGL(kf, grid, dim3(kSegThreads), 0, st, v, offsets, (int)n_tiles, static_cast<uint16_t*>(out),
+    hipLaunchKernelGGL(kf, grid, block, 0, st, v, offsets, (int)n_tiles, static_cast<uint16_t*>(out),
                        (long long)ldout);
   } else {
     auto kf = &segment_sum_kernel<f16_t>;
-    hipLaunchKernelGGL(kf, grid, dim3(kSegThreads), 0, st, v, offsets, (int)n_tiles, static_cast<f16_t*>(out),
+    hipLaunchKernelGGL(kf, grid, block, 0, st, v, offsets, (int)n_tiles, static_cast<f16_t*>(out),
                        (long long)ldout);
   }
   return launch_rc();

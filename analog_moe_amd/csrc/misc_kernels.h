@@ -448,23 +448,26 @@ __global__ __launch_bounds__(kThreads) void weight_abs_max_kernel(const T* __res
 // on (gridDim.y may exceed n_tiles) receive zero.  T: element type of out (one rounding of the fp32 sum).
 // The time is that of the longest expert's chain of loads: 1024 threads and eight values of each in flight (256 threads
 // with one load after the other took 13.6 us where one expert owns 30 000 of 131 072 rows, this takes 3.4 us).
+// Where the (expert, column) pairs alone fill the chip, a pair gets 256 threads: 8192 pairs (512 experts, 16 columns) of
+// 1024 threads take 16.5 us for 4096 rows and 19.7 for 262 144, of 256 threads 5.4 and 10.1; 2048 pairs 12.6 and 10.2.
 constexpr int kSegThreads = 1024;
+constexpr int seg_threads(long long pairs) { return pairs >= 1024 ? kThreads : kSegThreads; }
 template <typename T>
 __global__ __launch_bounds__(kSegThreads) void segment_sum_kernel(const float* __restrict__ v,
                                                                    const int32_t* __restrict__ offsets, int n_tiles,
                                                                    T* __restrict__ out, long long ldout) {
   constexpr int U = 8;
   __shared__ float red[kSegThreads / 64];
-  const int e = blockIdx.x, t = blockIdx.y;
+  const int e = blockIdx.x, t = blockIdx.y, threads = blockDim.x;
   const int tid = threadIdx.x, lane = tid & 63;
   float s = 0.f;
   if (t < n_tiles) {
     const int end = offsets[e + 1];
-    for (int i0 = offsets[e] + tid; i0 < end; i0 += U * kSegThreads) {
+    for (int i0 = offsets[e] + tid; i0 < end; i0 += U * threads) {
       float x[U];
 #pragma unroll
       for (int u = 0; u < U; u++) {
-        const int i = i0 + u * kSegThreads;
+        const int i = i0 + u * threads;
         x[u] = i < end ? v[(long long)i * n_tiles + t] : 0.f;
       }
 #pragma unroll
@@ -477,8 +480,7 @@ __global__ __launch_bounds__(kSegThreads) void segment_sum_kernel(const float* _
   __syncthreads();
   if (tid == 0) {
     float sum = 0.f;
-#pragma unroll
-    for (int w = 0; w < kSegThreads / 64; w++) sum += red[w];
+    for (int w = 0; w < threads / 64; w++) sum += red[w];
     out[(long long)e * ldout + t] = Elem<T>::cvt(sum);
   }
 }

@@ -346,6 +346,19 @@ def test_segment_sum_of_long_segments(ops, rows):
         assert np.all(np.abs(got[e] - part.sum(0)) <= bound)
 
 
+@pytest.mark.parametrize("E,cols", [(511, 2), (512, 2), (64, 16), (520, 16)])
+def test_segment_sum_of_many_segments(ops, E, cols):
+    """1024 threads per (expert, column) below 1024 pairs, 256 from there on; the same bound"""
+    g = np.random.default_rng(E)
+    off = np.concatenate(([0], np.cumsum(g.integers(0, 90, E)))).astype(np.int32)
+    off[E // 2:] += 9000                                         # one expert with many rows
+    v = g.standard_normal((int(off[-1]), cols)).astype(np.float32)
+    got = ops.segment_sum(torch.from_numpy(v).cuda(), torch.from_numpy(off).cuda(), E).cpu().numpy()
+    for e in range(E):
+        part = v[off[e]:off[e + 1]].astype(np.float64)
+        assert np.all(np.abs(got[e] - part.sum(0)) <= (len(part) + 1) * 2.0 ** -24 * np.abs(part).sum(0))
+
+
 # (the last two are large enough for the second stream in both directions)
 @pytest.mark.parametrize("case", util.LAYER_CALLS + [
     (4096, 512, 64, 256, 4, "bf16", None, True, True, 0.04),
