@@ -32,7 +32,7 @@ const char* amoe_strerror(int rc) {
 // ------------------------------------------------------------------------------ selection
 size_t amoe_prepare_sel_workspace(int64_t M, int32_t E) {
   if (M < 0 || E < 1) return 0;
-  const int64_t per = sel_by_groups(M, E) ? sel_span(M) : sel_unit(M);
+  const int64_t per = sel_by_groups(M, E) ? sel_span(M, E) : sel_unit(M);
   const int64_t units = (M + per - 1) / per;
   return (size_t)(units > 0 ? units : 1) * (size_t)E * sizeof(int32_t);
 }
@@ -50,7 +50,7 @@ int amoe_prepare_sel(const void* sel, int32_t sel_is_i64, int64_t M, int32_t E, 
   SelParams p;
   p.sel = sel; p.sel_is_i64 = sel_is_i64; p.M = M; p.E = E; p.k = k;
   const bool by_groups = sel_by_groups(M, E);
-  p.unit = by_groups ? sel_span(M) : sel_unit(M);
+  p.unit = by_groups ? sel_span(M, E) : sel_unit(M);
   p.n_units = (int)((M + p.unit - 1) / p.unit);
   p.key_bits = 0;
   while ((1 << p.key_bits) < E) p.key_bits++;

@@ -162,23 +162,27 @@ __global__ __launch_bounds__(kThreads) void sel_scatter_kernel(const SelParams p
 // and scatters.  Up to kSelSmall elements the second launch counts the keys themselves instead of a table and is the
 // only one.  The sort is on the path to the first GEMM of every step, so what matters is the number of launches and
 // the length of the dependent chain inside them, not the bytes.
-//   Span: the smallest that leaves at most kSelGroups groups, so that the table every workgroup reads stays at or
-//   below 128 KB.  One table row per wave, as the general path has it, is a table four times as large, and at 131 072
-//   elements and 128 experts it was too large for every workgroup to read: 19.4 us there and 19.0 at 64 experts,
-//   12.8 and 11.4 us as it is now (back to back in a graph).
+//   Span: the smallest that leaves at most kSelGroups groups, or as many as make a table of kSelTable counts, so that the
+//   table every workgroup reads stays at or below 128 KB and few experts still get many short groups.  One table row per
+//   wave, as the general path has it, is a table four times as large: 131 072 elements of 128 experts 19.9 us, 13.0 by
+//   groups, of 64 experts 18.5 and 11.5.  128 groups of up to 16384 elements whatever E is were too few and too long for few
+//   experts (8 experts, 262 144 elements 14.9 us, 1 000 000 40.1; as it is now 10.5 and 16.7), and a row of no multiple of
+//   four counts was read in one chain (250 experts, 131 072 elements 41.7 us; with eight loads in flight 18.1).
+//   kSelSpanMax: beyond it the general path is as fast (1 000 000 elements of 128 experts 56.2 us in spans of 8192, 55.4).
 //   kSelSmall: one launch that counts all keys takes 3.3 us at 8 elements, 4.0 at 512 (two launches: 5.9, 8.1) and grows
 //   by 0.8 us per 1024 elements; two launches take 7 us from there on.
 constexpr int kSelSmall = 4096;
-constexpr int kSelGroups = 128;
-constexpr int kSelSpanMax = 16384;
-__host__ __device__ inline int sel_span(long long M) {
+constexpr int kSelGroups = 128, kSelTable = 8192;
+constexpr int kSelSpanMax = 4096;
+__host__ __device__ inline int sel_groups_max(int E) { return kSelTable / E > kSelGroups ? kSelTable / E : kSelGroups; }
+__host__ __device__ inline int sel_span(long long M, int E) {
   int s = kThreads;
   if (M > kSelSmall)
-    while (s < kSelSpanMax && (M + s - 1) / s > kSelGroups) s <<= 1;
+    while (s < kSelSpanMax && (M + s - 1) / s > sel_groups_max(E)) s <<= 1;
   return s;
 }
 __host__ __device__ inline bool sel_by_groups(long long M, int E) {
-  return E <= kThreads && (M + sel_span(M) - 1) / sel_span(M) <= kSelGroups;
+  return E <= kThreads && (M + sel_span(M, E) - 1) / sel_span(M, E) <= sel_groups_max(E);
 }
 
 // counts of n keys from `first` into hist (LDS, zeroed), eight loads in flight per thread; true: an id out of range
@@ -266,6 +270,7 @@ __global__ __launch_bounds__(kThreads) void sel_group_scatter_kernel(const SelPa
     const int e = tid & (epad - 1), grp = tid / epad;
     int total = 0, before = 0;
     if (e < E) {
+#pragma unroll 8
       for (int u = grp; u < p.n_units; u += groups) {
         const int c = p.unit_hist[(long long)u * E + e];
         total += c;

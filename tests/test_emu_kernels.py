@@ -46,6 +46,14 @@ def test_prepare_sel_bit_exact(emu_ops, M, E, k):
     assert np.array_equal(got32[1].numpy(), want.perm)
 
 
+def test_expert_sort_of_few_experts_has_many_groups(emu_ops):
+    """128 groups were too few and too long for few experts: as many as a table of 8192 counts holds; spans up to 4096."""
+    ws = emu_ops.get_lib().amoe_prepare_sel_workspace
+    assert ws(262144, 8) == 1024 * 8 * 4 and ws(1000000, 8) == 977 * 8 * 4 and ws(1000000, 16) == 489 * 16 * 4
+    assert ws(262144, 64) == ws(524288, 64) == 128 * 64 * 4 and ws(20000, 1) == 79 * 4
+    assert ws(524289, 64) == 2049 * 64 * 4                                    # the general passes: units of 256
+
+
 CASES = {
     # name: (problem kwargs, layer kwargs, dtype, tol)
     "f32_plain": (dict(T=48, D=128, E=4, F=64, k=2), dict(), "f32", 1e-5),

@@ -321,10 +321,12 @@ def test_golden_fixture_parity(ops, name):
 
 
 @pytest.mark.parametrize("M,E,k", [(1, 1, 1), (255, 3, 1), (4096, 256, 8), (4097, 5, 1), (8200, 256, 4),
-                                   (131072, 128, 4), (262144, 255, 8), (2 ** 21 + 7, 7, 1), (9000, 257, 4)])
+                                   (131072, 128, 4), (262144, 255, 8), (2 ** 21 + 7, 7, 1), (9000, 257, 4),
+                                   (262144, 8, 8), (1000003, 16, 1), (524288, 64, 8), (524289, 64, 1), (131072, 66, 2), (70001, 1, 1)])
 @pytest.mark.parametrize("dt", [torch.int32, torch.int64])
 def test_prepare_sel_at_the_edges_of_its_paths(ops, M, E, k, dt):
-    """One launch up to 4096 elements, two beyond, the general passes beyond 256 experts or 2^21 elements."""
+    """One launch up to 4096 elements, two beyond, the general passes beyond 256 experts or, for each expert count, the
+    longest groups."""
     rng = np.random.default_rng(M + E)
     p = np.arange(1, E + 1) ** -1.2
     sel = rng.choice(E, size=M, p=p / p.sum())
