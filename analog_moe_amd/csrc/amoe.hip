@@ -165,12 +165,22 @@ int amoe_fwd_codes_supported(const amoe_fwd_args* a) {
 
 // Which kernel of gemm_direct.h takes the launch: one wave per 32 x 64 tile, eight waves per tile, or none.
 //
-// Against the tiled kernels: these re-read weights per 32 rows and rows per 64 columns.  In fp32, and where the tiled kernel
-// would run its element-wise edge code, one wave per tile was faster wherever measured (fp32, 16 experts k = 4, 2048 tokens
-// 412 -> 128: 26.8 against 53.7 us, 32768 tokens 183 against 196; bf16, 8192 tokens 128 -> 412: 38 against 73, 1024 -> 320 in two K-tiles
-// 112 against 284).  Edge-free 16-bit launches go there only while they are small: 512 -> 128 with 544 tiles 18.7 against
-// 21.7 us, with 2176 tiles 39.5 against 28.1.  A contraction of 256 with columns in groups of 256 stays with the
-// weights-in-registers kernel and its twins.
+// Against the tiled kernels: these re-read weights per 32 rows and rows per 64 columns.  What one wave per tile gains it gains
+// by overlapping the stages around the product, so it is taken in fp32, and where the tiled kernel would run its element-wise
+// edge code, but not
+//   in fp32 without an input stage past a wave per SIMD: 2048 -> 512, 1096 tiles 195 against 157 us, 64 -> 512, 3344 tiles
+//   23.3 against 20.1 (at 1 tile per SIMD and less 1.4 to 2 times faster);
+//   in fp32 with an input but no output stage in many whole column blocks: 64 -> 256, 32788 tiles 178 against 160 us, 128 ->
+//   256 257 against 235; up to 64 tiles per CU it is 1.15 to 1.3 times faster (128 -> 512, 4168 tiles 40.8 against 45.4), and
+//   with the ADC or noise at any size (32 768 tokens 412 -> 128, 8210 tiles 174 against 187; 224 -> 512, 9808 tiles 116
+//   against 168).  Loads that are exactly even over 8 experts can be tiled without a remainder, and lose up to a fifth
+//   (8192 rows 256 -> 1024 63.5 against 52.3 us);
+//   in 16 bits over a long contraction with many tiles, where the edge code is a small part: 1800 -> 512, 32904 tiles 853
+//   against 771 us, 2044 -> 512 944 against 916 (1500 -> 256, 16452 tiles 379 against 403, 1004 -> 512, 32904 tiles 522
+//   against 544).
+// bf16 with edges, 8192 tokens 128 -> 412: 38 against 73 us, 1024 -> 320 in two K-tiles 112 against 284.  Edge-free 16-bit
+// launches go there only while they are small: 512 -> 128 with 544 tiles 18.7 against 21.7 us, with 2176 tiles 39.5 against
+// 28.1.  A contraction of 256 with columns in groups of 256 stays with the weights-in-registers kernel and its twins.
 //
 // One wave or eight: a wave walks its contraction in 5 us + 45 ns (fp32) or 22 ns (16-bit) per element of K; eight waves
 // need 5 us + 12 ns or 6 ns, but fill a CU by themselves, so they do it once per 256 tiles (fp32 412 -> 128, 146 tiles 13.4
@@ -183,6 +193,11 @@ static int direct_choice(const amoe_fwd_args* a, const RowsParams& p, bool w_kc,
   const int64_t tiles = rows * ((a->N + kDirCols - 1) / kDirCols), cus = num_compute_units();
   const bool edge_free = !f32 && rows_all_interior(p, mode, a->N % kFCols == 0 && !w_kc ? kFBK : Elem<uint16_t>::kBK);
   if (edge_free && tiles > 3 * cus) return DIRECT_NO;
+  if (f32 && a->ir == nullptr && tiles > 4 * cus) return DIRECT_NO;
+  if (a->N % kTileCols == 0) {
+    if (f32 && !(a->out_bound > 0.f) && !(a->noise_std > 0.f) && tiles > 64 * cus) return DIRECT_NO;
+    if (!f32 && a->K >= 1400 && tiles * a->K > 28000000LL) return DIRECT_NO;
+  }
   const int64_t rounds = (tiles + cus - 1) / cus, K = a->K;
   const bool split = f32 ? rounds * (400 + K) * 5 < 2000 + 18 * K : rounds * (900 + K) < 800 + 4 * K;
   return split ? DIRECT_SPLIT : DIRECT_WAVE;
