@@ -58,14 +58,10 @@ def test_the_router_sees_who_watches():
 
 
 @pytest.mark.gpu
-def test_layer_in_eval_mode_refuses_a_dual_tensor_and_traces():
+def test_layer_in_eval_mode_refuses_a_dual_tensor():
     from analog_moe_amd import config as rpu
     with torch.device("cuda"):
         layer = moe_layer.AnalogSigmaMoELayer(rpu.TorchInferenceRPUConfig(), d_model=64, n_experts=4, expert_size=64, k=2).eval()
     x = torch.randn(1, 9, 64, device="cuda")
-    with torch.no_grad():
-        want = layer(x)[0]
-        traced = torch.jit.trace(lambda t: layer(t)[0], (torch.zeros_like(x),), check_trace=False)
-        assert torch.equal(traced(x), want)
-        with fwd_ad.dual_level(), pytest.raises(NotImplementedError):
-            layer(fwd_ad.make_dual(x, torch.ones_like(x)))
+    with torch.no_grad(), fwd_ad.dual_level(), pytest.raises(NotImplementedError):
+        layer(fwd_ad.make_dual(x, torch.ones_like(x)))
