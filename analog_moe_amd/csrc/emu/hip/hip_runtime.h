@@ -9,11 +9,14 @@
 #include <cmath>
 #include <cstdint>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <dlfcn.h>
 #include <map>
 #include <memory>
 #include <mutex>
 #include <sched.h>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -33,7 +36,7 @@ inline thread_local EmuIdx threadIdx, blockIdx, blockDim, gridDim;
 
 typedef int hipError_t;
 typedef void* hipStream_t;
-enum { hipSuccess = 0 };
+enum { hipSuccess = 0, hipErrorOutOfMemory = 2 };
 inline hipError_t hipGetLastError() { return hipSuccess; }
 // Launches run at once and in order, so streams and events order nothing here; what the calls would order is written down:
 // per stream the launches given to it, per event the stream and its count when it was recorded, per pair of streams how far
@@ -43,6 +46,7 @@ enum { hipEventDisableTiming = 2 };
 struct EmuOrder {
   std::mutex lock;
   uintptr_t handles = 0;
+  long long allowed = -1;                // events that can still be made (-1: any number)
   std::map<hipStream_t, long long> given;
   std::map<hipEvent_t, std::pair<hipStream_t, long long>> events;
   std::map<std::pair<hipStream_t, hipStream_t>, long long> waited;
@@ -54,6 +58,8 @@ inline void emu_note_launch(hipStream_t s) {
 }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
   std::lock_guard<std::mutex> l(emu_order.lock);
+  if (emu_order.allowed == 0) return hipErrorOutOfMemory;
+  if (emu_order.allowed > 0) emu_order.allowed--;
   *e = reinterpret_cast<hipEvent_t>(++emu_order.handles);
   return hipSuccess;
 }
@@ -73,7 +79,10 @@ inline hipError_t hipEventDestroy(hipEvent_t e) {
   emu_order.events.erase(e);
   return hipSuccess;
 }
-inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+extern "C" inline __attribute__((used)) void amoe_emu_allow_events(long long n) {
+  std::lock_guard<std::mutex> l(emu_order.lock);
+  emu_order.allowed = n;
+}
 // launches given to `other`, and how many of them stream s does not wait for
 extern "C" inline __attribute__((used)) long long amoe_emu_launches(hipStream_t other) {
   std::lock_guard<std::mutex> l(emu_order.lock);
@@ -90,8 +99,16 @@ inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 #define __align__(n) __attribute__((aligned(n)))
 #define HIP_SYMBOL(x) (&(x))
 template <class T> inline hipError_t hipGetSymbolAddress(void** p, T* sym) { *p = (void*)sym; return hipSuccess; }
-// a 3-CU device: the persistent kernels then run few workgroups with several work items each
-inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { *v = 3; return hipSuccess; }
+// A 3-CU device: the persistent kernels then run few workgroups with several work items each.  AMOE_EMU_CUS: another one,
+// for the launches that depend on how many there are (asked for once, by the first launch of a process).
+inline hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
+  const char* cus = getenv("AMOE_EMU_CUS");
+  *v = cus ? atoi(cus) : 3;
+  return hipSuccess;
+}
+// symbol of the kernel that was launched last
+inline std::string emu_last_kernel;
+extern "C" inline __attribute__((used)) const char* amoe_emu_last_kernel() { return emu_last_kernel.c_str(); }
 
 // Barrier for heavily oversubscribed threads (256 per workgroup on a few cores): waiters give up the core instead of
 // sleeping on a futex, which costs two system calls and a wake-up per thread and barrier.
@@ -143,6 +160,8 @@ template <class K, class... A>
 inline void emu_launch(K kernel, dim3 grid, dim3 block, A... args) {
   const unsigned nthreads = block.x;
   assert(nthreads % 64 == 0 && block.y == 1 && block.z == 1);
+  Dl_info symbol{};
+  emu_last_kernel = dladdr(reinterpret_cast<const void*>(kernel), &symbol) && symbol.dli_sname ? symbol.dli_sname : "";
   for (unsigned bz = 0; bz < grid.z; bz++)
   for (unsigned by = 0; by < grid.y; by++)
   for (unsigned bx = 0; bx < grid.x; bx++) {

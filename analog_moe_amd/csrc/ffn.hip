@@ -97,36 +97,40 @@ inline bool overlap_companions(const amoe_ffn_args* a) {
 }
 
 // `to` continues after what `from` has been given so far
-int order_after(hipStream_t to, hipStream_t from) {
-  hipEvent_t e;
-  if (hipError_t rc = hipEventCreateWithFlags(&e, hipEventDisableTiming)) return (int)rc;
+int order_after(hipStream_t to, hipStream_t from, hipEvent_t e) {
   hipError_t rc = hipEventRecord(e, from);
   if (rc == hipSuccess) rc = hipStreamWaitEvent(to, e, 0);
-  (void)hipEventDestroy(e);                          // (released once the stream has passed it)
   return (int)rc;
 }
 
 // Launches on the second stream beside those on the first.  However the call ends, the first stream continues after both:
-// what a launch uses belongs to the caller again once the call has returned.
+// what a launch uses belongs to the caller again once the call has returned.  Both events are there before anything is
+// launched on the second stream, so that joining it needs nothing that could still be refused.
 struct Fork {
   hipStream_t main, side;
+  hipEvent_t start = nullptr, done = nullptr;
   bool open = false;
   Fork(hipStream_t main_, void* side_stream, bool wanted)
       : main(main_), side(wanted && side_stream ? static_cast<hipStream_t>(side_stream) : main_) {}
   int begin() {
     if (side == main) return AMOE_OK;
-    const int rc = order_after(side, main);
-    open = rc == AMOE_OK;
-    return rc;
+    hipError_t rc = hipEventCreateWithFlags(&start, hipEventDisableTiming);
+    if (rc == hipSuccess) rc = hipEventCreateWithFlags(&done, hipEventDisableTiming);
+    if (rc != hipSuccess) return (int)rc;
+    const int ordered = order_after(side, main, start);
+    open = ordered == AMOE_OK;
+    return ordered;
   }
   int join() {
     if (!open) return AMOE_OK;
     open = false;
-    const int rc = order_after(main, side);
-    if (rc) (void)hipStreamSynchronize(side);        // no event to wait for: the host waits
-    return rc;
+    return order_after(main, side, done);
   }
-  ~Fork() { (void)join(); }
+  ~Fork() {
+    (void)join();
+    if (start) (void)hipEventDestroy(start);         // (released once the streams have passed them)
+    if (done) (void)hipEventDestroy(done);
+  }
   Fork(const Fork&) = delete;
   Fork& operator=(const Fork&) = delete;
 };

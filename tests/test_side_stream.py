@@ -66,3 +66,20 @@ def test_backward(emu_ops):
     before = launches(SIDE)
     rc = lib.amoe_ffn_bwd(args, ws.data_ptr(), ws.numel(), MAIN, SIDE)
     assert rc != 0 and launches(SIDE) == before + 2 and not_waited(MAIN, SIDE) == 0
+
+
+@pytest.mark.parametrize("allowed", [0, 1])
+def test_events_that_cannot_be_made(emu_ops, allowed):
+    """without both of its events the second stream is given nothing, as nothing could be made to wait for it later"""
+    lib = emu_ops.get_lib()
+    launches, not_waited = streams(lib)
+    lib.amoe_emu_allow_events.argtypes, lib.amoe_emu_allow_events.restype = [ctypes.c_longlong], None
+    t, args = arguments(1, 6144, 1, 512, 1, ffn.FFNConfig(inp_res=-1.0, out_bound=12.0, out_res=254.0))
+    ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8)
+    before = launches(SIDE)
+    lib.amoe_emu_allow_events(allowed)
+    try:
+        rc = lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), MAIN, SIDE)
+    finally:
+        lib.amoe_emu_allow_events(-1)
+    assert rc > 0 and launches(SIDE) == before and not_waited(MAIN, SIDE) == 0
