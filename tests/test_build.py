@@ -23,12 +23,14 @@ def test_build_uses_no_file_of_the_test_tree(tmp_path):
     for name in ("analog_moe_amd", "include"):
         shutil.copytree(os.path.join(ROOT, name), tmp_path / name, ignore=skip)
     shutil.copy(os.path.join(ROOT, "__graft_entry__.py"), tmp_path)
+    os.chmod(tmp_path / "analog_moe_amd" / "csrc" / "emu" / "build.sh", 0o644)       # a copy may lose the mode
+    (tmp_path / "tests" / "emu" / "libamoe_emu.so").mkdir(parents=True)              # ... and its tests be untouchable
     got = subprocess.run([sys.executable, "-c", DRY], cwd=tmp_path, env={**os.environ, "MAX_JOBS": "1"},
                          capture_output=True, text=True)
     assert got.returncode == 0, got.stderr
     runs = [line.split()[1:] for line in got.stdout.splitlines() if line.startswith("RUN")]
-    scripts = [cmd[0] for cmd in runs if cmd[0] != "hipcc"]
-    assert len(scripts) == 1 and os.access(scripts[0], os.X_OK) and str(tmp_path / "tests") not in " ".join(sum(runs, []))
+    assert [cmd for cmd in runs if cmd[0] != "hipcc"] == [["sh", str(tmp_path / "analog_moe_amd" / "csrc" / "emu" / "build.sh")]]
+    assert str(tmp_path / "tests") not in " ".join(sum(runs, []))
     # the host build's translation units find every header and declaration in the copy
     csrc = tmp_path / "analog_moe_amd" / "csrc"
     for unit in ("amoe.hip", "ffn.hip", "router.hip"):
