@@ -277,7 +277,7 @@ def counter_noise(rows: np.ndarray, block_starts: np.ndarray, n_cols: int, tile:
 def cvmm_fwd(x, sel_index, sel_sorted, keys, inp_res=-1.0, ir=None, out_index=None,
              abs_max=None, noise=None, *, bounds: Optional[Sequence[int]] = None,
              wmax=None, out_bound=-1.0, out_res=-1.0, noise_std=0.0, noise_seed=None,
-             dtype="f32", relu=False, return_codes=False):
+             dtype="f32", relu=False, return_codes=False, noise_int=None):
     """cvmm_kernel (cvmm.py:89-231) row by row, grouped per expert.
 
     x [R_in, K]; sel_index [M] input row per sorted position; sel_sorted [M] expert per
@@ -285,7 +285,8 @@ def cvmm_fwd(x, sel_index, sel_sorted, keys, inp_res=-1.0, ir=None, out_index=No
     off); out_index [M] output row per sorted position (None -> sel_index);
     abs_max [R_in] per input row (None = off); noise [n_tiles, M_out, N] or [M_out, N]
     per OUTPUT row, already scaled (None = off), or generated from ``noise_seed`` as
-    ``noise_std * wmax[e] * counter_noise``.  wmax [E, N] or [E, 1].
+    ``noise_std * wmax[e] * counter_noise``.  wmax [E, N] or [E, 1].  noise_int [n_tiles, M, N]: the
+    integers of that generator per given position, for a call with some of a selection's rows only.
 
     Per tile t with K-range [b_t, b_t+1):
         c_t = dac(x[:, range]) @ W[e][range, :]  (+ noise_t)  -> adc -> * abs_max * ir_t
@@ -330,10 +331,10 @@ def cvmm_fwd(x, sel_index, sel_sorted, keys, inp_res=-1.0, ir=None, out_index=No
             c = (a.astype(np.float64) @ w_op[e, lo:hi, :].astype(np.float64)).astype(F32)
             if noise is not None:
                 c = (c + noise[t, rout, :]).astype(F32)
-            elif noise_seed is not None and noise_std > 0:
+            elif (noise_seed is not None or noise_int is not None) and noise_std > 0:
                 # 32-row blocks are counted from the expert's first sorted position
                 starts = pos[0] + (np.arange(len(pos)) // 32) * 32
-                zi = counter_noise_int(rout, starts, N, t, noise_seed).astype(F32)
+                zi = (counter_noise_int(rout, starts, N, t, noise_seed) if noise_int is None else noise_int[t][pos]).astype(F32)
                 nz = ((F32(noise_std) * wmax[e][None, :]).astype(F32) * NOISE_SCALE).astype(F32)
                 # one fused multiply-add, as the kernel does it (the product is exact in float64)
                 c = (zi.astype(np.float64) * nz.astype(np.float64) + c.astype(np.float64)).astype(F32)

@@ -4,8 +4,10 @@ scheduling and the analog pro/epilogues against the oracle without a GPU; the ma
 instruction and LDS-transpose stand-ins reproduce the operand layouts measured on MI355X.
 The product path is untouched: these tests point analog_moe_amd.ops at the host build by
 monkeypatching."""
+import ctypes
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -361,12 +363,34 @@ def test_layer_calls_equal_the_single_calls(emu_ops, case):
 
 
 
-@pytest.mark.parametrize("dtype,K,N,kc,tiles,stages", [
-    (torch.bfloat16, 130, 66, False, 2, "noisy"), (torch.bfloat16, 576, 64, True, 1, "noisy"), (torch.float16, 64, 2, False, 1, "plain"),
-    (torch.float32, 301, 34, False, 1, "noisy"), (torch.float32, 36, 61, True, 2, "dac")])
+SMALL_TILES = [("bfloat16", 130, 66, False, 2, "noisy"), ("bfloat16", 576, 64, True, 1, "noisy"), ("float16", 64, 2, False, 1, "plain"),
+               ("float16", 300, 34, False, 1, "noisy"), ("float32", 301, 34, False, 1, "noisy"), ("float32", 36, 61, True, 2, "dac")]
+
+
+def last_kernel(lib):
+    lib.amoe_emu_last_kernel.restype = ctypes.c_char_p
+    return lib.amoe_emu_last_kernel().decode()
+
+
+@pytest.mark.parametrize("dtype,K,N,kc,tiles,stages", SMALL_TILES)
 def test_forward_small_tiles(emu_ops, dtype, K, N, kc, tiles, stages):
-    util.check_forward_small_tiles(emu_ops, "cpu", dtype, K, N, kc, tiles, stages)
-    util.check_forward_small_tiles(emu_ops, "cpu", dtype, K, N, kc, tiles, stages, copies=3)     # one wave per tile
+    """one wave per tile: on three compute units eight would take these tiles in several rounds"""
+    for copies in (1, 3):
+        util.check_forward_small_tiles(emu_ops, "cpu", getattr(torch, dtype), K, N, kc, tiles, stages, copies=copies)
+        assert "direct_wave_kernel" in last_kernel(emu_ops.get_lib())
+
+
+def test_forward_small_tiles_over_eight_waves(emu_ops):
+    """the same launches on 256 compute units (a process of its own: the library asks once how many there are)"""
+    child = ("import torch; from analog_moe_amd import _abi, ops; from tests import test_emu_kernels as t, util\n"
+             "ops._LIB, ops._stream, ops._need_gpu = _abi.bind(t.EMU_SO), (lambda x: None), (lambda *a: None)\n"
+             "for dt, *case in t.SMALL_TILES:\n"
+             "    util.check_forward_small_tiles(ops, 'cpu', getattr(torch, dt), *case)\n"
+             "    assert 'direct_fwd_kernel' in t.last_kernel(ops.get_lib()), (dt, case)\n"
+             "print('all ran')\n")
+    got = subprocess.run([sys.executable, "-c", child], cwd=os.path.dirname(HERE), env={**os.environ, "AMOE_EMU_CUS": "256"},
+                         capture_output=True, text=True)
+    assert got.returncode == 0 and got.stdout.endswith("all ran\n"), got.stderr
 
 
 @pytest.mark.parametrize("dtype,K,N", util.PLAIN_BWDX[:5])
