@@ -71,15 +71,24 @@ def _p(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+# What arrives as the kernels want it, which is nearly always, is passed on as it is: a view costs a microsecond of the host.
 def _dense(t: torch.Tensor) -> torch.Tensor:
-    t = t.detach()
-    return t if t.is_contiguous() else t.contiguous()
+    return t if t.is_contiguous() else t.detach().contiguous()
+
+
+def _fp32(t: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+    return t if t is None or (t.dtype == torch.float32 and t.is_contiguous()) else ops._f32c(t)
+
+
+def _rows(t: torch.Tensor) -> torch.Tensor:
+    """A matrix whose rows are adjacent elements."""
+    return t if t.stride(1) == 1 else t.detach().contiguous()
 
 
 def _operand(w: torch.Tensor) -> torch.Tensor:
     """Weights of a forward product: the kernels take any strides as long as one of the two dimensions is adjacent."""
-    w = w.detach()
-    return w if w.stride(2) == 1 or w.stride(1) == 1 else w.contiguous()
+    _, inner, last = w.stride()
+    return w if last == 1 or inner == 1 else w.detach().contiguous()
 
 
 def _bounds(bounds, K: int):
@@ -122,7 +131,7 @@ def _rows_of(t: torch.Tensor, rows: int, cols: int, name: str) -> torch.Tensor:
     """t as a contiguous [rows, cols]."""
     if t.shape == (rows, cols) and t.is_contiguous():
         return t
-    if t.shape[-1] != cols or t.numel() != rows * cols:
+    if t.dim() == 0 or t.shape[-1] != cols or t.numel() != rows * cols:
         raise ValueError(f"{name} must be [{rows}, {cols}], not {tuple(t.shape)}")
     return t.detach().reshape(rows, cols).contiguous()
 
@@ -134,18 +143,18 @@ def _check_heads(sel: torch.Tensor, gate: torch.Tensor, M: int, k: int) -> None:
 
 
 def _int_ids(sel_idx: torch.Tensor) -> torch.Tensor:
-    sel = sel_idx.detach()
-    if sel.dtype not in (torch.int32, torch.int64):
-        sel = sel.to(torch.int64)
-    return sel if sel.is_contiguous() else sel.contiguous()
+    if sel_idx.dtype not in (torch.int32, torch.int64):
+        sel_idx = sel_idx.detach().to(torch.int64)
+    return _dense(sel_idx)
 
 
 def _range_table(input_range: torch.Tensor, E: int, cfg: FFNConfig) -> torch.Tensor:
     """The parameter as the library reads it, [2, E, columns].  Types it does not know are converted, but for the launch that makes the
     range tables together with max |W| and takes the parameter as it is (TypeError)."""
-    with_wmax = _reads_wmax(cfg) and cfg.wmax_up is None
-    input_range = input_range.reshape(2, E, -1)
-    if input_range.dtype in raw.DTYPE_CODES or (with_wmax and not cfg.noise_per_channel):
+    shape = input_range.shape
+    if len(shape) != 3 or shape[0] != 2 or shape[1] != E:
+        input_range = input_range.detach().reshape(2, E, -1)
+    if input_range.dtype in raw.DTYPE_CODES or (_reads_wmax(cfg) and cfg.wmax_up is None and not cfg.noise_per_channel):
         raw.dtype_code(input_range)
         return _dense(input_range)
     return _dense(input_range.detach().float())
@@ -157,7 +166,7 @@ def _noise(t: Optional[torch.Tensor], bounds, M: int, N: int) -> Optional[torch.
         return None
     if t.numel() != _n_tiles(bounds) * M * N:
         raise ValueError(f"injected noise must be [{_n_tiles(bounds)}, {M}, {N}], not {tuple(t.shape)}")
-    return ops._f32c(t)
+    return _fp32(t)
 
 
 def _reads_wmax(cfg: FFNConfig) -> bool:
@@ -167,7 +176,6 @@ def _reads_wmax(cfg: FFNConfig) -> bool:
 def _wmax_tables(cfg: FFNConfig, keys: torch.Tensor, values: torch.Tensor):
     """The caller's max |W| tables as the library takes them (fp32; None: it makes them) and whether they have a column per
     output channel.  Each table says for itself whether it is [E] or [E, N]; the library has one flag for both."""
-    E, F, V = *keys.shape[::2], values.shape[2]
     if not _reads_wmax(cfg):
         return (None, None), False
     if cfg.wmax_up is None:
@@ -175,14 +183,15 @@ def _wmax_tables(cfg: FFNConfig, keys: torch.Tensor, values: torch.Tensor):
             return (None, None), cfg.noise_per_channel
         # (the library's own reduction walks dense weights)
         return tuple(ops.weight_abs_max(w, cfg.noise_per_channel) for w in (keys, values)), cfg.noise_per_channel
-    given = ((cfg.wmax_up, F), (cfg.wmax_down, V))
+    E = keys.shape[0]
+    given = ((cfg.wmax_up, keys.shape[2]), (cfg.wmax_down, values.shape[2]))
     if any(t is None or t.numel() // E not in (1, N) for t, N in given):
         raise ValueError("max |W| tables must be [E] or [E, output channels]")
     wide = [t.numel() // E == N != 1 for t, N in given]
     late = cfg.wmax_down
     if cfg.down_ready is not None and (late.dtype != torch.float32 or not late.is_contiguous() or wide[0] != wide[1]):
         torch.cuda.current_stream().wait_event(cfg.down_ready)
-    tables = [ops._f32c(t) for t, _ in given]
+    tables = [_fp32(t) for t, _ in given]
     if any(wide):
         tables = [t if w else t.reshape(-1)[:E, None].expand(E, N).contiguous() for t, w, (_, N) in zip(tables, wide, given)]
     return tuple(tables), any(wide)
@@ -199,8 +208,8 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
     lib = ops.get_lib()
     if cfg.down_ready is not None and not values.is_contiguous():    # (torch may read them below)
         torch.cuda.current_stream().wait_event(cfg.down_ready)
-    x, keys, values, own_gate = ops._rows2d(x.detach()), _operand(keys), _operand(values), _dense(gate)
-    gate = own_gate if own_gate.dtype == x.dtype else own_gate.to(x.dtype)
+    x, keys, values, own_gate = _rows(x), _operand(keys), _operand(values), _dense(gate)
+    gate = own_gate if own_gate.dtype == x.dtype else own_gate.detach().to(x.dtype)
     sel = _int_ids(sel_idx)
     dev, dt = x.device, x.dtype
     (E, D, F), V = keys.shape, values.shape[2]
@@ -255,9 +264,13 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
     (``amoe_ffn_bwd``)."""
     ops._need_gpu(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn)
     lib = ops.get_lib()
-    x = ops._rows2d(x.detach())
-    keys, values = (w.detach() if w.stride(2) == 1 else w.detach().contiguous() for w in (keys, values))
-    gate_c, sel = _dense(gate).to(x.dtype), _int_ids(sel_idx)
+    if x.dim() != 2:
+        x = x.detach().reshape(-1, x.shape[-1])
+    x = _rows(x)
+    keys, values = (w if w.stride(2) == 1 else w.detach().contiguous() for w in (keys, values))
+    gate_c, sel = _dense(gate), _int_ids(sel_idx)
+    if gate_c.dtype != x.dtype:
+        gate_c = gate_c.detach().to(x.dtype)
     (E, D, F), V = keys.shape, values.shape[2]
     T, k = x.shape[0], gate.shape[-1]
     M = T * k
@@ -273,7 +286,7 @@ def ffn_backward(dy, x, keys, values, gate, sel_idx, p1, z, z_scale, perm, in_in
             raise ValueError(f"{name} must hold {n} values")
     if (ir_up is None) != (ir_dn is None):
         raise ValueError("input ranges of both projections or of none")
-    ir_up, ir_dn = ops._f32c(ir_up), ops._f32c(ir_dn)
+    ir_up, ir_dn = _fp32(ir_up), _fp32(ir_dn)
     if ir_up is not None and (ir_up.shape != (E, _n_tiles(cfg.bounds_up)) or ir_dn.shape != (E, _n_tiles(cfg.bounds_down))):
         raise ValueError("input ranges must be [E, K-tiles of the projection]")
     grad_x = x.new_empty(x.shape)
