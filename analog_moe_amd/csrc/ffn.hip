@@ -1,5 +1,5 @@
-// The expert feed-forward of a layer as one call per direction: the single entry points in their order, on two streams
-// where the launches are long enough to gain from it.
+// The expert feed-forward of a layer as one call per direction: the single entry points in their order, in the backward
+// direction on two streams where the launches are long enough to gain from it.
 #include <amoe.h>
 
 #include "host_util.h"
@@ -85,13 +85,18 @@ BwdScratch bwd_scratch(const amoe_ffn_args* a, Arena& m) {
   return s;
 }
 
-// Two streams pay for their events (about 10 us of latency per fork and join on the GPU, a few on the host) only where
-// the launches they overlap are long: the tables read the weights, the companions of the backward pass stream the
-// k-head tensors.
+// A fork and a join cost 10 to 20 us of the GPU's time.  The forward call has nothing long enough to hide behind the other
+// branch: its tables beside the sort lost at every size (us per call, one stream and two: one token of 64 experts, 16 MB of
+// weights 33 / 55, 64 MB 50 / 72; 1000 tokens 100 / 118; 16384 tokens 294 / 304; 32768 tokens, 512 MB 1054 / 1065).  In the
+// backward call the companions stream the k-head tensors beside the weight gradients, whose last tiles leave CUs idle where
+// the loads are uneven.  us per call, one stream and two, by the bytes of those tensors (z: load of the
+// experts by Zipf(1.2), otherwise even):
+//   16 experts, bf16: 8 MB 76 / 81, 16 MB 99 / 99, z 24 MB 103 / 101, 32 MB 105 / 111, 40 MB 115 / 118, z 125 / 120, 128 MB
+//   238 / 228, z 256 / 233; fp32: 40 MB 179 / 178, 64 MB 228 / 222, 96 MB 252 / 243, z 292 / 279; 412 features: 19 MB 146 / 150,
+//   31 MB 179 / 174, fp32 63 MB 260 / 250
+//   64 experts, bf16: 16 MB 117 / 132, z 48 MB 184 / 178, 128 MB 203 / 207, z 285 / 273, 512 MB 529 / 535, z 748 / 692
+// The line lies where uneven loads begin to gain; even loads lose up to 6 % beyond it, and gain 2 to 5 % where experts are few.
 constexpr long long kOverlapBytes = 24LL << 20;
-inline bool overlap_tables(const amoe_ffn_args* a) {
-  return a->E * (a->D + a->V) * a->F * (long long)esize((int)a->dtype) >= kOverlapBytes;
-}
 inline bool overlap_companions(const amoe_ffn_args* a) {
   return rows_of(a) * (a->D + a->V) * (long long)esize((int)a->dtype) >= kOverlapBytes;
 }
@@ -208,7 +213,7 @@ size_t amoe_ffn_bwd_workspace(const amoe_ffn_args* a) {
   return m.used;
 }
 
-int amoe_ffn_fwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes, void* stream, void* side_stream) {
+int amoe_ffn_fwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes, void* stream, void* /* side_stream */) {
   if (int rc = check_args(a)) return rc;
   if (!workspace || !a->y || (has_ranges(a) && !a->input_range)) return AMOE_ENULL;
   if (has_ranges(a) && (a->ir_cols < a->n_up || a->ir_cols < a->n_dn)) return AMOE_ESHAPE;
@@ -219,12 +224,9 @@ int amoe_ffn_fwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int64_t M = rows_of(a);
   const bool ranges = has_ranges(a), gen = generates_noise(a), chain = chained(a);
-  // max |W| per expert and the fp32 input-range tables only read parameters: they can run next to the expert sort
-  Fork fork(st, side_stream, s.wmax_up && overlap_tables(a));
-  if (int rc = fork.begin()) return rc;
   if (s.wmax_up || ranges) {
-    Stage t(a, 1, fork.side);
-    if (int rc = tables(a, s, fork.side)) return rc;
+    Stage t(a, 1, st);
+    if (int rc = tables(a, s, st)) return rc;
   }
   {
     Stage t(a, 0, st);
@@ -232,7 +234,6 @@ int amoe_ffn_fwd(const amoe_ffn_args* a, void* workspace, size_t workspace_bytes
                                   a->in_index, a->offsets, nullptr, s.sort, amoe_prepare_sel_workspace(M, (int32_t)a->E), st))
       return rc;
   }
-  if (int rc = fork.join()) return rc;
   const float* wmax_up = a->wmax_up ? a->wmax_up : s.wmax_up;
   const float* wmax_dn = a->wmax_dn ? a->wmax_dn : s.wmax_dn;
 

@@ -244,7 +244,7 @@ def ffn_forward(x, keys, values, input_range, gate, sel_idx, cfg: FFNConfig):
                  y, p1, z, z_scale, perm, in_index, offsets, ir_up, ir_dn, noise=noise, wmax=wmax,
                  per_channel=per_channel)
     ws = torch.empty(lib.amoe_ffn_fwd_workspace(args), dtype=torch.uint8, device=dev)
-    _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), ops._side(x)), "amoe_ffn_fwd")
+    _abi.check(lib, lib.amoe_ffn_fwd(args, ws.data_ptr(), ws.numel(), ops._stream(x), None), "amoe_ffn_fwd")
     del held
     if codes and gate is not own_gate:
         y = ops.gate_reduce_codes(z, z_scale, sel, own_gate)

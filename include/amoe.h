@@ -439,8 +439,9 @@ typedef struct amoe_ffn_args {
 /* Bytes of scratch memory the call needs (reads sizes and settings only).  Nothing in it outlives the call. */
 size_t amoe_ffn_fwd_workspace(const amoe_ffn_args* args);
 size_t amoe_ffn_bwd_workspace(const amoe_ffn_args* args);
-/* Launches on `stream`; launches that can run beside them go to `side_stream` (NULL: none do), which is joined with
- * `stream` before the call returns, so that memory order on `stream` alone is enough for the caller. */
+/* Launches on `stream`; launches that can run beside them may go to `side_stream` (NULL: none do; the forward call has
+ * none that gain by it), which is joined with `stream` before the call returns, so that memory order on `stream` alone is
+ * enough for the caller. */
 int amoe_ffn_fwd(const amoe_ffn_args* args, void* workspace, size_t workspace_bytes, void* stream, void* side_stream);
 int amoe_ffn_bwd(const amoe_ffn_args* args, void* workspace, size_t workspace_bytes, void* stream, void* side_stream);
 /* Name of stage i of a direction, NULL past the last. */
