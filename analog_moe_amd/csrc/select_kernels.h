@@ -8,9 +8,12 @@ namespace amoe {
 
 constexpr int kSelPerLane = 8;            // experts per lane: E <= 512
 // Rows a wave walks through (its usage sums stay in registers meanwhile).  A row is a serial chain of about a
-// microsecond, so few rows take a wave each -- 1717 rows of 64 experts: 35.4 us with eight rows per wave -- and only
-// where two waves per SIMD are there anyway do they take more, for fewer partial usage sums to add.
-__host__ __device__ inline int select_rows_per_wave(long long rows) { return rows <= 2048 ? 1 : rows <= 16384 ? 2 : 8; }
+// microsecond, so few rows take a wave each; many rows take more each, for fewer partial usage sums to add.  us per launch for
+// 1, 2 and 8 rows per wave, with the usage sums (and without):
+//   64 experts, k = 8: 2048 rows 14.9 18.2 39.2 (4.9 7.9 26.6), 4096 17.2 19.3 39.9 (6.3 8.4 26.9), 8192 22.5 21.4 39.9 (9.7
+//   10.3 27.0), 32768 51.2 46.3 48.7 (28.7 28.8 34.4), 65536 89.9 78.2 79.1 (53.3 52.9 59.5), 131072 167 142 132 (103 101 106)
+//   16 experts, k = 4: 4096 rows 15.3 15.3 23.0, 32768 34.5 29.2 28.8, 131072 105 80 64; 128 experts: 4096 21.9 21.9 39.4
+__host__ __device__ inline int select_rows_per_wave(long long rows) { return rows <= 4096 ? 1 : rows <= 32768 ? 2 : 8; }
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

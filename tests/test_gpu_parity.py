@@ -391,6 +391,12 @@ def test_select_rows(ops, dtype, T, E, k):
     util.check_select_rows(ops, "cuda", dtype, T, E, k)
 
 
+@pytest.mark.parametrize("T", [4096, 4097, 32768, 32771])
+def test_select_with_usage_sums(ops, T):
+    """Both sides of the lines between one, two and eight rows per wave."""
+    util.check_select(ops, torch.float32, device="cuda", T=T)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("T,D,E,k,tiles,adc", [(1, 1024, 64, 8, 1, True), (2049, 412, 16, 4, 1, True), (4100, 1024, 64, 8, 2, True),
                                                (8200, 520, 128, 128, 8, False), (77, 2050, 65, 1, 4, True), (31, 4, 1, 1, 1, True)])
