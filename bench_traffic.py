@@ -27,9 +27,12 @@ ROLES = {"fwd": ("fwd_up", "fwd_down"), "xgrad": ("xgrad_down", "xgrad_up"), "wg
 
 
 def source_digest() -> str:
-    """sha256 over the kernel sources (names and contents), the same for the profiling run and for bench.py"""
+    """sha256 over the kernel sources (names and contents), the same for the profiling run and for bench.py; the headers of
+    the host build (emu/) are not part of the library"""
     h = hashlib.sha256()
     for dirpath, _, files in sorted(os.walk(CSRC)):
+        if "emu" in os.path.relpath(dirpath, CSRC).split(os.sep):
+            continue
         for f in sorted(files):
             if f.endswith((".h", ".hip")):
                 h.update(f.encode())
@@ -61,6 +64,10 @@ def family(kernel: str):
     if "ws256_kernel<" in kernel:                # <T, weights-K-contiguous, ...>: the input gradient reads W that way
         args = kernel.split("ws256_kernel<", 1)[1].split(">", 1)[0].split(",")
         return "xgrad" if args[1].strip() == "true" else "fwd"
+    for direct in ("direct_wave_kernel<", "direct_fwd_kernel<"):       # <T, weights-K-contiguous, ...> likewise
+        if direct in kernel:
+            args = kernel.split(direct, 1)[1].split(">", 1)[0].split(",")
+            return "xgrad" if args[1].strip() == "true" else "fwd"
     if "fwd256_kernel" in kernel:
         return "fwd"
     if "bwdx256_kernel" in kernel:

@@ -13,6 +13,9 @@ def test_kernel_families():
     assert BT.family("void amoe::wgrad_reduce_kernel<unsigned short>(amoe::WgradParams)") is None
     assert BT.family("void amoe::gemm_rows_kernel<float, true, 2, false>(amoe::RowsParams)") == "xgrad"
     assert BT.family("void amoe::gemm_rows_kernel<float, false, 1, false>(amoe::RowsParams)") == "fwd"
+    assert BT.family("void amoe::direct_wave_kernel<unsigned short, false, true>(amoe::RowsParams)") == "fwd"
+    assert BT.family("void amoe::direct_wave_kernel<float, true, false>(amoe::RowsParams)") == "xgrad"
+    assert BT.family("void amoe::direct_fwd_kernel<unsigned short, false>(amoe::RowsParams)") == "fwd"
     assert BT.family("void amoe::head_reduce_kernel<unsigned short>(...)") is None
 
 
@@ -66,3 +69,14 @@ def test_recorded_traffic_file_is_well_formed():
         rec = json.load(fh)
     assert set(rec["launches"]) == {"fwd_up", "fwd_down", "xgrad_down", "xgrad_up", "wgrad_down", "wgrad_up"}
     assert all(v["total_bytes"] > 1e8 for v in rec["launches"].values())
+
+
+def test_the_host_builds_headers_are_no_kernel_sources(tmp_path, monkeypatch):
+    monkeypatch.setattr(BT, "CSRC", str(tmp_path))
+    (tmp_path / "emu" / "hip").mkdir(parents=True)
+    (tmp_path / "intrin").mkdir()
+    digests = []
+    for path in ("a.hip", "emu/hip/hip_runtime.h", "emu/gfx950_intrin.h", "intrin/gfx950_intrin.h"):
+        (tmp_path / path).write_text("x")
+        digests.append(BT.source_digest())
+    assert digests[0] == digests[1] == digests[2] != digests[3]
