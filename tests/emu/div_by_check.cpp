@@ -1,6 +1,6 @@
 // Host check of amoe::div_by (csrc/common.h: one multiplication and two fused multiply-adds with y = 1/b) against the
 // correctly rounded IEEE quotient a / b, over the operand ranges of the DAC stage (|a| <= |b| scaled, b a positive
-// input range or quantisation step).  Built on demand by tests/test_oracle.py with the stand-in headers of tests/emu.
+// input range or quantisation step).  Built on demand by tests/test_oracle.py with the stand-in headers of csrc/emu.
 #include <cstdint>
 #include <cstring>
 #include <cmath>
