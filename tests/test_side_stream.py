@@ -2,7 +2,6 @@
 once the call has returned, with an error as without one."""
 import ctypes
 
-import pytest
 import torch
 
 from analog_moe_amd import ffn
