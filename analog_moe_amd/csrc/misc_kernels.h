@@ -480,7 +480,8 @@ __global__ __launch_bounds__(kSegThreads) void segment_sum_kernel(const float* _
   __syncthreads();
   if (tid == 0) {
     float sum = 0.f;
-    for (int w = 0; w < threads / 64; w++) sum += red[w];
+#pragma unroll
+    for (int w = 0; w < kSegThreads / 64; w++) sum += w < threads / 64 ? red[w] : 0.f;      // (all reads in flight at once)
     out[(long long)e * ldout + t] = Elem<T>::cvt(sum);
   }
 }
